@@ -71,6 +71,14 @@ struct GemmPlan {
   int64_t splits;  // k-ranges (1: K' not split)
 };
 
+// compute units of the current device
+int device_cus(int* cus) {
+  int dev = 0;
+  SILE_HIP_CHECK(hipGetDevice(&dev));
+  SILE_HIP_CHECK(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
+  return *cus > 0 ? SILE_OK : SILE_ERR_RUNTIME;
+}
+
 // seconds per element of K' for one tile, with w workgroups of that size
 // running at once on `cus` CUs (fitted: 256 x 256 16 ns up to cus / 2
 // workgroups, 21.8 ns at cus; 128 x 128 7.2 ns up to cus / 2, 7.8 ns at cus,
@@ -922,16 +930,69 @@ int sile_hip_attention_f32_kt(int64_t n_q, int64_t n_k, int64_t head_dim, const 
   if (!q || !kt || !v || !o) return fail(SILE_ERR_SHAPE, "NULL operand");
   if (ldq < head_dim || ldkt < n_k || ldv < head_dim || ldo < head_dim)
     return fail(SILE_ERR_SHAPE, "leading dimension smaller than the matrix extent");
-  const int64_t blocks = (n_q + 63) / 64;
-  if (blocks > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "attention too large");
-  const int dp = (int)((head_dim + 15) / 16 * 16);
+  // A workgroup takes 32 queries (one workgroup a CU; its 8 waves take key
+  // blocks of 32 in turn), and the keys are split into ranges where that
+  // leaves CUs idle.  The range count with the least modelled time: a SIMD
+  // takes 1 + 3.15 dp / 128 us a key block (4.15 measured at d = 128, flatter
+  // below), and ranges add 8 us and 0.1 us each (the second launch, and the
+  // event that orders its scratch).  Measured at 1024 x 4096, d = 128: 141, 83,
+  // 50, 36, 46 us with 1, 2, 4, 8, 16 ranges; 300 x 700, d = 80: 26, 23, 20, 17,
+  // 18; 128 x 4096, d = 64: 80, 50, 32, 23, 20.  A captured call is not split
+  // (events recorded at call time do not order a graph's replays), nor is one
+  // whose scratch cannot be allocated.
+  const int64_t q_tiles = (n_q + 31) / 32, key_blocks = (n_k + 31) / 32;
+  // row pitches past 2^26 do not fit the kernels' 32-bit lane offsets
+  const bool far = ldkt > (1 << 26) || ldv > (1 << 26);
+  const int dp = far ? (head_dim <= 32 ? 32 : 128) : (int)((head_dim + 15) / 16 * 16);
+  const int pitch = (dp + 31) / 32 * 32;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  int splits = 1, cus = 0;
+  int64_t per_split = key_blocks;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  const bool capturing =
+      hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+  if (!capturing && device_cus(&cus) == SILE_OK) {
+    double best = 1e30;
+    for (int64_t z = 1; z <= std::min<int64_t>(64, key_blocks) && (z == 1 || z * q_tiles <= 2 * cus);
+         ++z) {
+      const int64_t rounds = (q_tiles * z + cus - 1) / cus;
+      const int64_t per_simd = ((key_blocks + z - 1) / z + 3) / 4;
+      const double t = (1.0 + 3.15 * dp / 128) * (double)(rounds * per_simd) +
+                       (z > 1 ? 8.0 + 0.1 * (double)z : 0.0);
+      if (t < best) {
+        best = t;
+        splits = (int)z;
+      }
+    }
+  }
+  void* ws = nullptr;
+  if (splits > 1) {
+    per_split = (key_blocks + splits - 1) / splits;
+    splits = (int)((key_blocks + per_split - 1) / per_split);
+    if (scratch_acquire((size_t)(splits * n_q) * (pitch + 2) * sizeof(float), s, &ws) != SILE_OK) {
+      ws = nullptr;
+      splits = 1;
+      per_split = key_blocks;
+    }
+  }
+  if (q_tiles * splits > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "attention too large");
   char name[64];
-  snprintf(name, sizeof name, "sile_attn_f32_kt_d%d", dp);
+  snprintf(name, sizeof name, "sile_attn_f32_kt_%s%d", far ? "far" : "d", dp);
   int d = (int)head_dim;
-  void* params[] = {(void*)&q, &ldq, (void*)&kt, &ldkt, (void*)&v, &ldv, &o, &ldo,
-                    &n_q, &n_k, &d, &scale, &m0};
-  int rc = launch(Module::kAttention, name, dim3((unsigned)blocks), dim3(256), params,
-                  static_cast<hipStream_t>(stream));
+  float* out = ws ? static_cast<float*>(ws) : o;
+  float* ml = ws ? out + (int64_t)splits * n_q * pitch : nullptr;
+  void* params[] = {(void*)&q, &ldq, (void*)&kt, &ldkt, (void*)&v, &ldv, &out, &ldo, &ml,
+                    &n_q, &n_k, &d, &scale, &m0, &splits, &per_split};
+  int rc = launch(Module::kAttention, name, dim3((unsigned)(q_tiles * splits)), dim3(512), params, s);
+  if (ws) {
+    if (rc == SILE_OK) {
+      int pt = pitch;
+      void* cp[] = {&out, &ml, &o, &ldo, &n_q, &d, &pt, &splits};
+      rc = launch(Module::kAttention, "sile_attn_f32_combine",
+                  dim3((unsigned)((n_q + 7) / 8)), dim3(256), cp, s);
+    }
+    scratch_release(s);
+  }
   return rc == SILE_OK ? ok() : rc;
 }
 

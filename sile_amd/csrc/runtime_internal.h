@@ -56,7 +56,8 @@ int kernel_matmul_seeded(void* const* buffers, int64_t num_threadgroups, int64_t
                          const float* seed, const int64_t* seed_shape, float seed_value,
                          hipStream_t s);
 // Device scratch shared by the calls on one device, in two slots: slot 0 the
-// split-K GEMM's fp32 partials and the transposed form's planes, slot 1 a
+// split-K GEMM's fp32 partials, the transposed form's planes and the fp32
+// attention's partial results, slot 1 a
 // row-major B transposed for the column-major kernels (each at most
 // 256 MiB).  scratch_acquire makes stream s wait for the kernels of the
 // slot's previous user (an event, so calls on different streams are ordered

@@ -357,6 +357,45 @@ def test_attention_f32_kt_matches_the_program(hip, n_q, n_k, d, pad, m0):
     assert (got[:, d:] == 7.0).all()
 
 
+@pytest.mark.parametrize("n_q,n_k,d,pad,m0", [
+    (32, 32, 128, 0, -1e30),      # one key block
+    (33, 33, 33, 1, -1e30),       # a query, a key and a dim past one tile
+    (31, 1000, 17, 0, -1e30),     # key ranges, a partial last block, dims padded to 32
+    (65, 257, 1, 2, -1e30),       # one dim
+    (40, 2049, 47, 0, -3.0),      # many ranges; max from the initial value
+    (64, 700, 66, 1, -1e30),      # dims padded to 80
+    (70, 300, 95, 3, -1e30),
+    (34, 3000, 112, 0, -1e30),
+    (513, 4096, 127, 1, -1e30),   # the last dim of 128 missing
+    (8200, 64, 20, 0, -1e30),     # more query tiles than CUs: no ranges
+])
+def test_attention_f32_kt_tiles_and_ranges(hip, n_q, n_k, d, pad, m0):
+    """The edges of the 32-query tiles, 32-key blocks and 16-dim steps, and the
+    key ranges added by a second kernel; the same bounds as above."""
+    test_attention_f32_kt_matches_the_program(hip, n_q, n_k, d, pad, m0)
+
+
+@pytest.mark.parametrize("d,ldkt,ldv", [(3, (1 << 26) + 1, 3), (33, 40, (1 << 26) + 1)])
+def test_attention_f32_kt_far_pitches(hip, d, ldkt, ldv):
+    """Row pitches past the 32-bit lane offsets (kt's rows 256 MiB apart, or
+    v's): the kernels with a 64-bit address a load."""
+    n_q, n_k = 33, 3
+    say(f"attention_f32_kt d={d} ldkt={ldkt} ldv={ldv}")
+    q, kt, v = _dsl_attn_inputs(n_q, n_k, d, d)
+    dq, do = hip.DeviceBuffer.from_array(q), hip.DeviceBuffer(n_q * d * 4)
+    dk = hip.DeviceBuffer(((d - 1) * ldkt + n_k) * 4)
+    dv = hip.DeviceBuffer(((n_k - 1) * ldv + d) * 4)
+    for buf, rows, ld in ((dk, kt, ldkt), (dv, v, ldv)):
+        for i, row in enumerate(np.ascontiguousarray(rows)):
+            hip.call("sile_hip_memcpy_htod", buf.ptr + i * ld * 4, row.ctypes.data, row.nbytes)
+    hip.attention_f32_kt(n_q, n_k, d, dq.ptr, d, dk.ptr, ldkt, dv.ptr, ldv, do.ptr, d, 0.5, -1e30)
+    hip.synchronize()
+    ref = cpuref.dsl_attention_f32(q, kt, v, n_k, 0.5, -1e30, d=d, n_q=n_q, s_k=n_k)
+    assert_close(do.download(np.float32, (n_q, d)), ref, atol=1e-5, rtol=1e-4, what="far pitches")
+    for b in (dq, dk, dv, do):
+        b.close()
+
+
 def test_attention_f32_kt_closed_forms(hip):
     """An initial max above every score gives 0 / 0 everywhere, as the
     program does; no keys gives 0 / 0 too."""
