@@ -1,5 +1,5 @@
 // Flash-attention forward on the gfx950 matrix cores, any sequence length,
-// head_dim a multiple of 16 up to 256.
+// head_dim a multiple of 8 up to 256.
 //
 //   O = softmax(Q K^T * scale [+ causal mask]) V     Q, K, V, O: [B*H, S, D] 16-bit
 //
@@ -61,7 +61,8 @@ struct AttnArgs {
   int32_t q_blocks;     // S / kBQ
   float scale_log2;     // softmax scale * log2(e)
   int32_t causal;
-  int32_t xcd_map;      // 1: head-per-XCD launch order (bh % 8 == 0)
+  int32_t xcd_map;      // head-per-XCD launch order (bh % 8 == 0): 1 a head's blocks together,
+                        // 2 the first unit of all the XCD's heads, then the second, ...
   int32_t pair;         // 1: causal query blocks in balanced pairs
 };
 
@@ -93,6 +94,21 @@ struct AttnArgs {
 // 16 cc + 8 + 4 g for k-group g = lane / 32) give the 8 slots whose keys are
 // exactly those P's accumulator rows hold for that k-group.
 //
+// Key groups: a launch of few query blocks leaves CUs idle, so the keys of a
+// block can be shared by kG = 2 or 4 groups of the workgroup's waves (head_dim
+// up to 128; 128 or 64 queries a workgroup).  Group kg takes key blocks kg,
+// kg + kG, ... with K and V stages of its own, all groups in step; at the end
+// groups 1 .. hand their (m, l, O) to group 0 through the same LDS, fp32.  The
+// price is that a tile is loaded for fewer queries (an iteration of the key
+// loop takes 0.72 - 0.95 us with one group, 0.95 - 1.35 with four), so the host
+// takes groups only where they fill CUs (flash_plan): B*H = 16, S = 1000,
+// D = 64, full: 21.4 us -> 11.2; 12 x 794 x 80 causal 32 -> 11.6; 8 x 4096 x 128
+// causal 106 -> 53.
+//
+// A head_dim that is an odd multiple of 8 has zeros in the upper half of its
+// last 16-dim step (both operands) and O^T rows past it that are not stored;
+// 2 x 2814 x 72 causal took 2355 us a query row a wave on the VALU and takes 22.
+//
 // LDS per stage: K and V [kNK][2 kDh B]; with 256-byte rows chunk c of row
 // r at c ^ (r & 15) (K) and c ^ 4 (r & 3) (V), with 128-byte rows at
 // c ^ ((r >> 1) & 7) and c ^ 2 (r & 3).
@@ -116,40 +132,51 @@ SILE_DEV float pair_sum(uint32_t pk, float acc) {
 
 // LDS bytes of the two stages (K and V tiles of kNK keys, rows of kDp
 // 16-bit elements each)
-template <int kNK, int kDp>
-constexpr int lds_bytes() { return 2 * 2 * kNK * 2 * kDp; }
+// for each key group; at least the (m, l, O) of the groups but one
+template <int kNK, int kDh, int kDp, int kW, int kG>
+constexpr int lds_bytes() {
+  const int stages = kG * 2 * 2 * kNK * 2 * kDp;
+  const int parts = (kG - 1) * (kW / kG) * (16 * ((kDh + 31) / 32) + 4) * 64 * 4;
+  return stages > parts ? stages : parts;
+}
 
-// kQT 32-query tiles per wave, kW waves per workgroup: kW * kQT * 32 queries
-// per workgroup (256 for every instantiation); kNK keys per block (32 or 64),
+// kQT 32-query tiles per wave, kW waves per workgroup in kG key groups:
+// kW / kG * kQT * 32 queries per workgroup (256, or 128 at kW = 4, with one); kNK keys per block (32 or 64),
 // i.e. kST = kNK / 32 S tiles of 32 keys x 32 queries per query tile.
-// kDh: the head dimension (a multiple of 16); kDp: the LDS row length (64,
+// kDh: the head dimension (a multiple of 8); kDp: the LDS row length (64,
 // 128 or 256 elements, at least kDh): the chunks of a row past kDh are
 // loaded as zeros (outside the buffer resources), so the products over them
 // add nothing and the O^T rows past kDh are zero and not stored.
-template <bool kBF16, int kQT, int kW, int kNK, int kDh, int kDp>
+template <bool kBF16, int kQT, int kW, int kNK, int kDh, int kDp, int kG>
 __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
                                             const uint16_t* __restrict__ K,
                                             const uint16_t* __restrict__ V,
                                             uint16_t* __restrict__ O, const AttnArgs& a,
-                                            uint8_t* smem) {
-  constexpr int kBQ = kW * kQT * 32;
+                                            uint8_t* smem_all) {
+  constexpr int kWG = kW / kG;           // waves sharing a key group's tiles
+  constexpr int kBQ = kWG * kQT * 32;
   constexpr int kST = kNK / 32;
   constexpr int kRow = 2 * kDp;          // bytes of a K or V row in LDS
   constexpr int kRowG = 2 * kDh;         // bytes of a K or V row in HBM
   constexpr int kChunks = kRow / 16;     // 16-byte chunks per LDS row
   constexpr int kChunksG = kRowG / 16;   // of them holding data
-  constexpr int kKK = kDh / 16;          // d-steps of S^T = K . Q^T
+  constexpr int kKK = (kDh + 15) / 16;   // d-steps of S^T = K . Q^T
   constexpr int kDT = (kDh + 31) / 32;   // 32-d tiles of O^T
   constexpr int kDmaRows = 1024 / kRow;  // rows one 1 KiB DMA instruction fills
-  static_assert(kDh % 16 == 0 && kDh <= kDp && (kDp == 64 || kDp == 128 || kDp == 256),
-                "head_dim a multiple of 16 up to the LDS row");
+  static_assert(kDh % 8 == 0 && kDh <= kDp && (kDp == 64 || kDp == 128 || kDp == 256),
+                "head_dim a multiple of 8 up to the LDS row");
+  static_assert(kG == 1 || kQT == 1, "key groups: one query tile a wave");
   constexpr int kTileB = kNK * kRow;     // one K or V tile
   constexpr int kStageB = 2 * kTileB;    // K + V
-  constexpr int kDmaPerWave = kTileB / 1024 / kW;  // 1 KiB DMA instructions per wave per tile
-  static_assert(kNK % 32 == 0 && kDmaPerWave >= 1 && (kTileB / 1024) % kW == 0,
+  constexpr int kDmaPerWave = kTileB / 1024 / kWG;  // 1 KiB DMA instructions per wave per tile
+  static_assert(kNK % 32 == 0 && kDmaPerWave >= 1 && (kTileB / 1024) % kWG == 0,
                 "tiles in 1 KiB slices, evenly over the waves");
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  // wave of its key group, and the group (0 when keys are not split)
+  const int wave = kG == 1 ? tid >> 6 : (tid >> 6) % kWG;
+  const int kg = kG == 1 ? 0 : __builtin_amdgcn_readfirstlane((tid >> 6) / kWG);
   const int g = lane >> 5, l32 = lane & 31;
+  uint8_t* const smem = smem_all + kg * 2 * kStageB;
 
   // Work unit u of a head: query block u, or with a.pair (causal) the pair of
   // query blocks (q_blocks - 1 - u, u), whose key ranges add up to the same
@@ -160,8 +187,10 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
   const int bid = blockIdx.x;
   if (a.xcd_map) {
     const int xcd = bid & 7, idx = bid >> 3;
-    bh = ((idx / units) << 3) + xcd;
-    u = idx % units;
+    const int heads = a.bh >> 3;   // of this XCD
+    const int hd = a.xcd_map == 1 ? idx / units : idx % heads;
+    bh = (hd << 3) + xcd;
+    u = a.xcd_map == 1 ? idx % units : idx / heads;
   } else {
     bh = bid % a.bh;
     u = bid / a.bh;
@@ -195,11 +224,16 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
       const int64_t qr = min((int64_t)(wq0 + qt * 32 + l32), S - 1);
       const uint16_t* qrow = Q + head_off + qr * kDh + 8 * g;
   #pragma unroll
-      for (int kk = 0; kk < kKK; ++kk) qf[qt][kk] = *reinterpret_cast<const u32x4*>(qrow + 16 * kk);
+      for (int kk = 0; kk < kKK; ++kk) {
+        if (16 * kk + 16 <= kDh)
+          qf[qt][kk] = *reinterpret_cast<const u32x4*>(qrow + 16 * kk);
+        else   // kDh % 16 == 8: the last step's upper 8 dims are zeros
+          qf[qt][kk] = g == 0 ? *reinterpret_cast<const u32x4*>(qrow + 16 * kk) : u32x4{0u, 0u, 0u, 0u};
+      }
     }
 
     // ---- LDS-DMA addressing: wave w's instruction i fills LDS rows
-    // kDmaRows (w + kW i) + lane / kChunks; lane l writes slot l % kChunks of
+    // kDmaRows (w + kWG i) + lane / kChunks; lane l writes slot l % kChunks of
     // its row, so it fetches the HBM chunk that belongs there under the
     // swizzle, or, for a chunk past the row's data, an offset past the
     // buffer (zeros) ----
@@ -207,7 +241,7 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
     int k_voff[kDmaPerWave], v_voff[kDmaPerWave];
   #pragma unroll
     for (int i = 0; i < kDmaPerWave; ++i) {
-      const int row = kDmaRows * (wave + kW * i) + lane / kChunks, pos = lane % kChunks;
+      const int row = kDmaRows * (wave + kWG * i) + lane / kChunks, pos = lane % kChunks;
       const int kc = pos ^ kswz(row), vc = pos ^ vswz(row);
       k_voff[i] = kc < kChunksG ? row * kRowG + kc * 16 : kv_bytes;
       v_voff[i] = vc < kChunksG ? row * kRowG + vc * 16 : kv_bytes;
@@ -220,15 +254,15 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
       uint8_t* base = smem + stage * kStageB + wave * 1024;
   #pragma unroll
       for (int i = 0; i < kDmaPerWave; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rsrc, (lds_ptr_t)(base + i * kW * 1024), 16,
-                                                 k_voff[i], blk * kNK * kRowG, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rsrc, (lds_ptr_t)(base + i * kWG * 1024), 16,
+                                                 k_voff[i], (blk * kG + kg) * kNK * kRowG, 0, 0);
     };
     auto dma_v = [&](int blk, int stage) {
       uint8_t* base = smem + stage * kStageB + kTileB + wave * 1024;
   #pragma unroll
       for (int i = 0; i < kDmaPerWave; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc, (lds_ptr_t)(base + i * kW * 1024), 16,
-                                                 v_voff[i], blk * kNK * kRowG, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc, (lds_ptr_t)(base + i * kWG * 1024), 16,
+                                                 v_voff[i], (blk * kG + kg) * kNK * kRowG, 0, 0);
     };
 
     // ---- fragment reads ----
@@ -339,7 +373,9 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
     // to even (the loop runs in pairs); keys past S load as zeros (outside
     // the K / V buffer resources) and are masked
     const int64_t kend = a.causal ? min((int64_t)(q0 + kBQ), S) : S;
-    int nb = (int)((kend + kNK - 1) / kNK);
+    // (with key groups, group kg takes blocks kg, kg + kG, ...: its block j is
+    // block j kG + kg, and the blocks past the last one are masked)
+    int nb = (int)((kend + kNK * kG - 1) / (kNK * kG));
     nb += nb & 1;
     const int last = nb - 1;
     const float c = a.scale_log2;
@@ -367,7 +403,7 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
                              u32x4 (&pnew)[kQT][2 * kST]) {
       constexpr bool kMasked = decltype(masked)::value;
       if constexpr (kMasked) {
-        const int kb = j * kNK;
+        const int kb = (j * kG + kg) * kNK;
   #pragma unroll
         for (int qt = 0; qt < kQT; ++qt) {
           // last key this lane's query sees: the query itself (causal) or S - 1
@@ -434,9 +470,11 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
   #pragma unroll
         for (int qt = 0; qt < kQT; ++qt) {
           const float m_new = grow_any ? __builtin_fmaxf(m_run[qt], mx[qt]) : m_run[qt];
-          const float alpha = exp2_fast((m_run[qt] - m_new) * c);
+          // a key group may have masked keys only so far: then every p is 0
+          const float m_use = kG > 1 && m_new == -__builtin_inff() ? 0.0f : m_new;
+          const float alpha = exp2_fast((m_run[qt] - m_use) * c);
           m_run[qt] = m_new;
-          const float mc = m_new * c;
+          const float mc = m_use * c;
           float rs = 0.0f;
   #pragma unroll
           for (int st = 0; st < kST; ++st)
@@ -472,7 +510,7 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
     // unneeded half of iterations jw and jw + 1 as well keeps registers of the
     // skipped branches live and spills.)
     const int jw = __builtin_amdgcn_readfirstlane(
-        (int)((a.causal ? min((int64_t)(wq0 + 32 * kQT - 1), S - 1) : S - 1) / kNK));
+        ((int)((a.causal ? min((int64_t)(wq0 + 32 * kQT - 1), S - 1) : S - 1) / kNK) + kG - kg) / kG - 1);
 
     // One iteration: everything up to the optional O rescale is one basic block,
     // so the scheduler interleaves the softmax VALU work of block j with the
@@ -496,7 +534,8 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
             for (int kk = 0; kk < kKK; ++kk) qf[qt][kk] = u32x4{0u, 0u, 0u, 0u};
         }
       }
-      if (!kMasked || j - 1 <= jw) {
+      // (a group without any block for this wave, jw = -1, has nothing to do)
+      if (!kMasked || (j - 1 <= jw && (kG == 1 || jw >= 0))) {
         // matrix cores: S_{j+1} and PV_{j-1}, interleaved step by step so that
         // consecutive MFMAs never accumulate into the same registers
         mma_block(kS ^ 1, kS ^ 1, snext, pprev, oacc);
@@ -513,7 +552,7 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
     };
     // blocks left of the workgroup's diagonal (causal) or of the block that
     // holds key S (S not a multiple of the block) need no mask
-    const int j_diag = a.causal ? q0 / kNK : (int)(S / kNK) & ~1;
+    const int j_diag = ((a.causal ? q0 / kNK : (int)(S / kNK)) / kG) & ~1;
     using Z = std::integral_constant<int, 0>;
     using One = std::integral_constant<int, 1>;
     int j = 0;
@@ -527,6 +566,53 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
     }
     // PV of the last block (nb is even: P_{nb-1} is in pprev, V_{nb-1} in stage 1)
     if (last <= jw) pv_block(1, pprev, oacc);
+
+    // ---- key groups: groups 1 .. hand (m, l, O) to group 0 through LDS ----
+    if constexpr (kG > 1) {
+      constexpr int kRegs = 16 * kDT;
+      __syncthreads();   // every read of the K and V stages is done
+      float* part = reinterpret_cast<float*>(smem_all);
+      auto slot = [&](int grp, int reg4) {   // 4 registers of a wave: 64 lanes x 16 bytes
+        return part + (((grp - 1) * kWG + wave) * (kRegs + 4) + 4 * reg4) * 64 + 4 * lane;
+      };
+      if (kg > 0) {
+  #pragma unroll
+        for (int t = 0; t < kRegs / 4; ++t) {
+          const f32x16& acc = oacc[0][t / 4];
+          const int e = 4 * (t % 4);
+          *reinterpret_cast<f32x4*>(slot(kg, t)) = f32x4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
+        }
+        *reinterpret_cast<f32x4*>(slot(kg, kRegs / 4)) = f32x4{m_run[0], l_run[0], 0.0f, 0.0f};
+      }
+      __syncthreads();
+      if (kg > 0) continue;
+      float mg[kG], lg[kG];
+      mg[0] = m_run[0];
+      lg[0] = l_run[0];
+      float m_all = mg[0];
+  #pragma unroll
+      for (int grp = 1; grp < kG; ++grp) {
+        const f32x4 w = *reinterpret_cast<const f32x4*>(slot(grp, kRegs / 4));
+        mg[grp] = w[0];
+        lg[grp] = w[1];
+        m_all = __builtin_fmaxf(m_all, mg[grp]);
+      }
+      const float w0 = exp2_fast((mg[0] - m_all) * c);
+      l_run[0] = lg[0] * w0;
+  #pragma unroll
+      for (int dt = 0; dt < kDT; ++dt) oacc[0][dt] *= w0;
+  #pragma unroll
+      for (int grp = 1; grp < kG; ++grp) {
+        const float w = exp2_fast((mg[grp] - m_all) * c);
+        l_run[0] += lg[grp] * w;
+  #pragma unroll
+        for (int t = 0; t < kRegs / 4; ++t) {
+          const f32x4 o4 = *reinterpret_cast<const f32x4*>(slot(grp, t));
+  #pragma unroll
+          for (int e = 0; e < 4; ++e) oacc[0][t / 4][4 * (t % 4) + e] += o4[e] * w;
+        }
+      }
+    }
 
     // ---- epilogue: O[q][d] = O^T[d][q] / l ----
   #pragma unroll
@@ -553,33 +639,53 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
 
 }  // namespace v2
 
-#define SILE_FA_V2_KERNEL(NAME, BF, QT, W, NK, DH, DP)                                        \
+#define SILE_FA_V2_KERNEL(NAME, BF, W, NK, DH, DP, G)                                         \
   extern "C" __global__ __launch_bounds__(W * 64, 1) void NAME(                               \
       const uint16_t* Q, const uint16_t* K, const uint16_t* V, uint16_t* O, AttnArgs a) {     \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[v2::lds_bytes<NK, DP>()];          \
-    v2::attn_fwd_v2<BF, QT, W, NK, DH, DP>(Q, K, V, O, a, smem);                              \
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[v2::lds_bytes<NK, DH, DP, W, G>()]; \
+    v2::attn_fwd_v2<BF, 1, W, NK, DH, DP, G>(Q, K, V, O, a, smem);                            \
   }
 // 8 waves x 32 queries (two waves per SIMD) for head_dim up to 128: 32-key
 // blocks over 256-byte LDS rows, 64-key blocks over 128-byte rows (the same
 // LDS bytes and MFMAs per block); 4 waves (one per SIMD, room for the O
 // accumulators) over 512-byte rows for head_dim up to 256.
-#define SILE_FA_V2_DTYPES(SUFFIX, W, NK, DH, DP)                                              \
-  SILE_FA_V2_KERNEL(sile_flash_attn_fwd_f16_##SUFFIX, false, 1, W, NK, DH, DP)                  \
-  SILE_FA_V2_KERNEL(sile_flash_attn_fwd_bf16_##SUFFIX, true, 1, W, NK, DH, DP)
-// every head dimension that is a multiple of 16 from 16 to 256
-SILE_FA_V2_DTYPES(v2w8_d16, 8, 64, 16, 64)
-SILE_FA_V2_DTYPES(v2w8_d32, 8, 64, 32, 64)
-SILE_FA_V2_DTYPES(v2w8_d48, 8, 64, 48, 64)
-SILE_FA_V2_DTYPES(v2w8_d64, 8, 64, 64, 64)
-SILE_FA_V2_DTYPES(v2w8_d80, 8, 32, 80, 128)
-SILE_FA_V2_DTYPES(v2w8_d96, 8, 32, 96, 128)
-SILE_FA_V2_DTYPES(v2w8_d112, 8, 32, 112, 128)
-SILE_FA_V2_DTYPES(v2w8, 8, 32, 128, 128)
-SILE_FA_V2_DTYPES(v2w4_d144, 4, 32, 144, 256)
-SILE_FA_V2_DTYPES(v2w4_d160, 4, 32, 160, 256)
-SILE_FA_V2_DTYPES(v2w4_d176, 4, 32, 176, 256)
-SILE_FA_V2_DTYPES(v2w4_d192, 4, 32, 192, 256)
-SILE_FA_V2_DTYPES(v2w4_d208, 4, 32, 208, 256)
-SILE_FA_V2_DTYPES(v2w4_d224, 4, 32, 224, 256)
-SILE_FA_V2_DTYPES(v2w4_d240, 4, 32, 240, 256)
-SILE_FA_V2_DTYPES(v2w4_d256, 4, 32, 256, 256)
+#define SILE_FA_V2_DTYPES(SUFFIX, W, NK, DH, DP, G)                                           \
+  SILE_FA_V2_KERNEL(sile_flash_attn_fwd_f16_##SUFFIX, false, W, NK, DH, DP, G)                 \
+  SILE_FA_V2_KERNEL(sile_flash_attn_fwd_bf16_##SUFFIX, true, W, NK, DH, DP, G)
+// up to 128: also with the keys in 2 or 4 groups of waves (128 or 64 queries)
+#define SILE_FA_V2_GROUPS(DH, NK, DP)                     \
+  SILE_FA_V2_DTYPES(v2w8_d##DH, 8, NK, DH, DP, 1)         \
+  SILE_FA_V2_DTYPES(v2w8_d##DH##_g2, 8, NK, DH, DP, 2)    \
+  SILE_FA_V2_DTYPES(v2w8_d##DH##_g4, 8, NK, DH, DP, 4)
+SILE_FA_V2_GROUPS(8, 64, 64)
+SILE_FA_V2_GROUPS(16, 64, 64)
+SILE_FA_V2_GROUPS(24, 64, 64)
+SILE_FA_V2_GROUPS(32, 64, 64)
+SILE_FA_V2_GROUPS(40, 64, 64)
+SILE_FA_V2_GROUPS(48, 64, 64)
+SILE_FA_V2_GROUPS(56, 64, 64)
+SILE_FA_V2_GROUPS(64, 64, 64)
+SILE_FA_V2_GROUPS(72, 32, 128)
+SILE_FA_V2_GROUPS(80, 32, 128)
+SILE_FA_V2_GROUPS(88, 32, 128)
+SILE_FA_V2_GROUPS(96, 32, 128)
+SILE_FA_V2_GROUPS(104, 32, 128)
+SILE_FA_V2_GROUPS(112, 32, 128)
+SILE_FA_V2_GROUPS(120, 32, 128)
+SILE_FA_V2_GROUPS(128, 32, 128)
+SILE_FA_V2_DTYPES(v2w4_d136, 4, 32, 136, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d144, 4, 32, 144, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d152, 4, 32, 152, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d160, 4, 32, 160, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d168, 4, 32, 168, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d176, 4, 32, 176, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d184, 4, 32, 184, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d192, 4, 32, 192, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d200, 4, 32, 200, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d208, 4, 32, 208, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d216, 4, 32, 216, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d224, 4, 32, 224, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d232, 4, 32, 232, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d240, 4, 32, 240, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d248, 4, 32, 248, 256, 1)
+SILE_FA_V2_DTYPES(v2w4_d256, 4, 32, 256, 256, 1)

@@ -130,6 +130,67 @@ GemmPlan gemm_plan(int64_t m, int64_t n, int64_t kp, int64_t half_steps, int64_t
   return best.splits > 1 && !(best_t < 0.95 * best_unsplit_t) ? best_unsplit : best;
 }
 
+// How the flash kernel's work is laid out: the keys of a query block shared by
+// `groups` groups of a workgroup's 8 waves (1, 2 or 4: 256, 128 or 64 queries a
+// workgroup; head_dim up to 128), and causal query blocks one by one or in
+// pairs of equal total length.
+struct FlashPlan {
+  int groups;
+  bool pair;
+  bool longest_first;   // unpaired causal: the longest blocks of all heads first
+};
+
+// The layout with the least modelled time.  A workgroup of 8 waves is alone on
+// its CU and takes `iters` rounds of one key block (32 keys; 64 up to head_dim
+// 64) a group, each tau us, and 5 us of prologue and epilogue a query block; a
+// launch is as long as its rounds of workgroups, unpaired causal ones (of
+// unequal length) 1.25 times the mean load of a CU or the longest block.  tau
+// grows with the groups, whose tiles are each loaded for fewer queries, and
+// with the share of CUs at work (the L2s' bandwidth and the clock).  Measured,
+// us a call with 1, 2, 4 groups: B*H = 16, S = 1000, D = 64, full: 22.3, 15.5,
+// 12.7; 8 x 4096 x 128 causal: 96, 59, 54 (in pairs 106, 64, 53); 32 x 1024 x
+// 128 causal: 32, 23, 31 (pairs 44, 30, 27); but 128 x 1024 x 128 causal in
+// pairs 56, 66, 102: where one group fills the CUs it stays the fastest.
+FlashPlan flash_plan(int64_t bh, int64_t seq, int head_dim, bool causal) {
+  FlashPlan best{1, causal, false};
+  int cus = 0;
+  if (head_dim > 128 || device_cus(&cus) != SILE_OK) return best;
+  const int64_t key_block = head_dim <= 64 ? 64 : 32;
+  double best_t = 1e30;
+  for (int g : {1, 2, 4}) {
+    const double lo = g == 1 ? 0.72 : g == 2 ? 0.82 : 0.95, hi = g == 1 ? 0.95 : g == 2 ? 1.1 : 1.35;
+    const int64_t q_blocks = (seq + 256 / g - 1) / (256 / g);
+    const double iters = (double)(((seq + key_block * g - 1) / (key_block * g) + 1) / 2 * 2);
+    const double merge = g == 1 ? 0.0 : g == 2 ? 0.5 : 1.5;
+    auto tau = [&](double busy) { return lo + (hi - lo) * std::min(1.0, busy / cus); };
+    for (bool pair : {true, false}) {
+      if (pair && !causal) continue;
+      const int64_t wgs = bh * (pair ? (q_blocks + 1) / 2 : q_blocks);
+      double t;
+      if (pair) {
+        const double two = q_blocks > 1 ? iters * (1.0 + 1.0 / (double)q_blocks) : iters;
+        t = (double)((wgs + cus - 1) / cus) *
+            (tau((double)wgs) * two + (5.0 + merge) * (q_blocks > 1 ? 2 : 1));
+      } else if (causal) {
+        const double each = tau(0.5 * (double)wgs), mean = 0.5 * (iters + 2);
+        t = std::max(each * iters + 5.0 + merge,
+                     1.25 * (double)wgs * (each * mean + 5.0 + merge) / cus);
+      } else {
+        t = (double)((wgs + cus - 1) / cus) * (tau((double)wgs) * iters + 5.0 + merge);
+      }
+      if (t < best_t) {
+        best_t = t;
+        best.groups = g;
+        best.pair = pair;
+      }
+    }
+  }
+  // the heads of an XCD (B*H a multiple of 8) have their K and V in its 4 MiB
+  // L2: their blocks may run in any order
+  best.longest_first = causal && !best.pair && bh / 8 * seq * head_dim * 4 <= (4ll << 20);
+  return best;
+}
+
 // fp32 -> 16-bit element bits, round to nearest even (NaN stays a quiet NaN),
 // for fill values converted on the host.
 uint32_t bf16_bits_rne(float f) {
@@ -1015,22 +1076,18 @@ int sile_hip_flash_attn_fwd(sile_dtype dtype, int64_t batch, int64_t heads, int6
     return fail(SILE_ERR_SHAPE, "sequence too long for one head (S=%lld)", (long long)seq_len);
 
   // MFMA flash kernel, 16-byte aligned operands, any S: the pipelined kernel
-  // (32-query waves, key blocks through LDS-DMA; causal query blocks taken
-  // in balanced pairs; keys and queries past S masked), one instantiation
-  // per head dimension (a multiple of 16 up to 256): 8 waves up to 128
-  // (32-key blocks, or 64-key blocks over 128-byte rows up to 64), 4 waves
-  // past 128.
+  // (32-query waves, key blocks through LDS-DMA; keys and queries past S
+  // masked; laid out by flash_plan), one instantiation per head dimension (a
+  // multiple of 8 up to 256) and key group count: 8 waves up to 128 (32-key
+  // blocks, or 64-key blocks over 128-byte rows up to 64), 4 waves past 128.
   const bool aligned = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o);
-  if (head_dim % 16 == 0 && head_dim >= 16 && head_dim <= 256 && aligned) {
+  if (head_dim % 8 == 0 && aligned) {
     const char* dt = dtype == SILE_F16 ? "f16" : "bf16";
     const int waves = head_dim <= 128 ? 8 : 4;
-    char suffix[32];
-    if (head_dim == 128)
-      snprintf(suffix, sizeof suffix, "v2w8");
-    else
-      snprintf(suffix, sizeof suffix, "v2w%d_d%d", waves, (int)head_dim);
-    const int64_t bq = 32 * waves;
-    const bool pair = causal;
+    const FlashPlan plan = flash_plan(bh, seq_len, (int)head_dim, causal != 0);
+    const int groups = plan.groups;
+    const int64_t bq = 32 * waves / groups;
+    const bool pair = plan.pair;
     const int64_t q_blocks = (seq_len + bq - 1) / bq;
     if (q_blocks > 0x7fffffffLL / std::max<int64_t>(bh, 1))
       return fail(SILE_ERR_SHAPE, "attention too large");
@@ -1040,11 +1097,12 @@ int sile_hip_flash_attn_fwd(sile_dtype dtype, int64_t batch, int64_t heads, int6
       float scale_log2;
       int32_t causal, xcd_map, pair;
     } fa{seq_len, (int32_t)bh, (int32_t)q_blocks, scale * 1.4426950408889634f,
-         causal ? 1 : 0, (bh % 8 == 0) ? 1 : 0, pair ? 1 : 0};
+         causal ? 1 : 0, (bh % 8 == 0) ? (plan.longest_first ? 2 : 1) : 0, pair ? 1 : 0};
     const int64_t units = pair ? (q_blocks + 1) / 2 : q_blocks;
     const int64_t blocks = bh * units;
     char name[64];
-    snprintf(name, sizeof name, "sile_flash_attn_fwd_%s_%s", dt, suffix);
+    int len = snprintf(name, sizeof name, "sile_flash_attn_fwd_%s_v2w%d_d%d", dt, waves, (int)head_dim);
+    if (groups > 1) snprintf(name + len, sizeof name - len, "_g%d", groups);
     const unsigned threads = 64 * waves;
     void* params[] = {(void*)&q, (void*)&k, (void*)&v, &o, &fa};
     int rc = launch(Module::kFlashAttn, name, dim3((unsigned)blocks), dim3(threads), params, s);

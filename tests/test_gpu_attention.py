@@ -292,6 +292,58 @@ def test_flash_many_work_items(hip, dt, causal, b, h, s, d):
         assert_close(got[bi, hi], ref, atol=ATOL, rtol=RTOL, what=f"attn b{bi} h{hi}")
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("d", [8, 24, 40, 56, 72, 88, 104, 120, 136, 200, 248])
+@pytest.mark.parametrize("s", [33, 777])
+def test_flash_head_dims_of_8(hip, dt, causal, d, s):
+    """Head dimensions that are odd multiples of 8: the last 16-dim step of
+    Q K^T and the last O^T tile are half zeros."""
+    b, h = 1, 3
+    say(f"flash D={d} {dt} causal={causal} S={s}")
+    scale = 1.0 / np.sqrt(d)
+    qkv = _inputs(b, h, s, d, dt, seed=63 + d)
+    got = _run(hip, dt, b, h, s, d, [x[0] for x in qkv], causal, scale)
+    qf, kf, vf = (x[1] for x in qkv)
+    for hi in range(h):
+        ref = cpuref.attention_fwd(qf[0, hi], kf[0, hi], vf[0, hi], scale, causal=causal)
+        assert_close(got[0, hi], ref, atol=ATOL, rtol=RTOL, what=f"D={d} h{hi}")
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("trend", ["flat", "rising"])
+@pytest.mark.parametrize("causal,h,s,d", [
+    (False, 8, 33, 128), (True, 8, 97, 96),      # 2 groups, one with no key for some queries
+    (True, 8, 5, 64), (False, 3, 1, 40),
+    (True, 40, 520, 128), (False, 32, 700, 128),  # 2 groups, ragged ends; longest blocks first
+    (True, 32, 1100, 64),
+    (True, 32, 2048, 80),                         # 2 groups in pairs
+    (True, 8, 1500, 128), (False, 16, 1000, 64),  # 4 groups
+    (True, 8, 4096, 64),                          # 4 groups, long
+    (True, 128, 300, 72), (False, 128, 300, 64),  # one group
+    (True, 256, 384, 128)])
+def test_flash_key_groups(hip, dt, trend, causal, h, s, d):
+    """The layouts the plan picks by shape: a query block's keys in 1, 2 or 4
+    groups of waves merged through LDS, causal blocks paired or one by one.
+    rising: later keys raise the running max past the lazy margin, so the
+    groups end at different maxima."""
+    say(f"flash groups {dt} {trend} causal={causal} H={h} S={s} D={d}")
+    scale = 1.0 / np.sqrt(d)
+    r = rng(s + d)
+    q, k, v = (r.normal(size=(1, h, s, d)).astype(np.float32) for _ in range(3))
+    if trend == "rising":
+        q += 1.0
+        k += 2.0 * np.linspace(0.0, 1.0, s, dtype=np.float32)[None, None, :, None]
+    rnd = f16_round if dt == "f16" else bf16_round
+    qkv = [rnd(x) for x in (q, k, v)]
+    got = _run(hip, dt, 1, h, s, d, [x[0] for x in qkv], causal, scale)
+    assert np.isfinite(got).all()
+    qf, kf, vf = (x[1] for x in qkv)
+    for hi in sorted({0, 7, h // 2, h - 1} & set(range(h))):
+        ref = cpuref.attention_fwd(qf[0, hi], kf[0, hi], vf[0, hi], scale, causal=causal)
+        assert_close(got[0, hi], ref, atol=ATOL, rtol=RTOL, what=f"h{hi}")
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_flash_long_sequence(hip, causal):
     """S = 65536 (B = 1, H = 8, D = 128, f16): block, key and byte offsets at
