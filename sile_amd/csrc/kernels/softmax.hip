@@ -16,11 +16,10 @@
 //    the fastest copy measured on the device; the row max and sum are wave
 //    all-reductions plus one exchange of per-wave partials through LDS;
 //  * other widths: kL lanes per row for rows of up to 32 chunks (4..32 rows
-//    per wave), one wave per row with the row in registers (whole chunks, or
-//    a masked last chunk) up to 8192, one row per 1024-thread workgroup with
-//    a masked last chunk up to 1024 * 8 chunks, two passes over the row by
-//    one workgroup beyond that; a three-pass element-wise kernel when the
-//    rows are not 16-byte aligned.
+//    per wave, four times as many in flight in large launches), a wave a row up
+//    to 256 chunks, then a workgroup a row with the row in registers up to
+//    65536 elements, two passes over the row by one workgroup beyond that.
+// Rows may start at any element: the 128-bit accesses need no alignment.
 // Wave all-reductions use DPP row permutes (common.h); exp(x - m) is
 // 2^((x - m) * log2 e) on v_exp_f32.
 #include "common.h"
@@ -29,29 +28,34 @@ using namespace sile;
 
 enum DType : int { kF32 = 0, kF16 = 1, kBF16 = 2 };
 
+// 16 bytes at any element address: rows of any pitch and start take the
+// 128-bit accesses (the memory pipeline takes unaligned ones).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
 template <int kT>
 struct Elem;
 template <>
 struct Elem<kF32> {
   using Storage = float;
   SILE_DEV static void load8(const float* p, float v[8]) {
-    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
-    const f32x4 b = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p + 4));
+    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(p));
+    const f32x4 b = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(p + 4));
     v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3];
     v[4] = b[0]; v[5] = b[1]; v[6] = b[2]; v[7] = b[3];
   }
   SILE_DEV static void store8(float* p, const float v[8]) {
     f32x4 a = {v[0], v[1], v[2], v[3]}, b = {v[4], v[5], v[6], v[7]};
-    __builtin_nontemporal_store(a, reinterpret_cast<f32x4*>(p));
-    __builtin_nontemporal_store(b, reinterpret_cast<f32x4*>(p + 4));
+    __builtin_nontemporal_store(a, reinterpret_cast<f32x4_any*>(p));
+    __builtin_nontemporal_store(b, reinterpret_cast<f32x4_any*>(p + 4));
   }
   SILE_DEV static void load4(const float* p, float v[4]) {
-    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(p));
     v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3];
   }
   SILE_DEV static void store4(float* p, const float v[4]) {
     f32x4 a = {v[0], v[1], v[2], v[3]};
-    __builtin_nontemporal_store(a, reinterpret_cast<f32x4*>(p));
+    __builtin_nontemporal_store(a, reinterpret_cast<f32x4_any*>(p));
   }
   SILE_DEV static float load1(const float* p) { return *p; }
   SILE_DEV static void store1(float* p, float v) { *p = v; }
@@ -60,7 +64,7 @@ template <>
 struct Elem<kF16> {
   using Storage = uint16_t;
   SILE_DEV static void load8(const uint16_t* p, float v[8]) {
-    const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+    const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       // copy the element out first: hipcc's __builtin_bit_cast of an
@@ -75,7 +79,7 @@ struct Elem<kF16> {
     u32x4 w;
 #pragma unroll
     for (int i = 0; i < 4; ++i) w[i] = pack_f16x2(v[2 * i], v[2 * i + 1]);
-    __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p));
+    __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any*>(p));
   }
   SILE_DEV static float load1(const uint16_t* p) { return f16_to_f32(*p); }
   SILE_DEV static void store1(uint16_t* p, float v) { *p = f16_rne(v); }
@@ -84,7 +88,7 @@ template <>
 struct Elem<kBF16> {
   using Storage = uint16_t;
   SILE_DEV static void load8(const uint16_t* p, float v[8]) {
-    const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+    const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       v[2 * i] = bits_f32(w[i] << 16);
@@ -95,7 +99,7 @@ struct Elem<kBF16> {
     u32x4 w;
 #pragma unroll
     for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-    __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p));
+    __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any*>(p));
   }
   SILE_DEV static float load1(const uint16_t* p) { return bf16_to_f32(*p); }
   SILE_DEV static void store1(uint16_t* p, float v) { *p = bf16_rne(v); }
@@ -137,179 +141,124 @@ SILE_DEV float normalise(float e, float s, float inv) {
     return e * inv;
 }
 
-// ---- register-resident row softmax: cols == kChunks * 64 * chunk_elems ----
-template <int kIn, int kOut, int kChunks>
-__device__ __forceinline__ void softmax_row_regs(const typename Elem<kIn>::Storage* __restrict__ xr,
-                                                 typename Elem<kOut>::Storage* __restrict__ yr,
-                                                 int lane) {
+// ---- row softmax in registers: kT threads a row, kC chunks a thread ----
+// Chunk j of thread t at column (j * kT + t) * E.  kT = 64: a wave a row, four
+// rows a workgroup; kT = 256, 512, 1024: a workgroup a row, its wave maxima and
+// sums exchanged through LDS.  The host takes the kC that covers the row (at
+// most one chunk more past 8), so only the last chunks can pass its end: the
+// chunk the row ends in is moved back to end there, its elements that the
+// chunk before it holds left out of the sum and stored twice with the same
+// value, and chunks past the row are -inf (exp 0) and not stored.  Every load
+// is issued before the first value is used, and every load of a row before its
+// first store.  HBM-bound: fp32
+// 4097 x 3001 (odd pitch) ran three element-wise passes in 53 us before these
+// shapes took unaligned rows, 16-bit 4096 x 6000 29.7 us with a wave a row.
+template <int kIn, int kOut, int kT, int kC>
+__device__ __forceinline__ void softmax_rows_tile_kernel(const void* x, void* y, int64_t rows,
+                                                         int64_t cols, int64_t ldx,
+                                                         int64_t ldy) {
   constexpr int kE = chunk_elems<kIn, kOut>();
-  float v[kChunks][kE];
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j) load_chunk<kIn, kE>(xr + (j * 64 + lane) * kE, v[j]);
-  float m = -__builtin_inff();
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j)
-#pragma unroll
-    for (int i = 0; i < kE; ++i) m = fmax_ordered(m, v[j][i]);
-  m = wave_max(m);
-  float s = 0.0f;
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j)
-#pragma unroll
-    for (int i = 0; i < kE; ++i) {
-      v[j][i] = exp2_fast((v[j][i] - m) * kLog2e);
-      s += v[j][i];
-    }
-  s = wave_sum(s);
-  const float inv = 1.0f / s;
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j) {
-#pragma unroll
-    for (int i = 0; i < kE; ++i) v[j][i] = normalise<kOut>(v[j][i], s, inv);
-    store_chunk<kOut, kE>(yr + (j * 64 + lane) * kE, v[j]);
-  }
-}
-
-// ---- register-resident row softmax of any width up to kChunks * 64 * E ----
-// Chunks wholly inside the row are 128-bit accesses; the one chunk the row
-// ends in is read and written element by element; positions past the row are
-// -inf (exp 0) and never stored.
-template <int kIn, int kOut, int kChunks>
-__device__ __forceinline__ void softmax_row_masked(const typename Elem<kIn>::Storage* __restrict__ xr,
-                                                   typename Elem<kOut>::Storage* __restrict__ yr,
-                                                   int lane, int cols) {
-  constexpr int kE = chunk_elems<kIn, kOut>();
-  float v[kChunks][kE];
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j) {
-    const int c0 = (j * 64 + lane) * kE;
-    if (c0 + kE <= cols) {
-      load_chunk<kIn, kE>(xr + c0, v[j]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < kE; ++i)
-        v[j][i] = c0 + i < cols ? Elem<kIn>::load1(xr + c0 + i) : -__builtin_inff();
-    }
-  }
-  float m = -__builtin_inff();
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j)
-#pragma unroll
-    for (int i = 0; i < kE; ++i) m = fmax_ordered(m, v[j][i]);
-  m = wave_max(m);
-  float s = 0.0f;
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j)
-#pragma unroll
-    for (int i = 0; i < kE; ++i) {
-      v[j][i] = exp2_fast((v[j][i] - m) * kLog2e);  // -inf -> 0
-      s += v[j][i];
-    }
-  s = wave_sum(s);
-  const float inv = 1.0f / s;
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j) {
-    const int c0 = (j * 64 + lane) * kE;
-#pragma unroll
-    for (int i = 0; i < kE; ++i) v[j][i] = normalise<kOut>(v[j][i], s, inv);
-    if (c0 + kE <= cols) {
-      store_chunk<kOut, kE>(yr + c0, v[j]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < kE; ++i)
-        if (c0 + i < cols) Elem<kOut>::store1(yr + c0 + i, v[j][i]);
-    }
-  }
-}
-
-template <int kIn, int kOut, int kChunks>
-__device__ __forceinline__ void softmax_rows_masked_kernel(const void* x, void* y, int64_t rows,
-                                                           int64_t cols, int64_t ldx,
-                                                           int64_t ldy) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  using TI = typename Elem<kIn>::Storage;
-  using TO = typename Elem<kOut>::Storage;
-  softmax_row_masked<kIn, kOut, kChunks>(static_cast<const TI*>(x) + row * ldx,
-                                         static_cast<TO*>(y) + row * ldy, lane, (int)cols);
-}
-
-template <int kIn, int kOut, int kChunks>
-__device__ __forceinline__ void softmax_rows_regs_kernel(const void* x, void* y, int64_t rows,
-                                                         int64_t ldx, int64_t ldy) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  using TI = typename Elem<kIn>::Storage;
-  using TO = typename Elem<kOut>::Storage;
-  softmax_row_regs<kIn, kOut, kChunks>(static_cast<const TI*>(x) + row * ldx,
-                                       static_cast<TO*>(y) + row * ldy, lane);
-}
-
-// ---- any width: three passes over the row (L2-resident after the first) ----
-template <int kIn, int kOut>
-__device__ __forceinline__ void softmax_rows_generic_kernel(const void* x, void* y, int64_t rows,
-                                                            int64_t cols, int64_t ldx,
-                                                            int64_t ldy) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  constexpr int kWaves = kT / 64;
+  constexpr int kWhole = kC - (kC > 8 ? 2 : 1);   // chunks inside the row for every thread
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int t = kT == 64 ? lane : threadIdx.x;
+  const int64_t row = kT == 64 ? (int64_t)blockIdx.x * 4 + wave : blockIdx.x;
   if (row >= rows) return;
   using TI = typename Elem<kIn>::Storage;
   using TO = typename Elem<kOut>::Storage;
   const TI* xr = static_cast<const TI*>(x) + row * ldx;
   TO* yr = static_cast<TO*>(y) + row * ldy;
+  const int n = (int)cols;
+  float v[kC][kE];
+#pragma unroll
+  for (int j = 0; j < kC; ++j) {
+    const int c0 = (j * kT + t) * kE;
+    if (j < kWhole) {
+      load_chunk<kIn, kE>(xr + c0, v[j]);
+    } else if (c0 < n) {
+      load_chunk<kIn, kE>(xr + min(c0, n - kE), v[j]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kE; ++i) v[j][i] = -__builtin_inff();
+    }
+  }
   float m = -__builtin_inff();
-  for (int64_t c = lane; c < cols; c += 64) m = fmax_ordered(m, Elem<kIn>::load1(xr + c));
+#pragma unroll
+  for (int j = 0; j < kC; ++j)
+#pragma unroll
+    for (int i = 0; i < kE; ++i) m = fmax_ordered(m, v[j][i]);
   m = wave_max(m);
+  __shared__ float part[2][kWaves];
+  if constexpr (kT > 64) {
+    if (lane == 0) part[0][wave] = m;
+    __syncthreads();
+    m = part[0][0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) m = fmax_ordered(m, part[0][w]);
+  }
   float s = 0.0f;
-  for (int64_t c = lane; c < cols; c += 64) s += exp2_fast((Elem<kIn>::load1(xr + c) - m) * kLog2e);
+#pragma unroll
+  for (int j = 0; j < kC; ++j) {
+    const int twice = j < kWhole ? 0 : (j * kT + t + 1) * kE - n;   // elements moved back over
+#pragma unroll
+    for (int i = 0; i < kE; ++i) {
+      v[j][i] = exp2_fast((v[j][i] - m) * kLog2e);   // -inf -> 0
+      s += j < kWhole || i >= twice ? v[j][i] : 0.0f;
+    }
+  }
   s = wave_sum(s);
+  if constexpr (kT > 64) {
+    if (lane == 0) part[1][wave] = s;
+    __syncthreads();
+    s = part[1][0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) s += part[1][w];
+  }
   const float inv = 1.0f / s;
-  for (int64_t c = lane; c < cols; c += 64)
-    Elem<kOut>::store1(
-        yr + c, normalise<kOut>(exp2_fast((Elem<kIn>::load1(xr + c) - m) * kLog2e), s, inv));
+#pragma unroll
+  for (int j = 0; j < kC; ++j) {
+    const int c0 = (j * kT + t) * kE;
+#pragma unroll
+    for (int i = 0; i < kE; ++i) v[j][i] = normalise<kOut>(v[j][i], s, inv);
+    if (j < kWhole)
+      store_chunk<kOut, kE>(yr + c0, v[j]);
+    else if (c0 < n)
+      store_chunk<kOut, kE>(yr + min(c0, n - kE), v[j]);
+  }
 }
 
-#define SILE_SOFTMAX_REGS(NAME, IN, OUT, CH)                                                 \
-  extern "C" __global__ __launch_bounds__(256) void NAME(const void* x, void* y, int64_t rows, \
-                                                         int64_t ldx, int64_t ldy) {         \
-    softmax_rows_regs_kernel<IN, OUT, CH>(x, y, rows, ldx, ldy);                             \
+#define SILE_SOFTMAX_TILE(TAG, IN, OUT, T, CH)                                                 \
+  extern "C" __global__ __launch_bounds__(T < 256 ? 256 : T)                                   \
+      void sile_softmax_rows_##TAG##_t##T##c##CH(const void* x, void* y, int64_t rows,         \
+                                                 int64_t cols, int64_t ldx, int64_t ldy) {     \
+    softmax_rows_tile_kernel<IN, OUT, T, CH>(x, y, rows, cols, ldx, ldy);                      \
   }
-#define SILE_SOFTMAX_WIDTHS(TAG, IN, OUT)                      \
-  SILE_SOFTMAX_REGS(sile_softmax_rows_##TAG##_c1, IN, OUT, 1)   \
-  SILE_SOFTMAX_REGS(sile_softmax_rows_##TAG##_c2, IN, OUT, 2)   \
-  SILE_SOFTMAX_REGS(sile_softmax_rows_##TAG##_c4, IN, OUT, 4)   \
-  SILE_SOFTMAX_REGS(sile_softmax_rows_##TAG##_c8, IN, OUT, 8)   \
-  SILE_SOFTMAX_REGS(sile_softmax_rows_##TAG##_c16, IN, OUT, 16) \
-  extern "C" __global__ __launch_bounds__(256) void sile_softmax_rows_##TAG##_any(          \
-      const void* x, void* y, int64_t rows, int64_t cols, int64_t ldx, int64_t ldy) {      \
-    softmax_rows_generic_kernel<IN, OUT>(x, y, rows, cols, ldx, ldy);                      \
-  }
-
-SILE_SOFTMAX_WIDTHS(f16_f16, kF16, kF16)
-SILE_SOFTMAX_WIDTHS(bf16_bf16, kBF16, kBF16)
-SILE_SOFTMAX_WIDTHS(f32_f32, kF32, kF32)
-SILE_SOFTMAX_REGS(sile_softmax_rows_f32_f32_c32, kF32, kF32, 32)
-SILE_SOFTMAX_WIDTHS(f16_f32, kF16, kF32)
-
-#define SILE_SOFTMAX_MASKED(NAME, IN, OUT, CH)                                                 \
-  extern "C" __global__ __launch_bounds__(256) void NAME(const void* x, void* y, int64_t rows,   \
-                                                         int64_t cols, int64_t ldx, int64_t ldy) { \
-    softmax_rows_masked_kernel<IN, OUT, CH>(x, y, rows, cols, ldx, ldy);                         \
-  }
-#define SILE_SOFTMAX_MASKED_WIDTHS(TAG, IN, OUT)                  \
-  SILE_SOFTMAX_MASKED(sile_softmax_rows_##TAG##_m1, IN, OUT, 1)   \
-  SILE_SOFTMAX_MASKED(sile_softmax_rows_##TAG##_m2, IN, OUT, 2)   \
-  SILE_SOFTMAX_MASKED(sile_softmax_rows_##TAG##_m4, IN, OUT, 4)   \
-  SILE_SOFTMAX_MASKED(sile_softmax_rows_##TAG##_m8, IN, OUT, 8)   \
-  SILE_SOFTMAX_MASKED(sile_softmax_rows_##TAG##_m16, IN, OUT, 16)
-SILE_SOFTMAX_MASKED_WIDTHS(f16_f16, kF16, kF16)
-SILE_SOFTMAX_MASKED_WIDTHS(bf16_bf16, kBF16, kBF16)
-SILE_SOFTMAX_MASKED_WIDTHS(f32_f32, kF32, kF32)
-SILE_SOFTMAX_MASKED(sile_softmax_rows_f32_f32_m32, kF32, kF32, 32)
-SILE_SOFTMAX_MASKED_WIDTHS(f16_f32, kF16, kF32)
-
+#define SILE_SOFTMAX_TILES(TAG, IN, OUT)     \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 64, 1)     \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 64, 2)     \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 64, 3)     \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 64, 4)     \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 256, 2)    \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 256, 3)    \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 256, 4)    \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 512, 3)    \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 512, 4)    \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 512, 5)    \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 512, 6)    \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 1024, 4)   \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 1024, 5)   \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 1024, 6)   \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 1024, 7)   \
+  SILE_SOFTMAX_TILE(TAG, IN, OUT, 1024, 8)
+SILE_SOFTMAX_TILES(f16_f16, kF16, kF16)
+SILE_SOFTMAX_TILES(bf16_bf16, kBF16, kBF16)
+SILE_SOFTMAX_TILES(f32_f32, kF32, kF32)
+SILE_SOFTMAX_TILES(f16_f32, kF16, kF32)
+// (4-element chunks: 64 values a thread at 16)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 10)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 12)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 14)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 16)
 
 // ---- one row per workgroup: cols == kThreads * kChunks * E ----
 // The copy shape that moves the most bytes on MI355X (two 16-byte chunks per
@@ -409,141 +358,86 @@ SILE_DEV float group_sum(float v) {
   return v;
 }
 
-template <int kIn, int kOut, int kL>
+// kR rows a group of lanes, every load before the first value is used: with one
+// row a launch of many rows has too few bytes in flight (f16 65536 x 100: 10 us).
+// The chunk a row ends in is moved back to end there, as in the tile kernel;
+// rows shorter than a chunk go element by element.
+template <int kIn, int kOut, int kL, int kR>
 __device__ __forceinline__ void softmax_rows_narrow_kernel(const void* x, void* y, int64_t rows,
                                                            int64_t cols, int64_t ldx,
                                                            int64_t ldy) {
   static_assert(kL == 4 || kL == 8 || kL == 16 || kL == 32, "lanes per row");
   constexpr int kE = chunk_elems<kIn, kOut>();
+  constexpr int kWaveRows = 64 / kL;
   const int lane = threadIdx.x & 63, li = lane % kL;
-  const int64_t row = (int64_t)blockIdx.x * (256 / kL) + (threadIdx.x >> 6) * (64 / kL) + lane / kL;
-  const bool live = row < rows;
+  const int64_t row0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (kWaveRows * kR) + lane / kL;
   using TI = typename Elem<kIn>::Storage;
   using TO = typename Elem<kOut>::Storage;
-  const int c0 = li * kE;
-  float v[kE];
-  if (live && c0 + kE <= cols) {
-    load_chunk<kIn, kE>(static_cast<const TI*>(x) + row * ldx + c0, v);
-  } else {
+  const int n = (int)cols, c0 = li * kE, at = min(c0, n - kE), twice = c0 + kE - n;
+  float v[kR][kE];
 #pragma unroll
-    for (int i = 0; i < kE; ++i)
-      v[i] = live && c0 + i < cols ? Elem<kIn>::load1(static_cast<const TI*>(x) + row * ldx + c0 + i)
-                                   : -__builtin_inff();
+  for (int r = 0; r < kR; ++r) {
+    const int64_t row = row0 + r * kWaveRows;
+    const bool live = row < rows && c0 < n;
+    const TI* xr = static_cast<const TI*>(x) + (row < rows ? row : 0) * ldx;
+    if (live && n >= kE) {
+      load_chunk<kIn, kE>(xr + at, v[r]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kE; ++i)
+        v[r][i] = live && c0 + i < n ? Elem<kIn>::load1(xr + c0 + i) : -__builtin_inff();
+    }
   }
-  float m = -__builtin_inff();
 #pragma unroll
-  for (int i = 0; i < kE; ++i) m = fmax_ordered(m, v[i]);
-  m = group_max<kL>(m);
-  float s = 0.0f;
+  for (int r = 0; r < kR; ++r) {
+    const int64_t row = row0 + r * kWaveRows;
+    float m = -__builtin_inff();
 #pragma unroll
-  for (int i = 0; i < kE; ++i) {
-    v[i] = exp2_fast((v[i] - m) * kLog2e);   // -inf -> 0
-    s += v[i];
-  }
-  s = group_sum<kL>(s);
-  if (!live) return;
-  const float inv = 1.0f / s;
+    for (int i = 0; i < kE; ++i) m = fmax_ordered(m, v[r][i]);
+    m = group_max<kL>(m);
+    float s = 0.0f;
 #pragma unroll
-  for (int i = 0; i < kE; ++i) v[i] = normalise<kOut>(v[i], s, inv);
-  TO* yr = static_cast<TO*>(y) + row * ldy;
-  if (c0 + kE <= cols) {
-    store_chunk<kOut, kE>(yr + c0, v);
-  } else {
+    for (int i = 0; i < kE; ++i) {
+      v[r][i] = exp2_fast((v[r][i] - m) * kLog2e);   // -inf -> 0
+      s += i >= twice || n < kE ? v[r][i] : 0.0f;
+    }
+    s = group_sum<kL>(s);
+    if (row >= rows || c0 >= n) continue;   // (no lane exchanges below)
+    const float inv = 1.0f / s;
 #pragma unroll
-    for (int i = 0; i < kE; ++i)
-      if (c0 + i < cols) Elem<kOut>::store1(yr + c0 + i, v[i]);
+    for (int i = 0; i < kE; ++i) v[r][i] = normalise<kOut>(v[r][i], s, inv);
+    TO* yr = static_cast<TO*>(y) + row * ldy;
+    if (n >= kE) {
+      store_chunk<kOut, kE>(yr + at, v[r]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kE; ++i)
+        if (c0 + i < n) Elem<kOut>::store1(yr + c0 + i, v[r][i]);
+    }
   }
 }
 
-#define SILE_SOFTMAX_NARROW(NAME, IN, OUT, L)                                                    \
+#define SILE_SOFTMAX_NARROW(NAME, IN, OUT, L, R)                                                 \
   extern "C" __global__ __launch_bounds__(256) void NAME(const void* x, void* y, int64_t rows,   \
                                                          int64_t cols, int64_t ldx, int64_t ldy) { \
-    softmax_rows_narrow_kernel<IN, OUT, L>(x, y, rows, cols, ldx, ldy);                          \
+    softmax_rows_narrow_kernel<IN, OUT, L, R>(x, y, rows, cols, ldx, ldy);                       \
   }
-#define SILE_SOFTMAX_NARROW_WIDTHS(TAG, IN, OUT)                 \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n4, IN, OUT, 4)   \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n8, IN, OUT, 8)   \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n16, IN, OUT, 16) \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n32, IN, OUT, 32)
+#define SILE_SOFTMAX_NARROW_WIDTHS(TAG, IN, OUT)                       \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n4, IN, OUT, 4, 1)     \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n8, IN, OUT, 8, 1)     \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n16, IN, OUT, 16, 1)   \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n32, IN, OUT, 32, 1)   \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n4r4, IN, OUT, 4, 4)   \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n8r4, IN, OUT, 8, 4)   \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n16r4, IN, OUT, 16, 4) \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n32r4, IN, OUT, 32, 4)
 SILE_SOFTMAX_NARROW_WIDTHS(f16_f16, kF16, kF16)
 SILE_SOFTMAX_NARROW_WIDTHS(bf16_bf16, kBF16, kBF16)
 SILE_SOFTMAX_NARROW_WIDTHS(f32_f32, kF32, kF32)
 SILE_SOFTMAX_NARROW_WIDTHS(f16_f32, kF16, kF32)
 
-// ---- wide rows: one row per workgroup of 1024 threads ----
-// Masked form of the row-per-workgroup kernel for any width up to
-// 1024 * kChunks * E: chunk j of thread t at column (j * 1024 + t) * E, whole
-// chunks as 16-byte accesses, the chunk the row ends in element by element,
-// positions past the row -inf (exp 0) and never stored.
-template <int kIn, int kOut, int kChunks>
-__device__ __forceinline__ void softmax_rows_wide_regs_kernel(const void* x, void* y,
-                                                              int64_t rows, int64_t cols,
-                                                              int64_t ldx, int64_t ldy) {
-  constexpr int kT = 1024;
-  constexpr int kE = chunk_elems<kIn, kOut>();
-  constexpr int kWaves = kT / 64;
-  __shared__ float part[2][kWaves];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int64_t row = blockIdx.x;
-  if (row >= rows) return;
-  using TI = typename Elem<kIn>::Storage;
-  using TO = typename Elem<kOut>::Storage;
-  const TI* xr = static_cast<const TI*>(x) + row * ldx;
-  TO* yr = static_cast<TO*>(y) + row * ldy;
-  float v[kChunks][kE];
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j) {
-    const int64_t c0 = ((int64_t)j * kT + t) * kE;
-    if (c0 + kE <= cols) {
-      load_chunk<kIn, kE>(xr + c0, v[j]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < kE; ++i)
-        v[j][i] = c0 + i < cols ? Elem<kIn>::load1(xr + c0 + i) : -__builtin_inff();
-    }
-  }
-  float m = -__builtin_inff();
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j)
-#pragma unroll
-    for (int i = 0; i < kE; ++i) m = fmax_ordered(m, v[j][i]);
-  m = wave_max(m);
-  if (lane == 0) part[0][wave] = m;
-  __syncthreads();
-  m = part[0][0];
-#pragma unroll
-  for (int w = 1; w < kWaves; ++w) m = fmax_ordered(m, part[0][w]);
-  float s = 0.0f;
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j)
-#pragma unroll
-    for (int i = 0; i < kE; ++i) {
-      v[j][i] = exp2_fast((v[j][i] - m) * kLog2e);
-      s += v[j][i];
-    }
-  s = wave_sum(s);
-  if (lane == 0) part[1][wave] = s;
-  __syncthreads();
-  s = part[1][0];
-#pragma unroll
-  for (int w = 1; w < kWaves; ++w) s += part[1][w];
-  const float inv = 1.0f / s;
-#pragma unroll
-  for (int j = 0; j < kChunks; ++j) {
-    const int64_t c0 = ((int64_t)j * kT + t) * kE;
-#pragma unroll
-    for (int i = 0; i < kE; ++i) v[j][i] = normalise<kOut>(v[j][i], s, inv);
-    if (c0 + kE <= cols) {
-      store_chunk<kOut, kE>(yr + c0, v[j]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < kE; ++i)
-        if (c0 + i < cols) Elem<kOut>::store1(yr + c0 + i, v[j][i]);
-    }
-  }
-}
-
-// Rows past 1024 * 8 * E: two passes over the row by one workgroup of 1024
+// ---- wide rows ----
+// Rows past 65536 elements: two passes over the row by one workgroup of 1024
 // threads, 16-byte accesses.  Pass 1 keeps a running (max, sum) per thread
 // (the sum rescaled when the max grows), then the workgroup combines them:
 // M = max of the maxima, S = sum of sum_t * exp(m_t - M).  Pass 2 reads the
@@ -615,23 +509,15 @@ __device__ __forceinline__ void softmax_rows_wide_kernel(const void* x, void* y,
   }
 }
 
-#define SILE_SOFTMAX_WIDE_REGS(NAME, IN, OUT, CH)                                              \
-  extern "C" __global__ __launch_bounds__(1024) void NAME(const void* x, void* y, int64_t rows,  \
-                                                          int64_t cols, int64_t ldx, int64_t ldy) { \
-    softmax_rows_wide_regs_kernel<IN, OUT, CH>(x, y, rows, cols, ldx, ldy);                      \
-  }
-#define SILE_SOFTMAX_WIDE_WIDTHS(TAG, IN, OUT)                      \
-  SILE_SOFTMAX_WIDE_REGS(sile_softmax_rows_##TAG##_w2, IN, OUT, 2)   \
-  SILE_SOFTMAX_WIDE_REGS(sile_softmax_rows_##TAG##_w4, IN, OUT, 4)   \
-  SILE_SOFTMAX_WIDE_REGS(sile_softmax_rows_##TAG##_w8, IN, OUT, 8)   \
+#define SILE_SOFTMAX_WIDE(TAG, IN, OUT)                                                      \
   extern "C" __global__ __launch_bounds__(1024) void sile_softmax_rows_##TAG##_wide(          \
       const void* x, void* y, int64_t rows, int64_t cols, int64_t ldx, int64_t ldy) {        \
     softmax_rows_wide_kernel<IN, OUT>(x, y, rows, cols, ldx, ldy);                           \
   }
-SILE_SOFTMAX_WIDE_WIDTHS(f16_f16, kF16, kF16)
-SILE_SOFTMAX_WIDE_WIDTHS(bf16_bf16, kBF16, kBF16)
-SILE_SOFTMAX_WIDE_WIDTHS(f32_f32, kF32, kF32)
-SILE_SOFTMAX_WIDE_WIDTHS(f16_f32, kF16, kF32)
+SILE_SOFTMAX_WIDE(f16_f16, kF16, kF16)
+SILE_SOFTMAX_WIDE(bf16_bf16, kBF16, kBF16)
+SILE_SOFTMAX_WIDE(f32_f32, kF32, kF32)
+SILE_SOFTMAX_WIDE(f16_f32, kF16, kF32)
 
 // ---- row reduce (ReduceMax / ReduceSum along axis 1), fp32 result ----
 // op 0 = max, the reference's fold from x0 bit for bit (first_max_* in
@@ -644,88 +530,135 @@ SILE_DEV float max_result(float v, const typename Elem<kIn>::Storage* xr) {
   return x0 != x0 ? x0 : v;
 }
 
-template <int kIn>
-__device__ __forceinline__ void reduce_rows_kernel(int op, int vec, const void* x, float* out,
-                                                   int64_t rows, int64_t cols, int64_t ldx) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+// Rows in the softmax's shapes (softmax_rows_tile_kernel): kT threads a row,
+// kC chunks a thread, all loaded before the first is folded.  A lane folds its
+// chunks in column order.  A wave a row that folded each chunk as it came (one
+// load in flight) read bf16 16384 x 1000 at 4.8 TB/s.
+template <int kIn, int kT, int kC>
+__device__ __forceinline__ void reduce_rows_tile_kernel(int op, const void* x, float* out,
+                                                        int64_t rows, int64_t cols,
+                                                        int64_t ldx) {
+  constexpr int kE = chunk_elems<kIn, kF32>();
+  constexpr int kWaves = kT / 64;
+  constexpr int kWhole = kC - 1;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int t = kT == 64 ? lane : threadIdx.x;
+  const int64_t row = kT == 64 ? (int64_t)blockIdx.x * 4 + wave : blockIdx.x;
   if (row >= rows) return;
   using TI = typename Elem<kIn>::Storage;
   const TI* xr = static_cast<const TI*>(x) + row * ldx;
-  constexpr int kE = chunk_elems<kIn, kF32>();  // one 16-byte load per lane
-  const int64_t vec_cols = vec ? (cols & ~(int64_t)(kE - 1)) : 0;
+  const int n = (int)cols;
+  // the chunk the row ends in is moved back to end there: the elements it has
+  // twice do not change the max (the same value and column) and are left out of
+  // the sum; chunks past the row are NaN, which never enters the max
+  float v[kC][kE];
+#pragma unroll
+  for (int j = 0; j < kC; ++j) {
+    const int c0 = (j * kT + t) * kE;
+    if (j < kWhole) {
+      load_chunk<kIn, kE>(xr + c0, v[j]);
+    } else if (c0 < n) {
+      load_chunk<kIn, kE>(xr + min(c0, n - kE), v[j]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kE; ++i) v[j][i] = __builtin_nanf("");
+    }
+  }
+  __shared__ float part[kWaves];
+  __shared__ int part_col[kWaves];
   if (op == 0) {
     float m = -__builtin_inff();
     int mi = kNoCol;
-    int64_t c = (int64_t)lane * kE;
-    for (; c + kE <= vec_cols; c += 64 * kE) {
-      float v[kE];
-      load_chunk<kIn, kE>(xr + c, v);
 #pragma unroll
-      for (int i = 0; i < kE; ++i) first_max_fold(m, mi, v[i], (int)c + i);
+    for (int j = 0; j < kC; ++j) {
+      const int c0 = (j * kT + t) * kE, at = j < kWhole ? c0 : min(c0, n - kE);
+#pragma unroll
+      for (int i = 0; i < kE; ++i) first_max_fold(m, mi, v[j][i], at + i);
     }
-    for (int64_t cc = vec_cols + lane; cc < cols; cc += 64)
-      first_max_fold(m, mi, Elem<kIn>::load1(xr + cc), (int)cc);
     wave_first_max(m, mi);
-    if (lane == 0) out[row] = max_result<kIn>(m, xr);
+    if constexpr (kT > 64) {
+      if (lane == 0) {
+        part[wave] = m;
+        part_col[wave] = mi;
+      }
+      __syncthreads();
+      if (t == 0) {
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) first_max_merge(m, mi, part[w], part_col[w]);
+      }
+    }
+    if (t == 0) out[row] = max_result<kIn>(m, xr);
     return;
   }
   float acc = 0.0f;
-  int64_t c = (int64_t)lane * kE;
-  for (; c + kE <= vec_cols; c += 64 * kE) {
-    float v[kE];
-    load_chunk<kIn, kE>(xr + c, v);
 #pragma unroll
-    for (int i = 0; i < kE; ++i) acc = acc + v[i];
+  for (int j = 0; j < kC; ++j) {
+    const int twice = j < kWhole ? 0 : (j * kT + t + 1) * kE - n;
+#pragma unroll
+    for (int i = 0; i < kE; ++i) acc = acc + (j < kWhole || i >= twice ? v[j][i] : 0.0f);
   }
-  for (int64_t cc = vec_cols + lane; cc < cols; cc += 64) acc = acc + Elem<kIn>::load1(xr + cc);
   acc = wave_sum(acc);
-  if (lane == 0) out[row] = acc;
+  if constexpr (kT > 64) {
+    if (lane == 0) part[wave] = acc;
+    __syncthreads();
+    if (t == 0) {
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) acc = acc + part[w];
+    }
+  }
+  if (t == 0) out[row] = acc;
 }
 
-// Narrow rows (up to 32 chunks): kL lanes per row, one chunk per lane, 64 /
-// kL rows per wave; rows of 16-byte aligned chunks only.
-template <int kIn, int kL>
+// Narrow rows (up to 32 chunks): kL lanes per row, one chunk per lane, kR rows
+// a group of lanes (the narrow softmax's shapes).
+template <int kIn, int kL, int kR>
 __device__ __forceinline__ void reduce_rows_narrow_kernel(int op, const void* x, float* out,
                                                           int64_t rows, int64_t cols,
                                                           int64_t ldx) {
   constexpr int kE = chunk_elems<kIn, kF32>();
+  constexpr int kWaveRows = 64 / kL;
   const int lane = threadIdx.x & 63, li = lane % kL;
-  const int64_t row = (int64_t)blockIdx.x * (256 / kL) + (threadIdx.x >> 6) * (64 / kL) + lane / kL;
-  const bool live = row < rows;
+  const int64_t row0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (kWaveRows * kR) + lane / kL;
   using TI = typename Elem<kIn>::Storage;
-  const TI* xr = static_cast<const TI*>(x) + (live ? row : 0) * ldx;
-  const int c0 = li * kE;
-  if (op == 0) {
-    float m = -__builtin_inff();
-    int mi = kNoCol;
-    if (live && c0 + kE <= cols) {
-      float v[kE];
-      load_chunk<kIn, kE>(xr + c0, v);
+  const int n = (int)cols, c0 = li * kE, at = n >= kE ? min(c0, n - kE) : c0;
+  const int twice = n >= kE ? c0 + kE - n : 0;
+  float v[kR][kE];
 #pragma unroll
-      for (int i = 0; i < kE; ++i) first_max_fold(m, mi, v[i], c0 + i);
-    } else if (live) {
-      for (int i = 0; c0 + i < cols && i < kE; ++i)
-        first_max_fold(m, mi, Elem<kIn>::load1(xr + c0 + i), c0 + i);
+  for (int r = 0; r < kR; ++r) {
+    const int64_t row = row0 + r * kWaveRows;
+    const bool live = row < rows && c0 < n;
+    const TI* xr = static_cast<const TI*>(x) + (row < rows ? row : 0) * ldx;
+    if (live && n >= kE) {
+      load_chunk<kIn, kE>(xr + at, v[r]);
+    } else {
+      const float pad = op == 0 ? __builtin_nanf("") : 0.0f;
+#pragma unroll
+      for (int i = 0; i < kE; ++i)
+        v[r][i] = live && c0 + i < n ? Elem<kIn>::load1(xr + c0 + i) : pad;
     }
-    group_first_max<kL>(m, mi);
-    if (live && li == 0) out[row] = max_result<kIn>(m, xr);
-    return;
   }
-  float acc = 0.0f;
-  if (live && c0 + kE <= cols) {
-    float v[kE];
-    load_chunk<kIn, kE>(xr + c0, v);
 #pragma unroll
-    for (int i = 0; i < kE; ++i) acc = acc + v[i];
-  } else if (live) {
-    for (int i = 0; c0 + i < cols && i < kE; ++i) acc = acc + Elem<kIn>::load1(xr + c0 + i);
+  for (int r = 0; r < kR; ++r) {
+    const int64_t row = row0 + r * kWaveRows;
+    const TI* xr = static_cast<const TI*>(x) + (row < rows ? row : 0) * ldx;
+    if (op == 0) {
+      float m = -__builtin_inff();
+      int mi = kNoCol;
+#pragma unroll
+      for (int i = 0; i < kE; ++i) first_max_fold(m, mi, v[r][i], at + i);
+      group_first_max<kL>(m, mi);
+      if (row < rows && li == 0) out[row] = max_result<kIn>(m, xr);
+    } else {
+      float acc = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kE; ++i) acc = acc + (i >= twice ? v[r][i] : 0.0f);
+      acc = group_sum<kL>(acc);
+      if (row < rows && li == 0) out[row] = acc;
+    }
   }
-  acc = group_sum<kL>(acc);
-  if (live && li == 0) out[row] = acc;
 }
 
-// Wide rows, few of them: one row per workgroup of 1024 threads, 16-byte
+// Rows past 1024 x 5 chunks: one row per workgroup of 1024 threads, 16-byte
 // chunks strided by the workgroup, wave all-reductions plus one exchange of
 // the per-wave partials through LDS.
 template <int kIn>
@@ -742,16 +675,27 @@ __device__ __forceinline__ void reduce_rows_block_kernel(int op, const void* x, 
   using TI = typename Elem<kIn>::Storage;
   const TI* xr = static_cast<const TI*>(x) + row * ldx;
   const int64_t vec_cols = cols & ~(int64_t)(kE - 1);
+  constexpr int64_t kStep = (int64_t)kT * kE;
   if (op == 0) {
     float m = -__builtin_inff();
     int mi = kNoCol;
-    for (int64_t c = (int64_t)t * kE; c < vec_cols; c += (int64_t)kT * kE) {
+    int64_t c = (int64_t)t * kE;
+    for (; c + 3 * kStep < vec_cols; c += 4 * kStep) {   // four chunks in flight
+      float v[4][kE];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) load_chunk<kIn, kE>(xr + c + j * kStep, v[j]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < kE; ++i) first_max_fold(m, mi, v[j][i], (int)(c + j * kStep) + i);
+    }
+    for (; c < vec_cols; c += kStep) {
       float v[kE];
       load_chunk<kIn, kE>(xr + c, v);
 #pragma unroll
       for (int i = 0; i < kE; ++i) first_max_fold(m, mi, v[i], (int)c + i);
     }
-    for (int64_t c = vec_cols + t; c < cols; c += kT)
+    for (c = vec_cols + t; c < cols; c += kT)
       first_max_fold(m, mi, Elem<kIn>::load1(xr + c), (int)c);
     wave_first_max(m, mi);
     if (lane == 0) {
@@ -766,13 +710,23 @@ __device__ __forceinline__ void reduce_rows_block_kernel(int op, const void* x, 
     return;
   }
   float acc = 0.0f;
-  for (int64_t c = (int64_t)t * kE; c < vec_cols; c += (int64_t)kT * kE) {
+  int64_t c = (int64_t)t * kE;
+  for (; c + 3 * kStep < vec_cols; c += 4 * kStep) {
+    float v[4][kE];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) load_chunk<kIn, kE>(xr + c + j * kStep, v[j]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < kE; ++i) acc = acc + v[j][i];
+  }
+  for (; c < vec_cols; c += kStep) {
     float v[kE];
     load_chunk<kIn, kE>(xr + c, v);
 #pragma unroll
     for (int i = 0; i < kE; ++i) acc = acc + v[i];
   }
-  for (int64_t c = vec_cols + t; c < cols; c += kT) acc = acc + Elem<kIn>::load1(xr + c);
+  for (c = vec_cols + t; c < cols; c += kT) acc = acc + Elem<kIn>::load1(xr + c);
   acc = wave_sum(acc);
   if (lane == 0) part[wave] = acc;
   __syncthreads();
@@ -837,23 +791,20 @@ __device__ __forceinline__ void reduce_rows_rowblock_kernel(int op, const void* 
   }
 }
 
+#define SILE_REDUCE_NARROW(TAG, IN, NAME, L, R)                                               \
+  extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_##TAG##_##NAME(          \
+      int op, const void* x, float* out, int64_t rows, int64_t cols, int64_t ldx) {          \
+    reduce_rows_narrow_kernel<IN, L, R>(op, x, out, rows, cols, ldx);                       \
+  }
 #define SILE_REDUCE_SHAPES(TAG, IN)                                                           \
-  extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_##TAG##_n4(              \
-      int op, const void* x, float* out, int64_t rows, int64_t cols, int64_t ldx) {          \
-    reduce_rows_narrow_kernel<IN, 4>(op, x, out, rows, cols, ldx);                          \
-  }                                                                                         \
-  extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_##TAG##_n8(              \
-      int op, const void* x, float* out, int64_t rows, int64_t cols, int64_t ldx) {          \
-    reduce_rows_narrow_kernel<IN, 8>(op, x, out, rows, cols, ldx);                          \
-  }                                                                                         \
-  extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_##TAG##_n16(             \
-      int op, const void* x, float* out, int64_t rows, int64_t cols, int64_t ldx) {          \
-    reduce_rows_narrow_kernel<IN, 16>(op, x, out, rows, cols, ldx);                         \
-  }                                                                                         \
-  extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_##TAG##_n32(             \
-      int op, const void* x, float* out, int64_t rows, int64_t cols, int64_t ldx) {          \
-    reduce_rows_narrow_kernel<IN, 32>(op, x, out, rows, cols, ldx);                         \
-  }                                                                                         \
+  SILE_REDUCE_NARROW(TAG, IN, n4, 4, 1)                                                     \
+  SILE_REDUCE_NARROW(TAG, IN, n8, 8, 1)                                                     \
+  SILE_REDUCE_NARROW(TAG, IN, n16, 16, 1)                                                   \
+  SILE_REDUCE_NARROW(TAG, IN, n32, 32, 1)                                                   \
+  SILE_REDUCE_NARROW(TAG, IN, n4r4, 4, 4)                                                   \
+  SILE_REDUCE_NARROW(TAG, IN, n8r4, 8, 4)                                                   \
+  SILE_REDUCE_NARROW(TAG, IN, n16r4, 16, 4)                                                 \
+  SILE_REDUCE_NARROW(TAG, IN, n32r4, 32, 4)                                                 \
   extern "C" __global__ __launch_bounds__(1024) void sile_reduce_rows_##TAG##_block(          \
       int op, const void* x, float* out, int64_t rows, int64_t cols, int64_t ldx) {          \
     reduce_rows_block_kernel<IN>(op, x, out, rows, cols, ldx);                              \
@@ -870,22 +821,29 @@ SILE_REDUCE_SHAPES(f32, kF32)
 SILE_REDUCE_SHAPES(f16, kF16)
 SILE_REDUCE_SHAPES(bf16, kBF16)
 
-extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_f32(int op, int vec, const void* x,
-                                                                       float* out, int64_t rows,
-                                                                       int64_t cols, int64_t ldx) {
-  reduce_rows_kernel<kF32>(op, vec, x, out, rows, cols, ldx);
-}
-extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_f16(int op, int vec, const void* x,
-                                                                       float* out, int64_t rows,
-                                                                       int64_t cols, int64_t ldx) {
-  reduce_rows_kernel<kF16>(op, vec, x, out, rows, cols, ldx);
-}
-extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_bf16(int op, int vec, const void* x,
-                                                                        float* out, int64_t rows,
-                                                                        int64_t cols,
-                                                                        int64_t ldx) {
-  reduce_rows_kernel<kBF16>(op, vec, x, out, rows, cols, ldx);
-}
+#define SILE_REDUCE_TILE(TAG, IN, T, CH)                                                      \
+  extern "C" __global__ __launch_bounds__(T < 256 ? 256 : T)                                  \
+      void sile_reduce_rows_##TAG##_t##T##c##CH(int op, const void* x, float* out,            \
+                                                int64_t rows, int64_t cols, int64_t ldx) {    \
+    reduce_rows_tile_kernel<IN, T, CH>(op, x, out, rows, cols, ldx);                          \
+  }
+#define SILE_REDUCE_TILES(TAG, IN)    \
+  SILE_REDUCE_TILE(TAG, IN, 64, 1)    \
+  SILE_REDUCE_TILE(TAG, IN, 64, 2)    \
+  SILE_REDUCE_TILE(TAG, IN, 64, 3)    \
+  SILE_REDUCE_TILE(TAG, IN, 64, 4)    \
+  SILE_REDUCE_TILE(TAG, IN, 256, 2)   \
+  SILE_REDUCE_TILE(TAG, IN, 256, 3)   \
+  SILE_REDUCE_TILE(TAG, IN, 256, 4)   \
+  SILE_REDUCE_TILE(TAG, IN, 512, 3)   \
+  SILE_REDUCE_TILE(TAG, IN, 512, 4)   \
+  SILE_REDUCE_TILE(TAG, IN, 512, 5)   \
+  SILE_REDUCE_TILE(TAG, IN, 512, 6)   \
+  SILE_REDUCE_TILE(TAG, IN, 1024, 4)  \
+  SILE_REDUCE_TILE(TAG, IN, 1024, 5)
+SILE_REDUCE_TILES(f32, kF32)
+SILE_REDUCE_TILES(f16, kF16)
+SILE_REDUCE_TILES(bf16, kBF16)
 
 // ---- fp32 row sums in the order of the reference's fused load + reduce ----
 // The CPU backend sums a row it loads straight from a buffer

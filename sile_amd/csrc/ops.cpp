@@ -191,6 +191,29 @@ FlashPlan flash_plan(int64_t bh, int64_t seq, int head_dim, bool causal) {
   return best;
 }
 
+// Workgroups of one row a group of lanes from which on narrow rows are taken
+// four a group.
+constexpr int64_t kNarrowGroups = 2048;
+
+// Threads and 16-byte chunks a thread for a row of n chunks kept in registers
+// (threads 0: too wide, more than max_chunks of 1024 threads).  A wave a row up
+// to 4 chunks a lane; then a workgroup a row, of the fewest threads that keep a
+// thread's chunks to 4 (256), 6 (512) and the rest: few loads in flight a wave
+// and many waves read faster than a wave with 8 to 32 chunks (fp32 8192 x 4097:
+// 99 us with 32 chunks a lane; 16-bit 4096 x 6000: 29.7 us with 16).
+struct RowTile {
+  int threads, chunks;
+};
+RowTile row_tile(int64_t n, int max_chunks) {
+  if (n <= 256) return {64, (int)((n + 63) / 64)};
+  if (n <= 1024) return {256, (int)((n + 255) / 256)};
+  if (n <= 3072) return {512, (int)((n + 511) / 512)};
+  int64_t c = (n + 1023) / 1024;
+  if (c > 8) c += c & 1;
+  if (c > max_chunks) return {0, 0};
+  return {1024, (int)c};
+}
+
 // fp32 -> 16-bit element bits, round to nearest even (NaN stays a quiet NaN),
 // for fill values converted on the host.
 uint32_t bf16_bits_rne(float f) {
@@ -735,25 +758,16 @@ int sile_hip_softmax_rows(sile_dtype in_type, sile_dtype out_type, int64_t rows,
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t blocks = (rows + 3) / 4;
   if (blocks > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "too many rows");
-  // register-resident kernels: a row of chunks * 64 lanes * E elements, E = 4
-  // for fp32 -> fp32 (one 16-byte access per lane and chunk), 8 otherwise
+  // E = 4 elements a chunk (one 16-byte access per lane) for fp32 -> fp32, 8
+  // otherwise; rows may start at any element
   const bool f32_rows = in_type == SILE_F32 && out_type == SILE_F32;
   const int64_t elems = f32_rows ? 4 : 8;
-  const int64_t ib = dtype_bytes(in_type), ob = dtype_bytes(out_type);
-  const bool vec_ok = (ldx * ib) % 16 == 0 && (ldy * ob) % 16 == 0 && aligned16(x) && aligned16(y);
-  int chunks = 0;
-  if (vec_ok) {
-    for (int c : {1, 2, 4, 8, 16, 32})
-      if (cols == (int64_t)c * 64 * elems && (c < 32 || f32_rows)) chunks = c;
-  }
   char name[64];
   int rc;
   // rows of 256 / 512 / 1024 threads x 2 chunks: one row per workgroup
   int block_threads = 0;
-  if (vec_ok) {
-    for (int t : {256, 512, 1024})
-      if (cols == (int64_t)t * 2 * elems) block_threads = t;
-  }
+  for (int t : {256, 512, 1024})
+    if (cols == (int64_t)t * 2 * elems) block_threads = t;
   if (block_threads) {
     if (rows > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "too many rows");
     snprintf(name, sizeof name, "sile_softmax_rows_%s_b%d", tag, block_threads);
@@ -763,53 +777,29 @@ int sile_hip_softmax_rows(sile_dtype in_type, sile_dtype out_type, int64_t rows,
   }
   // rows of up to 32 chunks: kL lanes per row (the smallest of 4, 8, 16, 32
   // that covers it), several rows per wave
-  if (vec_ok && cols <= 32 * elems) {
+  if (cols <= 32 * elems) {
     int lanes = 4;
     while ((int64_t)lanes * elems < cols) lanes *= 2;
-    const int64_t per_block = 256 / lanes;
-    if ((rows + per_block - 1) / per_block > 0x7fffffffLL)
-      return fail(SILE_ERR_SHAPE, "too many rows");
-    snprintf(name, sizeof name, "sile_softmax_rows_%s_n%d", tag, lanes);
+    // four rows a group of lanes where that still leaves enough workgroups
+    const int r = rows * lanes >= 256 * kNarrowGroups ? 4 : 1;
+    const int64_t per_block = 256 / lanes * r;
+    snprintf(name, sizeof name, "sile_softmax_rows_%s_n%d%s", tag, lanes, r == 4 ? "r4" : "");
     void* params[] = {&x, &y, &rows, &cols, &ldx, &ldy};
     rc = launch(Module::kSoftmax, name, dim3((unsigned)((rows + per_block - 1) / per_block)),
                 dim3(256), params, s);
     return rc == SILE_OK ? ok() : rc;
   }
-  // other widths up to 8192 (16-bit) / 8192 (fp32): one pass with a masked
-  // last chunk, the smallest power-of-two chunk count that covers the row
-  int masked = 0;
-  if (!chunks && vec_ok) {
-    for (int c : {1, 2, 4, 8, 16, 32})
-      if (!masked && cols <= (int64_t)c * 64 * elems && (c < 32 || f32_rows)) masked = c;
-  }
-  // wider rows: one row per 1024-thread workgroup, in registers up to
-  // 1024 * 8 chunks, in two passes beyond
-  if (!chunks && !masked && vec_ok) {
-    if (rows > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "too many rows");
-    int wide = 0;
-    for (int c : {2, 4, 8})
-      if (!wide && cols <= (int64_t)c * 1024 * elems) wide = c;
-    if (wide)
-      snprintf(name, sizeof name, "sile_softmax_rows_%s_w%d", tag, wide);
-    else
-      snprintf(name, sizeof name, "sile_softmax_rows_%s_wide", tag);
-    void* params[] = {&x, &y, &rows, &cols, &ldx, &ldy};
-    rc = launch(Module::kSoftmax, name, dim3((unsigned)rows), dim3(1024), params, s);
-    return rc == SILE_OK ? ok() : rc;
-  }
-  if (masked) {
-    snprintf(name, sizeof name, "sile_softmax_rows_%s_m%d", tag, masked);
-    void* params[] = {&x, &y, &rows, &cols, &ldx, &ldy};
-    rc = launch(Module::kSoftmax, name, dim3((unsigned)blocks), dim3(256), params, s);
-  } else if (chunks) {
-    snprintf(name, sizeof name, "sile_softmax_rows_%s_c%d", tag, chunks);
-    void* params[] = {&x, &y, &rows, &ldx, &ldy};
-    rc = launch(Module::kSoftmax, name, dim3((unsigned)blocks), dim3(256), params, s);
-  } else {
-    snprintf(name, sizeof name, "sile_softmax_rows_%s_any", tag);
-    void* params[] = {&x, &y, &rows, &cols, &ldx, &ldy};
-    rc = launch(Module::kSoftmax, name, dim3((unsigned)blocks), dim3(256), params, s);
-  }
+  // other widths: in registers up to 65536 elements (64 a thread), in two
+  // passes over the row beyond
+  const RowTile tile = row_tile((cols + elems - 1) / elems, f32_rows ? 16 : 8);
+  void* params[] = {&x, &y, &rows, &cols, &ldx, &ldy};
+  if (tile.threads)
+    snprintf(name, sizeof name, "sile_softmax_rows_%s_t%dc%d", tag, tile.threads, tile.chunks);
+  else
+    snprintf(name, sizeof name, "sile_softmax_rows_%s_wide", tag);
+  if (tile.threads != 64 && rows > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "too many rows");
+  rc = launch(Module::kSoftmax, name, dim3((unsigned)(tile.threads == 64 ? blocks : rows)),
+              dim3(tile.threads == 64 ? 256 : tile.threads ? tile.threads : 1024), params, s);
   return rc == SILE_OK ? ok() : rc;
 }
 
@@ -834,25 +824,23 @@ int sile_hip_reduce_rows(sile_reduce_op op, sile_dtype in_type, int64_t rows, in
   const int64_t blocks = (rows + 3) / 4;
   if (blocks > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "too many rows");
   int iop = (int)op;
-  // The 128-bit paths need every row start 16-byte aligned; otherwise the
-  // wave-per-row kernel runs its scalar loop only.
-  int vec = aligned16(x) && (ldx * (int64_t)dtype_bytes(in_type)) % 16 == 0 ? 1 : 0;
   const int64_t elems = in_type == SILE_F32 ? 4 : 8;   // per 16-byte chunk
   char kname[64];
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (vec && cols <= 32 * elems) {
+  if (cols <= 32 * elems) {
     // up to 32 chunks: kL lanes per row, several rows per wave
     int lanes = 4;
     while ((int64_t)lanes * elems < cols) lanes *= 2;
-    const int64_t per_block = 256 / lanes;
-    snprintf(kname, sizeof kname, "%s_n%d", name, lanes);
+    const int r = rows * lanes >= 256 * kNarrowGroups ? 4 : 1;
+    const int64_t per_block = 256 / lanes * r;
+    snprintf(kname, sizeof kname, "%s_n%d%s", name, lanes, r == 4 ? "r4" : "");
     void* params[] = {&iop, &x, &out, &rows, &cols, &ldx};
     int rc = launch(Module::kSoftmax, kname, dim3((unsigned)((rows + per_block - 1) / per_block)),
                     dim3(256), params, s);
     return rc == SILE_OK ? ok() : rc;
   }
   for (int t : {256, 512}) {
-    if (vec && cols == (int64_t)t * 2 * elems) {
+    if (cols == (int64_t)t * 2 * elems) {
       // rows of 2 chunks per thread of a 256 / 512-thread workgroup (the
       // 1024-thread shape read 16384-wide f16 rows at 4.5 TB/s)
       if (rows > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "too many rows");
@@ -862,15 +850,15 @@ int sile_hip_reduce_rows(sile_reduce_op op, sile_dtype in_type, int64_t rows, in
       return rc == SILE_OK ? ok() : rc;
     }
   }
-  if (vec && cols >= 16384 && rows <= 4096) {
-    // few wide rows: a 1024-thread workgroup per row
+  const RowTile tile = row_tile((cols + elems - 1) / elems, 5);
+  if (tile.threads)
+    snprintf(kname, sizeof kname, "%s_t%dc%d", name, tile.threads, tile.chunks);
+  else
     snprintf(kname, sizeof kname, "%s_block", name);
-    void* params[] = {&iop, &x, &out, &rows, &cols, &ldx};
-    int rc = launch(Module::kSoftmax, kname, dim3((unsigned)rows), dim3(1024), params, s);
-    return rc == SILE_OK ? ok() : rc;
-  }
-  void* params[] = {&iop, &vec, &x, &out, &rows, &cols, &ldx};
-  int rc = launch(Module::kSoftmax, name, dim3((unsigned)blocks), dim3(256), params, s);
+  if (tile.threads != 64 && rows > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "too many rows");
+  void* params[] = {&iop, &x, &out, &rows, &cols, &ldx};
+  int rc = launch(Module::kSoftmax, kname, dim3((unsigned)(tile.threads == 64 ? blocks : rows)),
+                  dim3(tile.threads == 64 ? 256 : tile.threads ? tile.threads : 1024), params, s);
   return rc == SILE_OK ? ok() : rc;
 }
 

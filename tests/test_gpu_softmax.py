@@ -313,3 +313,102 @@ def test_reduce_rows_max_follows_the_fold(hip, dt, cols, pitch_pad):
     ref = cpuref.reduce_rows(np.ascontiguousarray(xf), cpuref.REDUCE_MAX, cols=cols)
     assert np.isnan(ref[0]) and not np.isnan(ref[1])
     assert_same_bits(got, ref, what=f"row max {dt} {cols}")
+
+
+def _offset_rows(hip, bits, rows, cols, ld, off):
+    """`bits` [rows, cols] in rows of `ld` elements, `off` elements into a buffer."""
+    host = np.zeros(off + rows * ld, bits.dtype)
+    host[off:].reshape(rows, ld)[:, :cols] = bits
+    buf = hip.DeviceBuffer.from_array(host)
+    return buf, buf.ptr + off * bits.itemsize
+
+
+# widths around the chunk counts where the kernel changes (32, 256, 1024, 3072
+# and 8192 chunks of 4 or 8 elements, 64 elements a thread) and inside each
+UNALIGNED_COLS = [1, 5, 7, 9, 37, 129, 250, 257, 777, 1021, 1025, 2047, 3001, 4097, 5001, 8191,
+                  9003, 12289, 20003, 24577, 33001, 47777, 57345, 65535, 65543]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32", "f16_f32"])
+@pytest.mark.parametrize("cols", UNALIGNED_COLS)
+def test_softmax_rows_at_any_element(hip, dt, cols):
+    """Odd pitches and starts: every row begins at another alignment.  -inf
+    runs at both ends of a row; the pitch padding of y keeps its fill."""
+    rows, ldx, ldy, off = 6, cols + 3, cols + 1, 1
+    say(f"softmax unaligned {dt} {rows}x{cols}")
+    x = (rng(cols).normal(size=(rows, cols)) * 2.0).astype(np.float32)
+    if cols > 8:
+        x[1, :cols // 2] = -np.inf
+        x[2, 1 - cols // 3:] = -np.inf
+    tin, tout = {"f16": (hip.F16, hip.F16), "bf16": (hip.BF16, hip.BF16), "f32": (hip.F32, hip.F32),
+                 "f16_f32": (hip.F16, hip.F32)}[dt]
+    bits, xf = (x, x) if dt == "f32" else bf16_round(x) if dt == "bf16" else f16_round(x)
+    dx, px = _offset_rows(hip, bits, rows, cols, ldx, off)
+    ydt = np.float32 if tout == hip.F32 else np.uint16
+    dy = hip.DeviceBuffer((off + rows * ldy) * np.dtype(ydt).itemsize)
+    dy.fill_bytes(0x33)
+    hip.softmax_rows(tin, tout, rows, cols, px, ldx, dy.ptr + off * np.dtype(ydt).itemsize, ldy)
+    hip.synchronize()
+    raw = dy.download(ydt, (off + rows * ldy,))
+    fill = np.frombuffer(b"\x33" * np.dtype(ydt).itemsize, ydt)[0]
+    assert raw[0] == fill and (raw[off:].reshape(rows, ldy)[:, cols:] == fill).all()
+    y = raw[off:].reshape(rows, ldy)[:, :cols]
+    y = (y if ydt == np.float32 else cpuref.f32_from_bf16(np.ascontiguousarray(y)) if dt == "bf16"
+         else np.ascontiguousarray(y).view(np.float16).astype(np.float32))
+    e = np.exp(xf.astype(np.float64) - xf.max(1, keepdims=True))
+    rtol = 2e-5 if tout == hip.F32 else 1e-2
+    assert_close(y, e / e.sum(1, keepdims=True), atol=1e-6, rtol=rtol, what="softmax")
+    for b in (dx, dy):
+        b.close()
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("cols", UNALIGNED_COLS + [131079])
+def test_reduce_rows_at_any_element(hip, dt, cols):
+    """Row max (bit for bit, with the fold's NaN and signed-zero rows) and row
+    sum (within 1e-5 of the row's absolute sum) at odd pitches and starts."""
+    x = (max_fold_probe_rows(cols, cols) if cols >= 37
+         else rng(cols).normal(size=(6, cols)).astype(np.float32))
+    rows, ldx, off = x.shape[0], cols + 3, 1
+    say(f"reduce unaligned {dt} {rows}x{cols}")
+    tin = {"f32": hip.F32, "f16": hip.F16, "bf16": hip.BF16}[dt]
+    bits, xf = (x, x) if dt == "f32" else bf16_round(x) if dt == "bf16" else f16_round(x)
+    dx, px = _offset_rows(hip, bits, rows, cols, ldx, off)
+    out = hip.DeviceBuffer(4 * rows)
+    hip.reduce_rows(hip.REDUCE_MAX, tin, rows, cols, px, ldx, out.ptr)
+    hip.synchronize()
+    assert_same_bits(out.download(np.float32, (rows,)), cpuref.reduce_rows(xf, cpuref.REDUCE_MAX), "row max")
+    x = rng(cols + 1).normal(size=(rows, cols)).astype(np.float32)
+    bits, xf = (x, x) if dt == "f32" else bf16_round(x) if dt == "bf16" else f16_round(x)
+    ds, ps = _offset_rows(hip, bits, rows, cols, ldx, off)
+    hip.reduce_rows(hip.REDUCE_SUM, tin, rows, cols, ps, ldx, out.ptr)
+    hip.synchronize()
+    got = out.download(np.float32, (rows,)).astype(np.float64)
+    assert (np.abs(got - xf.sum(1, dtype=np.float64))
+            <= 1e-5 * np.abs(xf).sum(1, dtype=np.float64)).all()
+    for b in (dx, ds, out):
+        b.close()
+
+
+@pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("cols", [3, 13, 64, 101, 250])
+def test_narrow_rows_four_a_group(hip, dt, cols):
+    """Launches large enough to take four rows a group of lanes, the last
+    workgroup and wave partly empty."""
+    rows = 140003 if cols <= 16 else 70001 if cols <= 64 else 40001
+    say(f"narrow many {dt} {rows}x{cols}")
+    x = rng(cols).normal(size=(rows, cols)).astype(np.float32)
+    bits, xf = (x, x) if dt == "f32" else f16_round(x)
+    t = hip.F32 if dt == "f32" else hip.F16
+    dx, out = hip.DeviceBuffer.from_array(bits), hip.DeviceBuffer(4 * rows)
+    dy = hip.DeviceBuffer(bits.nbytes)
+    hip.softmax_rows(t, t, rows, cols, dx.ptr, cols, dy.ptr, cols)
+    hip.reduce_rows(hip.REDUCE_MAX, t, rows, cols, dx.ptr, cols, out.ptr)
+    hip.synchronize()
+    np.testing.assert_array_equal(out.download(np.float32, (rows,)), xf.max(1))
+    y = dy.download(bits.dtype, (rows, cols))
+    y = y if dt == "f32" else y.view(np.float16).astype(np.float32)
+    e = np.exp(xf.astype(np.float64) - xf.max(1, keepdims=True))
+    assert_close(y, e / e.sum(1, keepdims=True), atol=1e-6, rtol=2e-5 if dt == "f32" else 1e-2)
+    for b in (dx, dy, out):
+        b.close()
