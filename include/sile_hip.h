@@ -276,7 +276,11 @@ int sile_hip_kernel_parallel_reduce(void *const *buffers, int64_t num_threadgrou
  *                        tiles' stores but M is a multiple of 4 and at least
  *                        one tile, the same kernels compute C^T into fp32
  *                        scratch and a second kernel writes C; other shapes:
- *                        64 x 64 tiles).
+ *                        64 x 64 tiles).  When A or a column-major B has at
+ *                        most 64 rows, a kernel that streams the other operand
+ *                        once (plain launch, also under capture) takes the
+ *                        place of either, wherever it is modelled faster or
+ *                        the tiles cannot take the shape.
  * When the tiles are fewer than the device's CUs and K' is long, K' may be
  * split into ranges computed side by side: their fp32 partial C planes go
  * to a device scratch buffer shared by all calls on the device (allocated on

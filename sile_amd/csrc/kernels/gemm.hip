@@ -924,6 +924,270 @@ SILE_GEMM_SMALL_KERNEL(sile_gemm_small_f16_f32, kF16, kOutF32)
 SILE_GEMM_SMALL_KERNEL(sile_gemm_small_fp8_bf16, kFP8, kOutBF16)
 SILE_GEMM_SMALL_KERNEL(sile_gemm_small_fp8_f32, kFP8, kOutF32)
 
+// ---------------------------------------------------------------------------
+// Few rows: one operand of at most 64 rows (a decoding step's activations)
+// against all rows of the other, HBM-bound on the other's bytes.
+//
+// A workgroup of 4 waves takes 16 kR rows of the large operand L and all of the
+// small one S (kM tiles of 16 rows) over all of K', so no second launch adds
+// partial planes and the launch has L's rows / (16 kR) workgroups to fill the
+// CUs.  Each wave takes a quarter of K' by itself: k-steps of 128 bytes a row
+// go from memory into a ring of kD slots of its own in LDS (buffer loads to
+// LDS, 8 whole lines an instruction), with no barrier in the loop, and the
+// waves' fp32 results are added in wave order at the end.  Rows past either
+// operand load as zeros; the last k-step's elements past K' are zeroed in both.
+// (Loading the 16 x 16 MFMAs' fragments, 16 rows of 64 bytes, straight into
+// registers ran 40 us at bf16 16 x 8192 x 8192: 80 clocks a load.)
+// bf16 16 x 8192 x 8192 (134 MB): 31.9 us as 128 x 128 tiles with a split K' and
+// its second launch, 24.7 here; 16 x 4096 x 4096 15.5 -> 8.3; fp8 16 x 8192 x 8192
+// 19.1 -> 13.1; 64 x 64 x 8192 (64 x 64 tiles before) 118 -> 13.
+// ---------------------------------------------------------------------------
+struct FewArgs {
+  int64_t ldl, lds, ldc;   // in elements
+  int64_t rows_l, kp;
+  int32_t rows_s;
+  int32_t l_is_b;          // C[s][l] (L is B) or C[l][s] (L is A)
+  int32_t stream_l;        // L is loaded non-temporally
+  float alpha;
+};
+
+template <int kKind, int kOut, int kR, int kM>
+__device__ __forceinline__ void gemm_few_body(const uint8_t* __restrict__ L,
+                                              const uint8_t* __restrict__ S, void* __restrict__ C,
+                                              const FewArgs& g) {
+  constexpr bool kIsFP8 = kKind == kFP8;
+  constexpr int kEB = kIsFP8 ? 1 : 2;
+  constexpr int kWaves = 4;
+  constexpr int kT = kR + kM;                    // 16-row tiles of a slot
+  constexpr int kSlotB = kT * 16 * kRowB;
+  constexpr int kD = 163840 / kWaves / kSlotB < 10 ? 163840 / kWaves / kSlotB : 10;
+  constexpr int kPitch = 16 * kR + 4;            // LDS floats per row of S (partial results)
+  static_assert(kWaves * 16 * kM * kPitch * 4 <= kWaves * kD * kSlotB, "partial results fit");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kWaves * kD * kSlotB];
+  auto part = reinterpret_cast<float (*)[16 * kM][kPitch]>(smem);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, grp = lane >> 4, swz = (r >> 1) & 7;
+  const int64_t l0 = (int64_t)blockIdx.x * (16 * kR);
+  const int l_rows = (int)min((int64_t)(16 * kR), g.rows_l - l0);
+  uint8_t* const ring = smem + wave * (kD * kSlotB);
+
+  // k-steps of 128 bytes of a row; this wave's are [k0, k1), from one of its
+  // own on around the range: workgroups in step would all read the same columns,
+  // whose lines lie on the same few memory channels when the pitch is a power
+  // of two
+  const int steps = (int)((g.kp * kEB + kRowB - 1) / kRowB);
+  const int per = (steps + kWaves - 1) / kWaves;
+  const int k0 = min(wave * per, steps), k1 = min(k0 + per, steps), mine = k1 - k0;
+  const int first = mine > 0 ? k0 + (int)((blockIdx.x * 5u) % (unsigned)mine) : k0;
+  auto after = [&](int ks) { return ks + 1 == k1 ? k0 : ks + 1; };
+
+  // an operand's rows up to the 16-byte chunk its last row's K' ends in
+  const int64_t kp_b = (g.kp * kEB + 15) & ~(int64_t)15;
+  const __amdgpu_buffer_rsrc_t l_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(L + l0 * g.ldl * kEB), (short)0, (int)((l_rows - 1) * g.ldl * kEB + kp_b), 0x00020000);
+  const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)S, (short)0, (int)((g.rows_s - 1) * g.lds * kEB + kp_b), 0x00020000);
+  // one instruction fills 8 rows: lane l row l / 8, position l % 8, which holds
+  // chunk c of the row at c ^ ((row >> 1) & 7) (two rows span the banks)
+  const int d_row = lane >> 3;
+  const int l_rs = (int)(g.ldl * kEB), s_rs = (int)(g.lds * kEB);
+  auto load_tiles = [&](auto rsrc, auto n_c, auto aux_c, int rs, int ks, uint8_t* dst) {
+#pragma unroll
+    for (int i = 0; i < decltype(n_c)::value; ++i) {
+      const int row = 8 * i + d_row;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc, (lds_ptr_t)(dst + i * 1024), 16,
+          row * rs + (((lane & 7) ^ ((row >> 1) & 7)) << 4) + ks * kRowB, 0, 0, decltype(aux_c)::value);
+    }
+  };
+  using LTiles = std::integral_constant<int, 2 * kR>;
+  using STiles = std::integral_constant<int, 2 * kM>;
+  using Plain = std::integral_constant<int, 0>;
+  using NonTemporal = std::integral_constant<int, 2>;
+  auto load = [&](int ks, int slot) {
+    uint8_t* dst = ring + slot * kSlotB;
+    if (g.stream_l)
+      load_tiles(l_rsrc, LTiles{}, NonTemporal{}, l_rs, ks, dst);
+    else
+      load_tiles(l_rsrc, LTiles{}, Plain{}, l_rs, ks, dst);
+    load_tiles(s_rsrc, STiles{}, Plain{}, s_rs, ks, dst + 2 * kR * 1024);
+  };
+
+  // sums of 4 k-steps, and their sum: chains of K' / 4 products rounded twice as
+  // far off as the split tiles' (4e-7 against 1.6e-7 at K' = 16384)
+  f32x4 acc[kR][kM], total[kR][kM];
+#pragma unroll
+  for (int i = 0; i < kR; ++i)
+#pragma unroll
+    for (int j = 0; j < kM; ++j) acc[i][j] = total[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto gather = [&]() {
+#pragma unroll
+    for (int i = 0; i < kR; ++i)
+#pragma unroll
+      for (int j = 0; j < kM; ++j) {
+        total[i][j] += acc[i][j];
+        acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+  };
+  // the 2 (16-bit: k halves; fp8: one fragment) 16-byte chunks of a lane
+  auto read = [&](const uint8_t* base, int t, u32x4 (&f)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int c = kIsFP8 ? 2 * grp + h : 4 * h + grp;
+      f[h] = *reinterpret_cast<const u32x4*>(base + (16 * t + r) * kRowB + ((c ^ swz) << 4));
+    }
+  };
+  auto compute = [&](int slot, int k_rem, auto last_c) {
+    const uint8_t* base = ring + slot * kSlotB;
+    u32x4 lf[kR][2], sf[kM][2];
+#pragma unroll
+    for (int t = 0; t < kR; ++t) read(base, t, lf[t]);
+#pragma unroll
+    for (int t = 0; t < kM; ++t) read(base, kR + t, sf[t]);
+    if constexpr (decltype(last_c)::value) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int e0 = (kIsFP8 ? 2 * grp + h : 4 * h + grp) * (16 / kEB);
+#pragma unroll
+        for (int t = 0; t < kR; ++t) lf[t][h] = mask_k<kIsFP8>(lf[t][h], e0, k_rem);
+#pragma unroll
+        for (int t = 0; t < kM; ++t) sf[t][h] = mask_k<kIsFP8>(sf[t][h], e0, k_rem);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kR; ++i)
+#pragma unroll
+      for (int j = 0; j < kM; ++j) {
+        if constexpr (kIsFP8) {
+          const i32x8 av = {(int)lf[i][0][0], (int)lf[i][0][1], (int)lf[i][0][2], (int)lf[i][0][3],
+                            (int)lf[i][1][0], (int)lf[i][1][1], (int)lf[i][1][2], (int)lf[i][1][3]};
+          const i32x8 bv = {(int)sf[j][0][0], (int)sf[j][0][1], (int)sf[j][0][2], (int)sf[j][0][3],
+                            (int)sf[j][1][0], (int)sf[j][1][1], (int)sf[j][1][2], (int)sf[j][1][3]};
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[i][j], 0, 0, 0, 0,
+                                                                       0, 0);
+        } else {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            if constexpr (kKind == kBF16)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  __builtin_bit_cast(bf16x8, lf[i][h]), __builtin_bit_cast(bf16x8, sf[j][h]),
+                  acc[i][j], 0, 0, 0);
+            else
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  __builtin_bit_cast(f16x8, lf[i][h]), __builtin_bit_cast(f16x8, sf[j][h]),
+                  acc[i][j], 0, 0, 0);
+          }
+        }
+      }
+  };
+  // Steps of the ring: the slot of step ks is loaded kD - 1 steps ahead, into
+  // the slot that step ks - 1 has finished reading.  A step waits for its own
+  // 2 kT loads with those of the kD - 2 newer steps in flight; the steps at the
+  // end of the range load nothing, so they wait for everything.
+  constexpr int kFly = (kD - 2) * 2 * kT;
+  static_assert(kFly <= 63, "vmcnt");
+  auto wait_vm = [](auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (0x7 << 4) | (0xf << 8));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const int k_rem = (int)(g.kp - (int64_t)(steps - 1) * (kRowB / kEB));   // of the last step
+  auto step = [&](int slot, int ks) {
+    if (ks == steps - 1 && k_rem < kRowB / kEB)
+      compute(slot, k_rem, std::true_type{});
+    else
+      compute(slot, 0, std::false_type{});
+  };
+  int slot = 0, fill = 0, i = 0, ks = first, ahead = first;
+  for (; fill < kD - 1 && fill < mine; ++fill) {
+    load(ahead, fill);
+    ahead = after(ahead);
+  }
+  for (; i + kD - 1 < mine; ++i) {
+    wait_vm(std::integral_constant<int, kFly>{});
+    load(ahead, fill);
+    ahead = after(ahead);
+    __builtin_amdgcn_sched_barrier(0);
+    step(slot, ks);
+    if ((i & 3) == 3) gather();
+    // the reads of this slot are done before the next step loads into it
+    __builtin_amdgcn_sched_barrier(0);
+    ks = after(ks);
+    fill = slot;
+    slot = slot + 1 == kD ? 0 : slot + 1;
+  }
+  if (i < mine) wait_vm(std::integral_constant<int, 0>{});
+  for (; i < mine; ++i) {
+    step(slot, ks);
+    ks = after(ks);
+    slot = slot + 1 == kD ? 0 : slot + 1;
+  }
+  gather();
+  __syncthreads();   // every read of the rings is done
+
+  // register e of a block: row 4 (l / 16) + e of L, row l % 16 of S
+#pragma unroll
+  for (int i = 0; i < kR; ++i)
+#pragma unroll
+    for (int j = 0; j < kM; ++j)
+      *reinterpret_cast<f32x4*>(&part[wave][16 * j + r][16 * i + 4 * grp]) = total[i][j];
+  __syncthreads();
+  constexpr int kQuads = 4 * kR;   // groups of 4 rows of L
+  for (int e = threadIdx.x; e < 16 * kM * kQuads; e += 64 * kWaves) {
+    // neighbouring threads store neighbouring elements of C
+    const int sr = g.l_is_b ? e / kQuads : e % (16 * kM);
+    const int lq = g.l_is_b ? e % kQuads : e / (16 * kM);
+    if (sr >= g.rows_s) continue;
+    f32x4 v = *reinterpret_cast<const f32x4*>(&part[0][sr][4 * lq]);
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) v += *reinterpret_cast<const f32x4*>(&part[w][sr][4 * lq]);
+    if (g.alpha != 1.0f) v *= g.alpha;
+    const int64_t lr = l0 + 4 * lq;
+    const int64_t idx = g.l_is_b ? sr * g.ldc + lr : lr * g.ldc + sr;
+    if (g.l_is_b && lr + 4 <= g.rows_l && (g.ldc & 3) == 0 &&
+        (reinterpret_cast<uintptr_t>(C) & (kOut == kOutF32 ? 15 : 7)) == 0) {
+      store_c4<kOut>(C, idx, v);
+      continue;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (lr + u >= g.rows_l) break;
+      const int64_t at = idx + (g.l_is_b ? u : u * g.ldc);
+      const float x = v[u];
+      if constexpr (kOut == kOutF32)
+        static_cast<float*>(C)[at] = x;
+      else if constexpr (kOut == kOutBF16)
+        static_cast<uint16_t*>(C)[at] = bf16_rne(x);
+      else
+        static_cast<uint16_t*>(C)[at] = f16_rne(x);
+    }
+  }
+}
+
+#define SILE_GEMM_FEW(NAME, KIND, OUT, R, M)                                                   \
+  extern "C" __global__ __launch_bounds__(256, 1) void NAME##_r##R##m##M(                      \
+      const void* L, const void* S, void* C, FewArgs g) {                                      \
+    gemm_few_body<KIND, OUT, R, M>(static_cast<const uint8_t*>(L),                             \
+                                   static_cast<const uint8_t*>(S), C, g);                      \
+  }
+#define SILE_GEMM_FEW_SHAPES(NAME, KIND, OUT) \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 1, 1)        \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 1, 2)        \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 1, 4)        \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 2, 1)        \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 2, 2)        \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 2, 4)        \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 4, 1)        \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 4, 2)        \
+  SILE_GEMM_FEW(NAME, KIND, OUT, 4, 4)
+SILE_GEMM_FEW_SHAPES(sile_gemm_few_bf16_bf16, kBF16, kOutBF16)
+SILE_GEMM_FEW_SHAPES(sile_gemm_few_bf16_f32, kBF16, kOutF32)
+SILE_GEMM_FEW_SHAPES(sile_gemm_few_f16_f16, kF16, kOutF16)
+SILE_GEMM_FEW_SHAPES(sile_gemm_few_f16_f32, kF16, kOutF32)
+SILE_GEMM_FEW_SHAPES(sile_gemm_few_fp8_bf16, kFP8, kOutBF16)
+SILE_GEMM_FEW_SHAPES(sile_gemm_few_fp8_f32, kFP8, kOutF32)
+
 // C = 0 for K' = 0 (K below one BK): the canonical matmul's sums start at
 // 0.0f and add no term (crates/sile-tile-ir/src/passes/lowering/canonical_matmul.rs:58-73,
 // k_limit = 0).  C is addressed in 16-bit words: n16 words per row, ldc16

@@ -69,6 +69,7 @@ constexpr int64_t kScratchPlanesMax = 256ll << 20;
 struct GemmPlan {
   int tile;        // 256 or 128
   int64_t splits;  // k-ranges (1: K' not split)
+  double seconds;  // modelled time
 };
 
 // compute units of the current device
@@ -93,7 +94,7 @@ double tile_time_per_k(int tile, int64_t w, int cus) {
 
 GemmPlan gemm_plan(int64_t m, int64_t n, int64_t kp, int64_t half_steps, int64_t cb, bool fp8,
                    int only_tile) {
-  GemmPlan best{only_tile ? only_tile : m >= 256 && n >= 256 ? 256 : 128, 1};
+  GemmPlan best{only_tile ? only_tile : m >= 256 && n >= 256 ? 256 : 128, 1, 0.0};
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
@@ -119,15 +120,34 @@ GemmPlan gemm_plan(int64_t m, int64_t n, int64_t kp, int64_t half_steps, int64_t
       }
       if (sp == 1 && t < best_unsplit_t) {
         best_unsplit_t = t;
-        best_unsplit = {tile, 1};
+        best_unsplit = {tile, 1, t};
       }
       if (t < best_t) {
         best_t = t;
-        best = {tile, sp};
+        best = {tile, sp, t};
       }
     }
   }
   return best.splits > 1 && !(best_t < 0.95 * best_unsplit_t) ? best_unsplit : best;
+}
+
+// 16-row tiles of the large operand a workgroup of the few-rows GEMM takes: the
+// most (1, 2 or 4) that still give a workgroup to nine CUs of ten.  *seconds:
+// its modelled time, the operands' bytes at 5.4 TB/s or the rounds of
+// workgroups (one a CU), each its rows' bytes at 105 GB/s and 1.5 us.  Measured
+// with 1 / 2 / 4 tiles: bf16 16 x 8192 x 8192 29.9 / 28.0 / 31.1 us, 16 x 1024 x
+// 16384 15.1 / 18.5 / 26.6, 16 x 16384 x 1024 12.3 / 9.3 / 7.9, 64 x 8192 x 8192
+// 46.9 / 33.4 / 41.9, 64 x 16384 x 8192 91.6 / 64.2 / 50.7.
+int gemm_few_tiles(int64_t rows_s, int64_t rows_l, int64_t row_bytes, double* seconds) {
+  int cus = 0;
+  if (device_cus(&cus) != SILE_OK) cus = 256;
+  int r = 4;
+  while (r > 1 && rows_l < (int64_t)(0.9 * 16 * r * cus)) r /= 2;
+  const int64_t s16 = rows_s <= 16 ? 16 : rows_s <= 32 ? 32 : 64;
+  const int64_t rounds = ((rows_l + 16 * r - 1) / (16 * r) + cus - 1) / cus;
+  *seconds = 3e-6 + std::max((double)((rows_s + rows_l) * row_bytes) / 5.4e12 + 1.5e-6,
+                             (double)rounds * ((double)((16 * r + s16) * row_bytes) / 105e9 + 1.5e-6));
+  return r;
 }
 
 // How the flash kernel's work is laid out: the keys of a query block shared by
@@ -555,6 +575,45 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
                      c, ldc, scale_a, scale_b, 0, tile_req, splits_req, stream);
     scratch_release(s, 1);
     return rc;
+  }
+  // few rows of A or of a column-major B: the kernel that streams the other
+  // operand once, where it is modelled faster than the tiles (or those cannot
+  // take the shape)
+  const int64_t rows_s = std::min(m, n), rows_l = std::max(m, n);
+  if (!b_row && !tile_req && !splits_req && rows_s <= 64 &&
+      64 * std::max(lda, ldb) * (int64_t)eb <= 0x7fffffffLL) {
+    double few_t = 0.0;
+    const int r = gemm_few_tiles(rows_s, rows_l, kp * (int64_t)eb, &few_t);
+    bool use = !lds_ok;
+    if (lds_ok) {
+      const GemmPlan plan = gemm_plan(m, n, kp, (kp + kstep - 1) / kstep, (int64_t)cb, fp8, 0);
+      // (the tiles' model leaves out the operands' bytes and ~4 us of what a
+      // launch of few tiles with a deep split measures)
+      const double bytes = (double)((rows_s + rows_l) * kp) * (double)eb;
+      use = few_t < std::max(plan.seconds, bytes / 5.1e12 + 4e-6 + (plan.splits > 1 ? 5.5e-6 : 0.0)) + 4e-6;
+    }
+    if (use) {
+      const bool l_is_b = m <= n;
+      struct {
+        int64_t ldl, lds, ldc, rows_l, kp;
+        int32_t rows_s, l_is_b, stream_l;
+        float alpha;
+      } fg{l_is_b ? ldb : lda, l_is_b ? lda : ldb, ldc, rows_l, kp, (int32_t)rows_s, l_is_b ? 1 : 0,
+           // past what the 256 MB Infinity Cache holds beside other operands,
+           // non-temporal loads stream faster (16 x 8192 x 8192, 134 MB: 28.0 ->
+           // 24.7 us); below they lose its hits (67 MB: 12.9 -> 13.5)
+           rows_l * kp * (int64_t)eb >= (96ll << 20) ? 1 : 0, scale_a * scale_b};
+      const void* lop = l_is_b ? b : a;
+      const void* sop = l_is_b ? a : b;
+      const int64_t wgs = (rows_l + 16 * r - 1) / (16 * r);
+      if (wgs > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "GEMM too large");
+      char fname[64];
+      snprintf(fname, sizeof fname, "sile_gemm_few_%s_r%dm%d", name + strlen("sile_gemm_nt_"), r,
+               rows_s <= 16 ? 1 : rows_s <= 32 ? 2 : 4);
+      void* fp[] = {&lop, &sop, &c, &fg};
+      int rc = launch(Module::kGemm, fname, dim3((unsigned)wgs), dim3(256), fp, s);
+      return rc == SILE_OK ? ok() : rc;
+    }
   }
   const bool transposed = !b_row && !lds_ok && !capturing && m % 4 == 0 && m >= 128 &&
                           m * n * 4 <= kScratchPlanesMax;

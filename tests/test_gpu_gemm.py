@@ -655,3 +655,61 @@ def test_gemm_tall(hip, m, n, k):
     rows = sorted({0, m - 1} | set(rng(97).integers(0, m, size=62).tolist()))
     ref = a_f[rows].astype(np.float64) @ b_f.astype(np.float64).T
     assert_close(got[rows], ref, atol=ATOL, rtol=RTOL, what="tall GEMM rows")
+
+
+@pytest.mark.parametrize("kind,out", [("bf16", "bf16"), ("bf16", "f32"), ("f16", "f16"),
+                                      ("f16", "f32"), ("fp8", "bf16"), ("fp8", "f32")])
+@pytest.mark.parametrize("m,n,k,bk", [
+    (1, 1, 8, 0), (1, 300, 64, 0), (16, 100, 72, 0), (5, 130, 777, 0),   # K' inside a k-step
+    (17, 257, 1000, 96), (33, 64, 200, 7),      # K' = 960 and 196, NaN past it
+    (64, 1030, 512, 0), (48, 7500, 136, 0),     # 4 tiles of S; 32 rows of L a workgroup
+    (16, 14760, 264, 0), (40, 14760, 80, 0),    # 64 rows a workgroup, the last one partial
+    (3, 4096, 16384, 0), (32, 512, 4096, 0),    # long K', rings that wrap many times
+    (130, 1, 64, 0), (300, 16, 777, 0), (1030, 33, 320, 0), (7500, 64, 100, 0)])  # L is A
+def test_few_rows(hip, kind, out, m, n, k, bk):
+    """One operand of at most 64 rows: the kernel that streams the other one.
+    Row pitches past K, NaN past K' in both operands, C in a wider pitch (odd,
+    so no 16-byte rows) whose columns past N keep their fill."""
+    say(f"few rows {kind}->{out} {m}x{n}x{k} bk={bk}")
+    kp = (k // bk) * bk if bk else k
+    ld = (k + 15) // 16 * 16 + 16
+    ldc = n + 3
+    a = (rng(m + k).normal(size=(m, k)) / (1 if kind == "fp8" else np.sqrt(k))).astype(np.float32)
+    bt = (rng(n + k).normal(size=(n, k)) / (1 if kind == "fp8" else np.sqrt(k))).astype(np.float32)
+    sa = sb = 1.0
+    if kind == "fp8":
+        a_q, sa, a_f = fp8_quantise(a)
+        b_q, sb, b_f = fp8_quantise(bt)
+        fill, t = 0x7F, hip.F8E4M3
+    else:
+        rnd = bf16_round if kind == "bf16" else f16_round
+        (a_q, a_f), (b_q, b_f) = rnd(a), rnd(bt)
+        fill, t = 0x7FFF, hip.BF16 if kind == "bf16" else hip.F16
+    bufs = []
+    for q in (a_q, b_q):
+        host = np.full((q.shape[0], ld), fill, q.dtype)   # NaN outside K'
+        host[:, :kp] = q[:, :kp]
+        bufs.append(hip.DeviceBuffer.from_array(host))
+    ct = {"bf16": hip.BF16, "f16": hip.F16, "f32": hip.F32}[out]
+    cdt = np.float32 if out == "f32" else np.uint16
+    dc = hip.DeviceBuffer(m * ldc * np.dtype(cdt).itemsize)
+    dc.fill_bytes(0x55)
+    hip.gemm(t, t, ct, m, n, k, bufs[0].ptr, ld, hip.ROW_MAJOR, bufs[1].ptr, ld, hip.COL_MAJOR,
+             dc.ptr, ldc, sa, sb, bk)
+    hip.synchronize()
+    raw = dc.download(cdt, (m, ldc))
+    keep = np.frombuffer(b"\x55" * np.dtype(cdt).itemsize, cdt)[0]
+    assert (raw[:, n:] == keep).all()
+    got = np.ascontiguousarray(raw[:, :n])
+    got = (got if out == "f32" else cpuref.f32_from_bf16(got) if out == "bf16"
+           else got.view(np.float16).astype(np.float32))
+    ref = a_f[:, :kp].astype(np.float64) @ b_f[:, :kp].astype(np.float64).T
+    if out == "f32" and kind != "fp8":
+        # fp32 sums of kp products: 2^-24 of the absolute sum a step, far less seen
+        bound = 1e-6 * (np.abs(a_f[:, :kp]).astype(np.float64) @ np.abs(b_f[:, :kp]).astype(np.float64).T)
+        assert (np.abs(got - ref) <= bound + 1e-30).all()
+    else:
+        rms = np.sqrt(np.mean(ref ** 2)) + 1e-30   # fp8: products aligned before they are added
+        assert_close(got, ref, atol=(2e-4 if kind == "fp8" else 1e-5) * rms, rtol=1e-2)
+    for b in bufs + [dc]:
+        b.close()
