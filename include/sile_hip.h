@@ -269,12 +269,11 @@ int sile_hip_kernel_parallel_reduce(void *const *buffers, int64_t num_threadgrou
  *                        row-major B (and every fp8 one) is first written
  *                        column-major into a second device scratch buffer
  *                        (at most 256 MiB; not under graph capture).  MFMA
- *                        path (N a multiple of 4, C's rows 16-byte aligned
- *                        and N >= 128, any M: 256 x 256 or 128 x 128 tiles
+ *                        path (N >= 128, any M, any pitch and start of C:
+ *                        256 x 256 or 128 x 128 tiles
  *                        through LDS,
- *                        the size chosen by shape; when C cannot take the
- *                        tiles' stores but M is a multiple of 4 and at least
- *                        one tile, the same kernels compute C^T into fp32
+ *                        the size chosen by shape; when N is below one tile
+ *                        but M is not, the same kernels compute C^T into fp32
  *                        scratch and a second kernel writes C; other shapes:
  *                        64 x 64 tiles).  When A or a column-major B has at
  *                        most 64 rows, a kernel that streams the other operand

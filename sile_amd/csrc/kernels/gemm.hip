@@ -27,17 +27,21 @@ enum Out : int { kOutBF16 = 0, kOutF16 = 1, kOutF32 = 2 };
 // fp32 C goes straight from the accumulators, 32 or 64 bytes of a row per
 // instruction: plain stores, so that L2 merges a row's pieces into whole
 // lines (non-temporal ones made the fp8 kernel's fp32 C 1.3x and its split-K
-// planes up to 2.7x slower).
+// planes up to 2.7x slower).  Stores of 8 and 16 bytes go to any element of C
+// (the memory pipeline takes unaligned ones), so C may have any pitch and start.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned int u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
 template <int kOut>
 SILE_DEV void store_c4(void* C, int64_t idx, f32x4 v) {
   if constexpr (kOut == kOutF32) {
-    *reinterpret_cast<f32x4*>(static_cast<float*>(C) + idx) = v;
+    *reinterpret_cast<f32x4_any*>(static_cast<float*>(C) + idx) = v;
   } else if constexpr (kOut == kOutBF16) {
     const u32x2 w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-    __builtin_nontemporal_store(w, reinterpret_cast<u32x2*>(static_cast<uint16_t*>(C) + idx));
+    __builtin_nontemporal_store(w, reinterpret_cast<u32x2_any*>(static_cast<uint16_t*>(C) + idx));
   } else {
     const u32x2 w = {pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
-    __builtin_nontemporal_store(w, reinterpret_cast<u32x2*>(static_cast<uint16_t*>(C) + idx));
+    __builtin_nontemporal_store(w, reinterpret_cast<u32x2_any*>(static_cast<uint16_t*>(C) + idx));
   }
 }
 
@@ -206,8 +210,7 @@ SILE_DEV void mma16x16(const u32x4& a, const u32x4& b, f32x4& c) {
 // into LDS rows of 2 kW + 16 bytes (the pad puts the rows that one put
 // instruction of the accumulator layouts writes on distinct banks), then
 // written back so that each store instruction covers whole 2 kW-byte rows of
-// C (16-byte stores, 512 / kW rows per instruction; 8-byte stores, half as
-// many, when C's rows are not 16-byte aligned).  Writing straight from the accumulator layouts touches 16 or 32
+// C (16-byte stores, 512 / kW rows per instruction).  Writing straight from the accumulator layouts touches 16 or 32
 // rows per instruction with 8 bytes each and ran 5 % slower at 8192^3, with
 // twice C's size written to HBM.  fill(put) calls put(row, col, v) for 4
 // consecutive columns of the wave's tile; the wave's LDS region is its own.
@@ -230,26 +233,14 @@ SILE_DEV void stage_and_store_c(void* C, int64_t ldc, int64_t m0, int64_t n0, ui
   __builtin_amdgcn_wave_barrier();
   const int lane = threadIdx.x & 63;
   uint16_t* cbase = static_cast<uint16_t*>(C) + m0 * ldc + n0;
-  if ((ldc & 7) == 0 && (reinterpret_cast<uintptr_t>(cbase) & 15) == 0) {
-    constexpr int kLanesPerRow = kW / 8, kRowsPerStore = 64 / kLanesPerRow;
-    const int lr = lane % kLanesPerRow, lg = lane / kLanesPerRow;
+  constexpr int kLanesPerRow = kW / 8, kRowsPerStore = 64 / kLanesPerRow;
+  const int lr = lane % kLanesPerRow, lg = lane / kLanesPerRow;
 #pragma unroll 8
-    for (int t = 0; t < kW / kRowsPerStore; ++t) {
-      const int row = kRowsPerStore * t + lg;
-      if (kGuardRows && row >= rows) continue;
-      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(cst + row * kRowBytes + lr * 16),
-                                  reinterpret_cast<u32x4*>(cbase + row * ldc + lr * 8));
-    }
-  } else {
-    constexpr int kLanesPerRow = kW / 4, kRowsPerStore = 64 / kLanesPerRow;
-    const int lr = lane % kLanesPerRow, lg = lane / kLanesPerRow;
-#pragma unroll 8
-    for (int t = 0; t < kW / kRowsPerStore; ++t) {
-      const int row = kRowsPerStore * t + lg;
-      if (kGuardRows && row >= rows) continue;
-      __builtin_nontemporal_store(*reinterpret_cast<const u32x2*>(cst + row * kRowBytes + lr * 8),
-                                  reinterpret_cast<u32x2*>(cbase + row * ldc + lr * 4));
-    }
+  for (int t = 0; t < kW / kRowsPerStore; ++t) {
+    const int row = kRowsPerStore * t + lg;
+    if (kGuardRows && row >= rows) continue;
+    __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(cst + row * kRowBytes + lr * 16),
+                                reinterpret_cast<u32x4_any*>(cbase + row * ldc + lr * 8));
   }
 }
 
@@ -621,25 +612,26 @@ SILE_GEMM_KERNEL_B(sile_gemm_nn128_f16_f32, kF16, kOutF32, 128, true)
 // tile of 128 x 128 bytes (128 rows of 128 or 64 elements) through LDS:
 // 16-byte loads along the input rows, 16-byte stores along the output rows
 // (each gathered from 16 / sizeof(T) input rows in LDS), when the tile lies
-// inside both matrices and `vec` says rows start on 16-byte boundaries;
-// element by element otherwise.  LDS rows are padded by 4 bytes, so the
+// inside both matrices; element by element otherwise.  Input rows may start
+// anywhere, output rows on 16-byte boundaries.  LDS rows are padded by 4 bytes, so the
 // gathers of one column touch distinct banks.
 template <typename T>
 __device__ __forceinline__ void transpose_body(const T* __restrict__ in, int64_t ldi,
                                                T* __restrict__ out, int64_t ldo, int64_t rows,
-                                               int64_t cols, int vec) {
+                                               int64_t cols) {
+  typedef unsigned int Chunk __attribute__((ext_vector_type(4), aligned(1)));
   constexpr int kR = 128, kC = 128 / sizeof(T), kE = 16 / sizeof(T);  // tile rows, cols
   constexpr int kPitch = 128 + 4;                                       // LDS row bytes
   __shared__ __attribute__((aligned(16))) uint8_t tile[kR * kPitch];
   const int t = threadIdx.x;
   const int64_t r0 = (int64_t)blockIdx.y * kR, c0 = (int64_t)blockIdx.x * kC;
   auto at = [&](int r, int c) -> T& { return *reinterpret_cast<T*>(tile + r * kPitch + c * sizeof(T)); };
-  if (vec && r0 + kR <= rows && c0 + kC <= cols) {
+  if (r0 + kR <= rows && c0 + kC <= cols) {
     // 128 rows x 8 chunks in, 4 a thread
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int e = j * 256 + t, r = e >> 3, ch = e & 7;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(in + (r0 + r) * ldi + c0 + ch * kE);
+      const u32x4 v = *reinterpret_cast<const Chunk*>(in + (r0 + r) * ldi + c0 + ch * kE);
       uint32_t* d = reinterpret_cast<uint32_t*>(tile + r * kPitch + ch * 16);
       d[0] = v[0]; d[1] = v[1]; d[2] = v[2]; d[3] = v[3];
     }
@@ -677,34 +669,34 @@ __device__ __forceinline__ void transpose_body(const T* __restrict__ in, int64_t
 }
 extern "C" __global__ __launch_bounds__(256) void sile_transpose_e1(const uint8_t* in, int64_t ldi,
                                                                     uint8_t* out, int64_t ldo,
-                                                                    int64_t rows, int64_t cols,
-                                                                    int vec) {
-  transpose_body<uint8_t>(in, ldi, out, ldo, rows, cols, vec);
+                                                                    int64_t rows, int64_t cols) {
+  transpose_body<uint8_t>(in, ldi, out, ldo, rows, cols);
 }
 extern "C" __global__ __launch_bounds__(256) void sile_transpose_e2(const uint16_t* in,
                                                                     int64_t ldi, uint16_t* out,
                                                                     int64_t ldo, int64_t rows,
-                                                                    int64_t cols, int vec) {
-  transpose_body<uint16_t>(in, ldi, out, ldo, rows, cols, vec);
+                                                                    int64_t cols) {
+  transpose_body<uint16_t>(in, ldi, out, ldo, rows, cols);
 }
 
 // Split K: the ring kernel above writes one fp32 plane of C per k-range
-// (planes `plane` elements apart, rows n elements long); this kernel adds the
-// planes in k-range order, scales by alpha and writes C in its type.  N is a
-// multiple of 4; workgroup (x, y) takes 4-element groups 256 x + t of rows
-// y, y + gridDim.y, ...
+// (planes `plane` elements apart, rows `pitch` elements apart); this kernel adds the
+// planes in k-range order, scales by alpha and writes C in its type.
+// Workgroup (x, y) takes 4-element groups 256 x + t of rows y, y + gridDim.y,
+// ... (the last group of a row moved back to end at N, at least 4).
 template <int kOut>
 __device__ __forceinline__ void splitk_reduce_body(const float* __restrict__ ws,
                                                    void* __restrict__ C, int64_t ldc, int64_t m,
-                                                   int64_t n, int64_t plane, int splits,
-                                                   float alpha) {
-  const int64_t c4 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+                                                   int64_t n, int64_t plane, int64_t pitch,
+                                                   int splits, float alpha) {
+  int64_t c4 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (c4 >= n) return;
+  c4 = min(c4, n - 4);
   for (int64_t row = blockIdx.y; row < m; row += gridDim.y) {
-    const float* src = ws + row * n + c4;
-    f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src));
+    const float* src = ws + row * pitch + c4;
+    f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(src));
     for (int z = 1; z < splits; ++z)
-      v += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + z * plane));
+      v += __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(src + z * plane));
     if (alpha != 1.0f) v *= alpha;
     store_c4<kOut>(C, row * ldc + c4, v);
   }
@@ -713,8 +705,9 @@ __device__ __forceinline__ void splitk_reduce_body(const float* __restrict__ ws,
 #define SILE_GEMM_SPLITK_REDUCE(NAME, OUT)                                                    \
   extern "C" __global__ __launch_bounds__(256) void NAME(const float* ws, void* C, int64_t ldc, \
                                                          int64_t m, int64_t n, int64_t plane,   \
-                                                         int splits, float alpha) {             \
-    splitk_reduce_body<OUT>(ws, C, ldc, m, n, plane, splits, alpha);                          \
+                                                         int64_t pitch, int splits,             \
+                                                         float alpha) {                         \
+    splitk_reduce_body<OUT>(ws, C, ldc, m, n, plane, pitch, splits, alpha);                   \
   }
 SILE_GEMM_SPLITK_REDUCE(sile_gemm_splitk_reduce_bf16, kOutBF16)
 SILE_GEMM_SPLITK_REDUCE(sile_gemm_splitk_reduce_f16, kOutF16)
@@ -775,7 +768,8 @@ SILE_GEMM_SPLITK_REDUCE_T(sile_gemm_splitk_reduce_t_f16, kOutF16)
 SILE_GEMM_SPLITK_REDUCE_T(sile_gemm_splitk_reduce_t_f32, kOutF32)
 
 // ---------------------------------------------------------------------------
-// Any shape: M or N below one 256 x 256 tile, or N not a multiple of 4.
+// Any shape: N below one 128 x 128 tile (and M too, or its C^T scratch not at
+// hand).
 //
 // 64 x 64 output tile per workgroup of 4 waves (2 x 2), a 32 x 32 block per
 // wave on v_mfma_f32_32x32x16_{bf16,f16} (16 k per MFMA) or
@@ -1145,8 +1139,7 @@ __device__ __forceinline__ void gemm_few_body(const uint8_t* __restrict__ L,
     if (g.alpha != 1.0f) v *= g.alpha;
     const int64_t lr = l0 + 4 * lq;
     const int64_t idx = g.l_is_b ? sr * g.ldc + lr : lr * g.ldc + sr;
-    if (g.l_is_b && lr + 4 <= g.rows_l && (g.ldc & 3) == 0 &&
-        (reinterpret_cast<uintptr_t>(C) & (kOut == kOutF32 ? 15 : 7)) == 0) {
+    if (g.l_is_b && lr + 4 <= g.rows_l) {
       store_c4<kOut>(C, idx, v);
       continue;
     }

@@ -517,19 +517,17 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
   if ((lda * eb) % 16 || !aligned16(a) || (!b_row && ((ldb * eb) % 16 || !aligned16(b))))
     return fail(SILE_ERR_SHAPE, "A, B and their leading dimensions must be 16-byte aligned");
   // the LDS kernels need N >= the tile edge (128 x 128 tiles take any M,
-  // 256 x 256 tiles M >= 256)
+  // 256 x 256 tiles M >= 256); a forced tile also asks for the rows of C that
+  // the header names
   const int64_t min_tile = tile_req ? tile_req : 128;
-  const bool lds_ok = (min_tile == 128 || m >= min_tile) && n >= min_tile && n % 4 == 0 &&
-                      (ldc * cb) % 16 == 0 && aligned16(c);
-  if (tile_req && !lds_ok)
+  const bool lds_ok = (min_tile == 128 || m >= min_tile) && n >= min_tile;
+  if (tile_req && !(lds_ok && n % 4 == 0 && (ldc * cb) % 16 == 0 && aligned16(c)))
     return fail(SILE_ERR_SHAPE,
                 "%d x %d tiles need %sN >= %d, N a multiple of 4 and C's rows 16-byte aligned",
                 tile_req, tile_req, tile_req == 256 ? "M, " : "", tile_req);
   // The transposed form runs C^T = B . A^T (A and B swapped) into fp32
-  // planes of C^T and writes them back transposed, for the shapes the direct
-  // form cannot take (N below one tile, N not a multiple of 4, C's rows not
-  // 16-byte aligned) whose M can be the column extent: a multiple of 4 and
-  // at least one tile.
+  // planes of C^T and writes them back transposed, where N is below one tile
+  // and M, as the column extent, is not.
   // Its fp32 planes (all of C^T) are kept to kScratchPlanesMax bytes.  The
   // forms that use the device scratch (this one and the K split) are left
   // out while the stream is being captured into a graph: the scratch is
@@ -560,8 +558,7 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
     int rc = scratch_acquire((size_t)(n * ldt) * eb, s, &bt, 1);
     if (rc != SILE_OK) return rc;
     int64_t rows = kp, cols = n, ldi = ldb, ldo = ldt;
-    int vec = (ldb * (int64_t)eb) % 16 == 0 && aligned16(b) ? 1 : 0;   // B^T rows are aligned
-    void* tp[] = {(void*)&b, &ldi, &bt, &ldo, &rows, &cols, &vec};
+    void* tp[] = {(void*)&b, &ldi, &bt, &ldo, &rows, &cols};
     const int64_t tcols = 128 / (int64_t)eb;   // a tile: 128 rows of 128 bytes
     if ((kp + 127) / 128 > 65535) {
       rc = fail(SILE_ERR_SHAPE, "K too large for the transpose");
@@ -615,8 +612,8 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
       return rc == SILE_OK ? ok() : rc;
     }
   }
-  const bool transposed = !b_row && !lds_ok && !capturing && m % 4 == 0 && m >= 128 &&
-                          m * n * 4 <= kScratchPlanesMax;
+  const bool transposed = !b_row && !lds_ok && !capturing && m >= 128 &&
+                          (m + 3) / 4 * 4 * n * 4 <= kScratchPlanesMax;
   if (!lds_ok && !transposed) {
     // the any-shape kernel, 64 x 64 tiles with fragments loaded straight
     // from the operands
@@ -639,6 +636,7 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
   const void* rb = transposed ? a : b;
   const int64_t rlda = transposed ? ldb : lda, rldb = transposed ? lda : ldb;
   const int64_t rm = transposed ? n : m, rn = transposed ? m : n;
+  const int64_t pitch = (rn + 3) / 4 * 4;   // of a row of the fp32 planes
   // a tile's panel of A or B is one buffer resource: 32-bit byte range
   if (256 * std::max(lda, b_row ? 0 : ldb) * (int64_t)eb > 0x7fffffffLL)
     return fail(SILE_ERR_SHAPE, "leading dimension too large for a 256-row panel (%lld, %lld)",
@@ -648,13 +646,13 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
   if (half_steps > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "GEMM K too large");
   GemmPlan plan = gemm_plan(rm, rn, kp, half_steps, (int64_t)cb, fp8, tile_req);
   if (splits_req) plan.splits = splits_req;
-  if (splits_req > 1 && (double)splits_req * (double)rm * (double)rn * 4.0 > (double)kScratchPlanesMax)
+  if (splits_req > 1 && (double)splits_req * (double)rm * (double)pitch * 4.0 > (double)kScratchPlanesMax)
     return fail(SILE_ERR_SHAPE,
                 "%d k-ranges of %lld x %lld fp32 planes exceed the %lld MiB of device scratch a "
                 "GEMM may use", splits_req, (long long)rm, (long long)rn,
                 (long long)(kScratchPlanesMax >> 20));
   if (capturing) plan.splits = 1;
-  if (transposed) plan.splits = std::max<int64_t>(1, std::min(plan.splits, kScratchPlanesMax / (rm * rn * 4)));
+  if (transposed) plan.splits = std::max<int64_t>(1, std::min(plan.splits, kScratchPlanesMax / (rm * pitch * 4)));
   const int64_t tiles_m = (rm + plan.tile - 1) / plan.tile;
   const int64_t tiles_n = (rn + plan.tile - 1) / plan.tile;
   if (tiles_m * tiles_n > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "GEMM too large");
@@ -680,35 +678,34 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
     int rc = launch(Module::kGemm, kname, dim3(tiles), dim3(256), params, s);
     return rc == SILE_OK ? ok() : rc;
   }
-  // fp32 planes in the device scratch (one per k-range; rows of rn, a
-  // multiple of 4), then their sum in k-range order, scaled, converted and,
+  // fp32 planes in the device scratch (one per k-range), then their sum in k-range order, scaled, converted and,
   // for the transposed form, transposed
   void* ws = nullptr;
-  int rc = scratch_acquire((size_t)(splits * rm * rn) * sizeof(float), s, &ws);
+  int rc = scratch_acquire((size_t)(splits * rm * pitch) * sizeof(float), s, &ws);
   if (rc != SILE_OK) return rc;
   snprintf(kname, sizeof kname, "%s%s_f32", tname, ab);
   const float alpha = g.alpha;
   g.alpha = 1.0f;
-  g.ldc = rn;
-  g.c_split = rm * rn;
+  g.ldc = pitch;
+  g.c_split = rm * pitch;
   void* params[] = {&ra, &rb, &ws, &g};
   rc = launch(Module::kGemm, kname, dim3(tiles, (unsigned)splits), dim3(256), params, s);
   if (rc == SILE_OK) {
     const char* out = c_type == SILE_BF16 ? "bf16" : c_type == SILE_F16 ? "f16" : "f32";
     char rname[64];
-    int64_t plane = rm * rn, ldc_ = ldc, m_ = m, n_ = n, pitch = rn;
+    int64_t plane = rm * pitch, ldc_ = ldc, m_ = m, n_ = n, pitch_ = pitch;
     int sp = (int)splits;
     float al = alpha;
     if (transposed) {
       snprintf(rname, sizeof rname, "sile_gemm_splitk_reduce_t_%s", out);
-      void* rp[] = {&ws, &c, &ldc_, &m_, &n_, &plane, &pitch, &sp, &al};
+      void* rp[] = {&ws, &c, &ldc_, &m_, &n_, &plane, &pitch_, &sp, &al};
       rc = launch(Module::kGemm, rname, dim3((unsigned)((m + 31) / 32), (unsigned)((n + 63) / 64)),
                   dim3(256), rp, s);
     } else {
       snprintf(rname, sizeof rname, "sile_gemm_splitk_reduce_%s", out);
-      void* rp[] = {&ws, &c, &ldc_, &m_, &n_, &plane, &sp, &al};
+      void* rp[] = {&ws, &c, &ldc_, &m_, &n_, &plane, &pitch_, &sp, &al};
       rc = launch(Module::kGemm, rname,
-                  dim3((unsigned)((n / 4 + 255) / 256), (unsigned)std::min<int64_t>(m, 65535)),
+                  dim3((unsigned)(((n + 3) / 4 + 255) / 256), (unsigned)std::min<int64_t>(m, 65535)),
                   dim3(256), rp, s);
     }
   }

@@ -713,3 +713,52 @@ def test_few_rows(hip, kind, out, m, n, k, bk):
         assert_close(got, ref, atol=(2e-4 if kind == "fp8" else 1e-5) * rms, rtol=1e-2)
     for b in bufs + [dc]:
         b.close()
+
+
+@pytest.mark.parametrize("kind,out", [("bf16", "bf16"), ("bf16", "f32"), ("f16", "f16"), ("fp8", "bf16"),
+                                      ("fp8", "f32")])
+@pytest.mark.parametrize("layout", ["col", "row"])
+@pytest.mark.parametrize("m,n,k,pad", [
+    (129, 129, 96, 0), (300, 131, 208, 1), (257, 513, 320, 3),   # N odd, C's rows at any element
+    (70, 255, 4096, 0), (128, 130, 8192, 5),                     # K' split: planes of odd rows
+    (2051, 2049, 128, 0),                                        # 256 x 256 tiles
+    (131, 101, 128, 0), (203, 127, 4096, 1)])                    # C^T planes, M not a multiple of 4
+def test_any_pitch_of_c(hip, kind, out, layout, m, n, k, pad):
+    """N and C's pitch and start at any element: the LDS tiles, the split-K sum
+    and the transposed form, every element against a float64 product; the pitch
+    padding keeps its fill.  Row-major B of odd N goes through the transpose."""
+    say(f"any C {kind}->{out} B {layout} {m}x{n}x{k} pad={pad}")
+    scale = 1 if kind == "fp8" else np.sqrt(k)
+    a = (rng(m + k).normal(size=(m, k)) / scale).astype(np.float32)
+    bt = (rng(n + k).normal(size=(n, k)) / scale).astype(np.float32)
+    sa = sb = 1.0
+    if kind == "fp8":
+        (a_q, sa, a_f), (b_q, sb, b_f) = fp8_quantise(a), fp8_quantise(bt)
+        t = hip.F8E4M3
+    else:
+        rnd = bf16_round if kind == "bf16" else f16_round
+        (a_q, a_f), (b_q, b_f) = rnd(a), rnd(bt)
+        t = hip.BF16 if kind == "bf16" else hip.F16
+    da = hip.DeviceBuffer.from_array(a_q)
+    db = hip.DeviceBuffer.from_array(b_q if layout == "col" else np.ascontiguousarray(b_q.T))
+    ct = {"bf16": hip.BF16, "f16": hip.F16, "f32": hip.F32}[out]
+    cdt = np.dtype(np.float32 if out == "f32" else np.uint16)
+    ldc = n + pad
+    dc = hip.DeviceBuffer((1 + m * ldc) * cdt.itemsize)
+    dc.fill_bytes(0x55)
+    hip.gemm(t, t, ct, m, n, k, da.ptr, k, hip.ROW_MAJOR, db.ptr, k if layout == "col" else n,
+             hip.COL_MAJOR if layout == "col" else hip.ROW_MAJOR, dc.ptr + cdt.itemsize, ldc, sa, sb)
+    hip.synchronize()
+    raw = dc.download(cdt, (1 + m * ldc,))
+    keep = np.frombuffer(b"\x55" * cdt.itemsize, cdt)[0]
+    assert raw[0] == keep and (raw[1:].reshape(m, ldc)[:, n:] == keep).all()
+    got = np.ascontiguousarray(raw[1:].reshape(m, ldc)[:, :n])
+    got = (got if out == "f32" else cpuref.f32_from_bf16(got) if out == "bf16"
+           else got.view(np.float16).astype(np.float32))
+    ref = a_f.astype(np.float64) @ b_f.astype(np.float64).T
+    rms = np.sqrt(np.mean(ref ** 2))
+    # 16-bit C: its rounding; fp32 C: fp32 sums (fp8: products aligned before they are added)
+    atol, rtol = (2e-4, 1e-2) if kind == "fp8" else (1e-5, 1e-5 if out == "f32" else 1e-2)
+    assert_close(got, ref, atol=atol * rms, rtol=rtol)
+    for b in (da, db, dc):
+        b.close()
