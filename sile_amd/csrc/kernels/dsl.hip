@@ -249,144 +249,113 @@ __device__ __forceinline__ void matvec_rows(const float* __restrict__ x, const f
   if (lane == 0) out[row] = acc;
 }
 
-// BK = 4 L with L = 1, 2, 4, 8 or 16 lanes a tile, x rows, y and BK allowing
-// 16-byte loads: the wave reads the row 256 elements at a time with one
-// 16-byte load per lane (coalesced; four such spans in flight), lane j holding
-// elements 4 j .. 4 j + 3 of a span, so tile g of a span lives on lanes
-// g L .. g L + L - 1 of one 16-lane DPP row.  Its sequential sum is carried
-// from lane to lane in L steps (a DPP shift by one lane), each lane adding its
-// four products in order, so the tile's partial, on its last lane, is the
-// reference's chain; the partials are then added to the accumulator in tile
-// order as above.
-template <int kL>
-__device__ __forceinline__ void matvec_rows_chain(const float* __restrict__ x,
-                                                  const float* __restrict__ y,
-                                                  float* __restrict__ out, const MatvecArgs& a) {
-#pragma clang fp contract(off)
-  constexpr int kU = 4;              // spans in flight
-  const int lane = threadIdx.x & 63, s = lane % kL;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= a.m) return;   // the whole wave
-  const float* xr = x + row * a.ldx;
-  const int64_t n = a.tiles * 4 * kL;   // elements of the whole tiles
-  float acc = a.seed;
-  for (int64_t base = 0; base < n; base += 256 * kU) {
-    f32x4 xv[kU], yv[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int64_t e = base + 256 * u + 4 * lane;
-      xv[u] = yv[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (e < n) {
-        xv[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(xr + e));
-        yv[u] = *reinterpret_cast<const f32x4*>(y + e);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int64_t b = base + 256 * u;
-      if (b >= n) break;
-      const float p0 = xv[u][0] * yv[u][0], p1 = xv[u][1] * yv[u][1];
-      const float p2 = xv[u][2] * yv[u][2], p3 = xv[u][3] * yv[u][3];
-      float p = 0.0f, carry = 0.0f;
-#pragma unroll
-      for (int step = 0; step < kL; ++step) {
-        float c = step == 0 ? p0 : carry + p0;
-        c = c + p1;
-        c = c + p2;
-        c = c + p3;
-        p = s == step ? c : p;
-        if (step + 1 < kL) carry = dpp<0x111>(p);   // row_shr:1
-      }
-      const int g_n = (int)min<int64_t>(64 / kL, (n - b) / (4 * kL));
-      for (int g = 0; g < g_n; ++g)
-        acc = acc + __builtin_bit_cast(
-                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), g * kL + kL - 1));
-    }
-  }
-  if (lane == 0) out[row] = acc;
-}
-
-// The same with kR rows per wave (the wave's rows read in turn, y once for
-// them all): each tile partial goes to LDS, and lane r < kR adds row r's
-// partials to its accumulator in tile order, so one add advances kR rows.
+// BK = 4 L with L = 1, 2, 4, 8 or 16 lanes a tile: a workgroup of 256 threads
+// takes kR rows, kU spans of 1024 elements of each at a time, one 16-byte load
+// a thread, row and span (coalesced; the next block's loads in flight).  Thread
+// t holds elements 4 t .. 4 t + 3 of a span, so a tile lies on L lanes of one
+// 16-lane DPP row.  Its sequential sum is carried from lane to lane in L steps
+// (a DPP shift by one lane), each lane adding its four products in order: the
+// tile's partial, on its last lane, is the reference's chain.  Partials go to
+// LDS, and lane r of the first wave adds row r's to its accumulator in tile
+// order while the others form the next block's (two LDS halves, one barrier a
+// block).  The ordered adds, ~8 clocks each, bound small BK: with a wave a row
+// (its adds between its own loads) 512 x 8192 ran 44 us at BK = 4 and 18 at 32,
+// and rows not 16-byte aligned a lane a tile (3000 x 3001, BK = 32: 58 us); now
+// 15.0, 6.2 and 7.9 us, and 8192 x 8192 51.9 -> 43.2 (6.2 TB/s).
 template <int kL, int kR, int kU>
-__device__ __forceinline__ void matvec_rows_multi(const float* __restrict__ x,
+__device__ __forceinline__ void matvec_rows_block(const float* __restrict__ x,
                                                   const float* __restrict__ y,
                                                   float* __restrict__ out, const MatvecArgs& a) {
 #pragma clang fp contract(off)
-  constexpr int kG = 64 / kL;        // tiles per span
-  __shared__ float part[4][kR][kG];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, s = lane % kL;
-  const int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * kR;
-  if (row0 >= a.m) return;   // the whole wave
+  typedef float Chunk __attribute__((ext_vector_type(4), aligned(4)));   // any element
+  constexpr int kG = 256 / kL;       // tiles per span
+  constexpr int kPitch = kU * kG + 4;
+  __shared__ __attribute__((aligned(16))) float part[2][kR][kPitch];
+  const int t = threadIdx.x, s = t % kL;
+  const int64_t row0 = (int64_t)blockIdx.x * kR;
+  const int rows = (int)min<int64_t>(kR, a.m - row0);
   const int64_t n = a.tiles * 4 * kL;   // elements of the whole tiles
-  float acc = a.seed;                   // lane r < kR: row row0 + r
-  for (int64_t base = 0; base < n; base += 256 * kU) {
-    f32x4 yv[kU], xv[kU][kR];
+  f32x4 xv[kU][kR], yv[kU];
+  auto load = [&](int64_t base) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
-      const int64_t e = base + 256 * u + 4 * lane;
+      const int64_t e = base + 1024 * u + 4 * t;
       yv[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (e < n) yv[u] = *reinterpret_cast<const f32x4*>(y + e);
+      if (e < n) yv[u] = *reinterpret_cast<const Chunk*>(y + e);
 #pragma unroll
       for (int r = 0; r < kR; ++r) {
         xv[u][r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (e < n && row0 + r < a.m)
+        if (e < n && r < rows)
           xv[u][r] = __builtin_nontemporal_load(
-              reinterpret_cast<const f32x4*>(x + (row0 + r) * a.ldx + e));
+              reinterpret_cast<const Chunk*>(x + (row0 + r) * a.ldx + e));
       }
     }
+  };
+  float acc = a.seed;                // thread r < kR: row row0 + r
+  if (n > 0) load(0);
+  int half = 0;
+  for (int64_t base = 0; base < n; base += 1024 * kU, half ^= 1) {
+    float p0[kU][kR], p1[kU][kR], p2[kU][kR], p3[kU][kR];
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int64_t b = base + 256 * u;
-      if (b >= n) break;
+    for (int u = 0; u < kU; ++u)
 #pragma unroll
       for (int r = 0; r < kR; ++r) {
-        const float p0 = xv[u][r][0] * yv[u][0], p1 = xv[u][r][1] * yv[u][1];
-        const float p2 = xv[u][r][2] * yv[u][2], p3 = xv[u][r][3] * yv[u][3];
+        p0[u][r] = xv[u][r][0] * yv[u][0];
+        p1[u][r] = xv[u][r][1] * yv[u][1];
+        p2[u][r] = xv[u][r][2] * yv[u][2];
+        p3[u][r] = xv[u][r][3] * yv[u][3];
+      }
+    if (base + 1024 * kU < n) load(base + 1024 * kU);
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int r = 0; r < kR; ++r) {
         float p = 0.0f, carry = 0.0f;
 #pragma unroll
         for (int step = 0; step < kL; ++step) {
-          float c = step == 0 ? p0 : carry + p0;
-          c = c + p1;
-          c = c + p2;
-          c = c + p3;
+          float c = step == 0 ? p0[u][r] : carry + p0[u][r];
+          c = c + p1[u][r];
+          c = c + p2[u][r];
+          c = c + p3[u][r];
           p = s == step ? c : p;
           if (step + 1 < kL) carry = dpp<0x111>(p);   // row_shr:1
         }
-        if (s == kL - 1) part[wave][r][lane / kL] = p;
+        if (s == kL - 1) part[half][r][u * kG + t / kL] = p;
       }
-      __builtin_amdgcn_wave_barrier();
-      const int g_n = (int)min<int64_t>(kG, (n - b) / (4 * kL));
-      if (lane < kR)
-        for (int g = 0; g < g_n; ++g) acc = acc + part[wave][lane][g];
-      __builtin_amdgcn_wave_barrier();
+    __syncthreads();
+    if (t < kR) {
+      const int tiles = (int)min<int64_t>(kU * kG, (n - base) / (4 * kL));
+      const float* w = part[half][t];
+      const int t4 = tiles & ~3;
+#pragma unroll 4
+      for (int i = 0; i < t4; i += 4) {
+        const f32x4 q = *reinterpret_cast<const f32x4*>(w + i);
+        acc = acc + q[0];
+        acc = acc + q[1];
+        acc = acc + q[2];
+        acc = acc + q[3];
+      }
+      for (int i = t4; i < tiles; ++i) acc = acc + w[i];
     }
   }
-  if (lane < kR && row0 + lane < a.m) out[row0 + lane] = acc;
+  if (t < rows) out[row0 + t] = acc;
 }
 
-#define SILE_MATVEC_MULTI(L, R, U)                                                             \
+#define SILE_MATVEC_BLOCK(L, R, U)                                                             \
   extern "C" __global__ __launch_bounds__(256) void sile_dsl_matvec_f32_l##L##_r##R(           \
       const float* x, const float* y, float* out, MatvecArgs a) {                              \
-    matvec_rows_multi<L, R, U>(x, y, out, a);                                                  \
+    matvec_rows_block<L, R, U>(x, y, out, a);                                                  \
   }
-// BK = 4 and 8 (16 or 32 tiles a span): 8 rows a wave, 4.73 and 4.84 TB/s
-// at 8192^2 against 2.08 and 3.70 with a row a wave; from BK = 16 on the
-// row-a-wave kernels are faster (4.82 TB/s at 16 against 4.64 with 8 rows)
-SILE_MATVEC_MULTI(1, 8, 2)
-SILE_MATVEC_MULTI(2, 8, 2)
-
-#define SILE_MATVEC_CHAIN(L)                                                                   \
-  extern "C" __global__ __launch_bounds__(256) void sile_dsl_matvec_f32_l##L(                 \
-      const float* x, const float* y, float* out, MatvecArgs a) {                              \
-    matvec_rows_chain<L>(x, y, out, a);                                                        \
-  }
-SILE_MATVEC_CHAIN(1)
-SILE_MATVEC_CHAIN(2)
-SILE_MATVEC_CHAIN(4)
-SILE_MATVEC_CHAIN(8)
-SILE_MATVEC_CHAIN(16)
+SILE_MATVEC_BLOCK(1, 4, 1)
+SILE_MATVEC_BLOCK(2, 4, 1)
+SILE_MATVEC_BLOCK(4, 4, 1)
+SILE_MATVEC_BLOCK(8, 4, 1)
+SILE_MATVEC_BLOCK(16, 4, 1)
+SILE_MATVEC_BLOCK(1, 1, 4)
+SILE_MATVEC_BLOCK(2, 1, 4)
+SILE_MATVEC_BLOCK(4, 1, 4)
+SILE_MATVEC_BLOCK(8, 1, 4)
+SILE_MATVEC_BLOCK(16, 1, 4)
 
 extern "C" __global__ __launch_bounds__(256) void sile_dsl_matvec_f32(const float* x,
                                                                        const float* y, float* out,

@@ -770,19 +770,19 @@ int sile_hip_matvec_f32(int64_t m, int64_t k, int64_t bk, const float* x, int64_
     int64_t m, ldx, tiles, bk;
     float seed;
   } args{m, ldx, k / bk, bk, seed};
-  // 16-byte loads when every tile of every row starts on a 16-byte boundary;
-  // tiles of 1 .. 16 such chunks: coalesced spans with the chain carried
-  // across lanes, else a lane per tile
-  const bool vec4 = bk % 4 == 0 && ldx % 4 == 0 && aligned16(x) && aligned16(y);
-  // (BK 4 and 8: 8 rows a wave, so that one in-order add serves 8 rows)
+  // tiles of 1 .. 16 16-byte chunks: coalesced spans, the chain carried across
+  // lanes; any other BK a lane a tile (16-byte loads where every tile of every
+  // row starts on a 16-byte boundary)
   char name[40];
   int64_t rows_per_block = 4;
-  if (vec4 && (bk == 4 || bk == 8)) {
-    snprintf(name, sizeof name, "sile_dsl_matvec_f32_l%d_r8", (int)(bk / 4));
-    rows_per_block = 32;
-  } else if (vec4 && (bk == 16 || bk == 32 || bk == 64)) {
-    snprintf(name, sizeof name, "sile_dsl_matvec_f32_l%d", (int)(bk / 4));
+  if (bk == 4 || bk == 8 || bk == 16 || bk == 32 || bk == 64) {
+    // a row a workgroup (four spans of it in flight) while that is needed to
+    // fill the CUs: 512 x 8192, BK 32: 6.2 us against 9.0 with four rows; 2048 x
+    // 8192: 14.3 against 13.8, 2048 x 2048, BK 8: 6.3 against 5.9
+    rows_per_block = m <= 1024 ? 1 : 4;
+    snprintf(name, sizeof name, "sile_dsl_matvec_f32_l%d_r%d", (int)(bk / 4), (int)rows_per_block);
   } else {
+    const bool vec4 = bk % 4 == 0 && ldx % 4 == 0 && aligned16(x) && aligned16(y);
     snprintf(name, sizeof name, "%s", vec4 ? "sile_dsl_matvec_f32_v4" : "sile_dsl_matvec_f32");
   }
   void* params[] = {(void*)&x, (void*)&y, &out, &args};

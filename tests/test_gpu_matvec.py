@@ -52,6 +52,13 @@ def _matvec(hip, x, y, bk, m=None, k=None, seed=0.0, x_off=0, y_off=0):
     # BK 4 and 8: eight rows a wave
     (13, 1000, 8, 1000, 0),      # a wave with 5 rows past m
     (37, 520, 4, 520, 0),        # 130 tiles, a partial last span
+    # the block kernel: one and four rows a workgroup (from 1025 rows on), spans
+    # of 1024 elements, blocks of one or four of them, rows at any element
+    (1, 4096, 4, 4096, 0), (3, 4100, 4, 4101, 1), (1024, 1028, 4, 1029, 3),
+    (1025, 1023, 4, 1023, 1), (1027, 2052, 8, 2055, 2), (2050, 5000, 16, 5001, 0),
+    (1030, 3001, 32, 3001, 1), (1026, 1100, 64, 1103, 3), (9, 9001, 64, 9001, 1),
+    (5, 8200, 32, 8201, 0), (6, 12300, 16, 12301, 2), (2, 8191, 8, 8191, 1),
+    (1100, 7, 8, 7, 0),          # BK > K: no tile, the seed
 ])
 def test_matvec_matches_the_oracle_bit_for_bit(hip, m, k, bk, ldx, x_off):
     say(f"matvec m={m} k={k} bk={bk} ldx={ldx} x_off={x_off}")
