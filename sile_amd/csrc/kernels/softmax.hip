@@ -666,10 +666,11 @@ __device__ __forceinline__ void reduce_rows_narrow_kernel(int op, const void* x,
   }
 }
 
-// Rows past 1024 x 5 chunks: one row per workgroup of 1024 threads, 16-byte
+// Rows past 1024 x 5 (16-bit: x 4) chunks: one row per workgroup of 1024 threads, 16-byte
 // chunks strided by the workgroup, wave all-reductions plus one exchange of
-// the per-wave partials through LDS.
-template <int kIn>
+// the per-wave partials through LDS.  kDeep: four chunks a thread in flight, for
+// launches of no more rows than CUs (the host's rule has the figures).
+template <int kIn, bool kDeep>
 __device__ __forceinline__ void reduce_rows_block_kernel(int op, const void* x, float* out,
                                                          int64_t rows, int64_t cols,
                                                          int64_t ldx) {
@@ -684,26 +685,39 @@ __device__ __forceinline__ void reduce_rows_block_kernel(int op, const void* x, 
   const TI* xr = static_cast<const TI*>(x) + row * ldx;
   const int64_t vec_cols = cols & ~(int64_t)(kE - 1);
   constexpr int64_t kStep = (int64_t)kT * kE;
+  // f(column, chunk) for this thread's whole chunks, in order
+  auto each_chunk = [&](auto&& f) {
+    int64_t c = (int64_t)t * kE;
+    if constexpr (kDeep) {
+      float v[4][kE];
+      for (; c + 3 * kStep < vec_cols; c += 4 * kStep) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) load_chunk<kIn, kE>(xr + c + j * kStep, v[j]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f(c + j * kStep, v[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (c + j * kStep < vec_cols) load_chunk<kIn, kE>(xr + c + j * kStep, v[j]);
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (c + j * kStep < vec_cols) f(c + j * kStep, v[j]);
+    } else {
+      for (; c < vec_cols; c += kStep) {
+        float v[kE];
+        load_chunk<kIn, kE>(xr + c, v);
+        f(c, v);
+      }
+    }
+  };
   if (op == 0) {
     float m = -__builtin_inff();
     int mi = kNoCol;
-    int64_t c = (int64_t)t * kE;
-    for (; c + 3 * kStep < vec_cols; c += 4 * kStep) {   // four chunks in flight
-      float v[4][kE];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) load_chunk<kIn, kE>(xr + c + j * kStep, v[j]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < kE; ++i) first_max_fold(m, mi, v[j][i], (int)(c + j * kStep) + i);
-    }
-    for (; c < vec_cols; c += kStep) {
-      float v[kE];
-      load_chunk<kIn, kE>(xr + c, v);
+    each_chunk([&](int64_t c, const float (&v)[kE]) {
 #pragma unroll
       for (int i = 0; i < kE; ++i) first_max_fold(m, mi, v[i], (int)c + i);
-    }
-    for (c = vec_cols + t; c < cols; c += kT)
+    });
+    for (int64_t c = vec_cols + t; c < cols; c += kT)
       first_max_fold(m, mi, Elem<kIn>::load1(xr + c), (int)c);
     wave_first_max(m, mi);
     if (lane == 0) {
@@ -718,23 +732,11 @@ __device__ __forceinline__ void reduce_rows_block_kernel(int op, const void* x, 
     return;
   }
   float acc = 0.0f;
-  int64_t c = (int64_t)t * kE;
-  for (; c + 3 * kStep < vec_cols; c += 4 * kStep) {
-    float v[4][kE];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) load_chunk<kIn, kE>(xr + c + j * kStep, v[j]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < kE; ++i) acc = acc + v[j][i];
-  }
-  for (; c < vec_cols; c += kStep) {
-    float v[kE];
-    load_chunk<kIn, kE>(xr + c, v);
+  each_chunk([&](int64_t, const float (&v)[kE]) {
 #pragma unroll
     for (int i = 0; i < kE; ++i) acc = acc + v[i];
-  }
-  for (c = vec_cols + t; c < cols; c += kT) acc = acc + Elem<kIn>::load1(xr + c);
+  });
+  for (int64_t c = vec_cols + t; c < cols; c += kT) acc = acc + Elem<kIn>::load1(xr + c);
   acc = wave_sum(acc);
   if (lane == 0) part[wave] = acc;
   __syncthreads();
@@ -811,7 +813,11 @@ __device__ __forceinline__ void reduce_rows_rowblock_kernel(int op, const void* 
   SILE_REDUCE_NARROW(TAG, IN, n32r4, 32, 4)                                                 \
   extern "C" __global__ __launch_bounds__(1024) void sile_reduce_rows_##TAG##_block(          \
       int op, const void* x, float* out, int64_t rows, int64_t cols, int64_t ldx) {          \
-    reduce_rows_block_kernel<IN>(op, x, out, rows, cols, ldx);                              \
+    reduce_rows_block_kernel<IN, false>(op, x, out, rows, cols, ldx);                       \
+  }                                                                                         \
+  extern "C" __global__ __launch_bounds__(1024) void sile_reduce_rows_##TAG##_block_deep(     \
+      int op, const void* x, float* out, int64_t rows, int64_t cols, int64_t ldx) {          \
+    reduce_rows_block_kernel<IN, true>(op, x, out, rows, cols, ldx);                        \
   }                                                                                         \
   extern "C" __global__ __launch_bounds__(256) void sile_reduce_rows_##TAG##_b256(            \
       int op, const void* x, float* out, int64_t rows, int64_t ldx) {                       \
@@ -843,11 +849,11 @@ SILE_REDUCE_SHAPES(bf16, kBF16)
   SILE_REDUCE_TILE(TAG, IN, 512, 4)   \
   SILE_REDUCE_TILE(TAG, IN, 512, 5)   \
   SILE_REDUCE_TILE(TAG, IN, 512, 6)   \
-  SILE_REDUCE_TILE(TAG, IN, 1024, 4)  \
-  SILE_REDUCE_TILE(TAG, IN, 1024, 5)
+  SILE_REDUCE_TILE(TAG, IN, 1024, 4)
 SILE_REDUCE_TILES(f32, kF32)
 SILE_REDUCE_TILES(f16, kF16)
 SILE_REDUCE_TILES(bf16, kBF16)
+SILE_REDUCE_TILE(f32, kF32, 1024, 5)
 
 // ---- fp32 row sums in the order of the reference's fused load + reduce ----
 // The CPU backend sums a row it loads straight from a buffer

@@ -412,3 +412,28 @@ def test_narrow_rows_four_a_group(hip, dt, cols):
     assert_close(y, e / e.sum(1, keepdims=True), atol=1e-6, rtol=2e-5 if dt == "f32" else 1e-2)
     for b in (dx, dy, out):
         b.close()
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("rows", [1, 256, 257, 300])
+@pytest.mark.parametrize("cols", [4 * 1024 * 8 + 1, 7 * 1024 * 8 + 3])
+def test_reduce_wide_rows_by_row_count(hip, dt, rows, cols):
+    """Rows past the register tiles, as many as the CUs and more: the loop with
+    four chunks in flight and the plain one.  Row max exact; row sums within
+    1e-5 of the row's absolute sum (fp32 chains of at most 68 + 16 + 6 adds)."""
+    say(f"reduce wide {dt} {rows}x{cols}")
+    tin = hip.F32 if dt == "f32" else hip.BF16
+    x = rng(rows + cols).normal(size=(rows, cols)).astype(np.float32)
+    bits, xf = (x, x) if dt == "f32" else bf16_round(x)
+    dx, px = _offset_rows(hip, bits, rows, cols, cols, 0)
+    out = hip.DeviceBuffer(4 * rows)
+    hip.reduce_rows(hip.REDUCE_MAX, tin, rows, cols, px, cols, out.ptr)
+    hip.synchronize()
+    np.testing.assert_array_equal(out.download(np.float32, (rows,)), xf.max(1))
+    hip.reduce_rows(hip.REDUCE_SUM, tin, rows, cols, px, cols, out.ptr)
+    hip.synchronize()
+    got = out.download(np.float32, (rows,)).astype(np.float64)
+    assert (np.abs(got - xf.sum(1, dtype=np.float64))
+            <= 1e-5 * np.abs(xf).sum(1, dtype=np.float64)).all()
+    for b in (dx, out):
+        b.close()
