@@ -420,7 +420,8 @@ int sile_hip_attention_f32_kt(int64_t n_q, int64_t n_k, int64_t head_dim, const 
  * bf16, any S.  D a multiple of 8 up to 256 with 16-byte aligned operands
  * runs on the matrix cores (up to 128 with a query block's keys split over the
  * waves of a workgroup where B * H * S is too small to fill the CUs, so a row's
- * rounding can depend on B, H and S); other D up to 256 (or unaligned operands) on a
+ * rounding can depend on B, H and S; the probabilities enter the second product
+ * in 16 bits, for D an odd multiple of 8 as two 16-bit parts); other D up to 256 (or unaligned operands) on a
  * VALU kernel of one wave per query row.  No reference counterpart: sile's DSL
  * cannot express attention (no mask/iota/transpose); built from the Tile IR
  * ops MmaF, ReduceMax, Exp, ReduceSum (crates/sile-tile-ir/src/ir.rs:128-262). */

@@ -55,6 +55,17 @@ SILE_DEV uint32_t pack2(float lo, float hi) {
   return kBF16 ? pack_bf16x2(lo, hi) : pack_f16x2(lo, hi);
 }
 
+// what is left of lo and hi beside their 16-bit values in `pk`, packed alike
+template <bool kBF16>
+SILE_DEV uint32_t rest2(float lo, float hi, uint32_t pk) {
+  if constexpr (kBF16) {
+    return pack2<kBF16>(lo - bits_f32(pk << 16), hi - bits_f32(pk & 0xffff0000u));
+  } else {
+    const f16x2 h = __builtin_bit_cast(f16x2, pk);
+    return pack2<kBF16>(lo - (float)h[0], hi - (float)h[1]);
+  }
+}
+
 struct AttnArgs {
   int64_t seq;          // S
   int32_t bh;           // B * H
@@ -106,8 +117,12 @@ struct AttnArgs {
 // causal 106 -> 53.
 //
 // A head_dim that is an odd multiple of 8 has zeros in the upper half of its
-// last 16-dim step (both operands) and O^T rows past it that are not stored;
-// 2 x 2814 x 72 causal took 2355 us a query row a wave on the VALU and takes 22.
+// last 16-dim step (both operands) and O^T rows past it that are not stored.
+// Without this kernel such calls take a wave a query row on the VALU with P in
+// fp32, so here P goes into the product as two 16-bit parts, its value and the
+// rest (16 bits of it in bf16, 22 in f16), and its sum is of the fp32 values.
+// 2 x 2814 x 72 causal: 2355 us on the VALU, 27 here (22 with P in one part); 64 x
+// 4096 x 120 causal: 380 us (270).
 //
 // LDS per stage: K and V [kNK][2 kDh B]; with 256-byte rows chunk c of row
 // r at c ^ (r & 15) (K) and c ^ 4 (r & 3) (V), with 128-byte rows at
@@ -163,6 +178,10 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
   constexpr int kKK = (kDh + 15) / 16;   // d-steps of S^T = K . Q^T
   constexpr int kDT = (kDh + 31) / 32;   // 32-d tiles of O^T
   constexpr int kDmaRows = 1024 / kRow;  // rows one 1 KiB DMA instruction fills
+  // P in two 16-bit parts (the header comment on odd multiples of 8)
+  constexpr bool kFullP = kDh % 16 == 8;
+  constexpr int kPV = 2 * kST;                 // 16-key chunks of a P block
+  constexpr int kPN = kFullP ? 2 * kPV : kPV;  // register quads of it: chunks, then their rests
   static_assert(kDh % 8 == 0 && kDh <= kDp && (kDp == 64 || kDp == 128 || kDp == 256),
                 "head_dim a multiple of 8 up to the LDS row");
   static_assert(kG == 1 || kQT == 1, "key groups: one query tile a wave");
@@ -306,7 +325,7 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
       }
       return out;
     };
-    auto pv_block = [&](int stage, const u32x4 (&pf)[kQT][2 * kST], f32x16 (&oacc)[kQT][kDT]) {
+    auto pv_block = [&](int stage, const u32x4 (&pf)[kQT][kPN], f32x16 (&oacc)[kQT][kDT]) {
       const uint8_t* vs = smem + stage * kStageB + kTileB;
   #pragma unroll
       for (int dt = 0; dt < kDT; ++dt)
@@ -315,15 +334,20 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
           const u32x4 vf = v_frag(vs, dt, cc);
   #pragma unroll
           for (int qt = 0; qt < kQT; ++qt) oacc[qt][dt] = mma32<kBF16>(vf, pf[qt][cc], oacc[qt][dt]);
+          if constexpr (kFullP) {
+  #pragma unroll
+            for (int qt = 0; qt < kQT; ++qt)
+              oacc[qt][dt] = mma32<kBF16>(vf, pf[qt][kPV + cc], oacc[qt][dt]);
+          }
         }
     };
 
     // S_{j+1} over (S tile, d-step) and PV_{j-1} over (d-tile, key chunk), one
     // step of each at a time: S step (st, kk) runs at step kKK st + kk, PV
     // (dt, cc) at step dt + kDT cc (kST kKK and 2 kST kDT steps: equal
-    // unless kDh % 32 == 16)
+    // when kDh % 32 is 0 or over 16)
     auto mma_block = [&](int kstage, int vstage, f32x16 (&sacc)[kQT][kST],
-                         const u32x4 (&pf)[kQT][2 * kST], f32x16 (&oa)[kQT][kDT]) {
+                         const u32x4 (&pf)[kQT][kPN], f32x16 (&oa)[kQT][kDT]) {
       const uint8_t* ks = smem + kstage * kStageB + kf_off;
       const uint8_t* vs = smem + vstage * kStageB + kTileB;
   #pragma unroll
@@ -346,6 +370,11 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
           const u32x4 vf = v_frag(vs, dt, cc);
   #pragma unroll
           for (int qt = 0; qt < kQT; ++qt) oa[qt][dt] = mma32<kBF16>(vf, pf[qt][cc], oa[qt][dt]);
+          if constexpr (kFullP) {
+  #pragma unroll
+            for (int qt = 0; qt < kQT; ++qt)
+              oa[qt][dt] = mma32<kBF16>(vf, pf[qt][kPV + cc], oa[qt][dt]);
+          }
         }
       }
     };
@@ -363,11 +392,11 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
       m_run[qt] = -__builtin_inff();
       l_run[qt] = 0.0f;
     }
-    u32x4 pprev[kQT][2 * kST];
+    u32x4 pprev[kQT][kPN];
   #pragma unroll
     for (int qt = 0; qt < kQT; ++qt)
   #pragma unroll
-      for (int cc = 0; cc < 2 * kST; ++cc) pprev[qt][cc] = u32x4{0u, 0u, 0u, 0u};
+      for (int cc = 0; cc < kPN; ++cc) pprev[qt][cc] = u32x4{0u, 0u, 0u, 0u};
 
     // key blocks: through the block's last query (causal) or S, rounded up
     // to even (the loop runs in pairs); keys past S load as zeros (outside
@@ -393,14 +422,14 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
     dma_v(0, 1);
     __syncthreads();
     f32x16 sa[kQT][kST], sb[kQT][kST];
-    u32x4 pb[kQT][2 * kST];
+    u32x4 pb[kQT][kPN];
     s_block(0, sa);
     __syncthreads();
 
     // The online softmax of S_j -> P_j on the VALU (causal / past-S mask
     // first when kMasked).
     auto softmax_block = [&](int j, auto masked, f32x16 (&scur)[kQT][kST],
-                             u32x4 (&pnew)[kQT][2 * kST]) {
+                             u32x4 (&pnew)[kQT][kPN]) {
       constexpr bool kMasked = decltype(masked)::value;
       if constexpr (kMasked) {
         const int kb = (j * kG + kg) * kNK;
@@ -432,16 +461,23 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
         for (int st = 0; st < kST; ++st)
   #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            u32x4 w;
+            u32x4 w, rest;
   #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
               const float p0 = exp2_fast(__builtin_fmaf(scur[qt][st][8 * h + 2 * jj], c, -mc));
               const float p1 = exp2_fast(__builtin_fmaf(scur[qt][st][8 * h + 2 * jj + 1], c, -mc));
               const uint32_t pk = pack2<kBF16>(p0, p1);
               w[jj] = pk;
-              rs = pair_sum<kBF16>(pk, rs);
+              if constexpr (kFullP) {
+                rest[jj] = rest2<kBF16>(p0, p1, pk);
+                rs += p0;
+                rs += p1;
+              } else {
+                rs = pair_sum<kBF16>(pk, rs);
+              }
             }
             pnew[qt][2 * st + h] = w;
+            if constexpr (kFullP) pnew[qt][kPV + 2 * st + h] = rest;
           }
         slow |= __builtin_amdgcn_ballot_w64(!(rs <= kBlockSumLimit)) != 0;
         rs_blk[qt] = rs;
@@ -480,16 +516,23 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
           for (int st = 0; st < kST; ++st)
   #pragma unroll
             for (int h = 0; h < 2; ++h) {
-              u32x4 w;
+              u32x4 w, rest;
   #pragma unroll
               for (int jj = 0; jj < 4; ++jj) {
                 const float p0 = exp2_fast(__builtin_fmaf(scur[qt][st][8 * h + 2 * jj], c, -mc));
                 const float p1 = exp2_fast(__builtin_fmaf(scur[qt][st][8 * h + 2 * jj + 1], c, -mc));
                 const uint32_t pk = pack2<kBF16>(p0, p1);
                 w[jj] = pk;
-                rs = pair_sum<kBF16>(pk, rs);
+                if constexpr (kFullP) {
+                  rest[jj] = rest2<kBF16>(p0, p1, pk);
+                  rs += p0;
+                  rs += p1;
+                } else {
+                  rs = pair_sum<kBF16>(pk, rs);
+                }
               }
               pnew[qt][2 * st + h] = w;
+              if constexpr (kFullP) pnew[qt][kPV + 2 * st + h] = rest;
             }
           rs_blk[qt] = rs;
           l_run[qt] *= alpha;
@@ -517,8 +560,8 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
     // MFMAs of blocks j + 1 (S) and j - 1 (PV).  kMasked selects the causal-mask
     // code, needed only on the workgroup's diagonal.
     auto iteration = [&](int j, auto stage_c, auto masked, f32x16 (&scur)[kQT][kST],
-                         f32x16 (&snext)[kQT][kST], const u32x4 (&pprev)[kQT][2 * kST],
-                         u32x4 (&pnew)[kQT][2 * kST]) {
+                         f32x16 (&snext)[kQT][kST], const u32x4 (&pprev)[kQT][kPN],
+                         u32x4 (&pnew)[kQT][kPN]) {
       constexpr int kS = decltype(stage_c)::value;
       constexpr bool kMasked = decltype(masked)::value;
       dma_k(min(j + 2, last), kS);
@@ -545,7 +588,7 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
   #pragma unroll
       for (int qt = 0; qt < kQT; ++qt) {
   #pragma unroll
-        for (int cc = 0; cc < 2 * kST; ++cc) asm volatile("" : "+v"(pnew[qt][cc]));
+        for (int cc = 0; cc < kPN; ++cc) asm volatile("" : "+v"(pnew[qt][cc]));
         asm volatile("" : "+v"(l_run[qt]));
       }
       __syncthreads();

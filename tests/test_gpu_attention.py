@@ -344,6 +344,40 @@ def test_flash_key_groups(hip, dt, trend, causal, h, s, d):
         assert_close(got[0, hi], ref, atol=ATOL, rtol=RTOL, what=f"h{hi}")
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("h,s,d", [(2, 300, 8), (3, 130, 40), (8, 700, 56), (2, 300, 72), (8, 520, 104),
+                                   (40, 520, 120), (1, 200, 136), (2, 330, 248)])
+def test_flash_head_dims_of_8_precision(hip, dt, causal, h, s, d):
+    """Odd multiples of 8 carry more of P than its 16-bit value: keys in pairs of
+    nearly equal scores against V rows of +64 and -64, so that a row's result is
+    the small difference of large products.  P's two 16-bit parts leave at most
+    2^-16 (bf16) and, down to the smallest f16, 2^-21 of each product of 64; the
+    bound is twice and four times that (fp32 exp2 and sums take the rest) and
+    the rounding of the result.  P in one 16-bit part is off by up to 2^-9 and
+    2^-12 of each product."""
+    say(f"flash precision D={d} {dt} causal={causal} H={h} S={s}")
+    scale = 1.0 / np.sqrt(d)
+    rnd = f16_round if dt == "f16" else bf16_round
+    r = rng(d + s)
+    q = r.normal(size=(1, h, s, d)).astype(np.float32)
+    k = r.uniform(-1.0, 1.0, size=(1, h, s, d)).astype(np.float32)
+    k[:, :, 1::2] = k[:, :, 0:s - s % 2:2]
+    k[:, :, 1::2, 0] += 0.0625
+    v = np.empty((1, h, s, d), np.float32)
+    v[:, :, 0::2], v[:, :, 1::2] = 64.0, -64.0
+    qkv = [rnd(x) for x in (q, k, v)]
+    got = _run(hip, dt, 1, h, s, d, [x[0] for x in qkv], causal, scale)
+    qf, kf, vf = (x[1][0].astype(np.float64) for x in qkv)
+    atol, rtol = (64 * 2.0 ** -15, 2.0 ** -8) if dt == "bf16" else (64 * 2.0 ** -19, 2.0 ** -11)
+    for hi in sorted({0, h // 2, h - 1}):
+        p = qf[hi] @ kf[hi].T * scale
+        if causal:
+            p[np.triu_indices(s, 1)] = -np.inf
+        p = np.exp(p - p.max(1, keepdims=True))
+        assert_close(got[0, hi], p @ vf[hi] / p.sum(1, keepdims=True), atol=atol, rtol=rtol, what=f"h{hi}")
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_flash_long_sequence(hip, causal):
     """S = 65536 (B = 1, H = 8, D = 128, f16): block, key and byte offsets at
