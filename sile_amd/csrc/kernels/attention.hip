@@ -100,7 +100,7 @@ extern "C" __global__ __launch_bounds__(256) void sile_attn_fwd_rowwise_bf16(
 //     8 (i / 4) + i % 4 and that + 4.  P never moves between lanes.
 // fp32 matrix instructions hold the SIMD against its VALU instructions
 // (measured: their cycles add up), so the loop is kept lean of those: scalar
-// row pointers, scores in log2 units, O rescaled only where a max moved.  The
+// row pointers, O rescaled only where a max moved.  The
 // next block's K and V are loaded into the registers right behind the products
 // that read them, a whole block (8192 matrix-core cycles at d = 128) ahead.
 //
@@ -229,9 +229,8 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
   }
   __syncthreads();
 
-  const float c = scale * kLog2e;
   f32x16 oacc[kT];
-  float m = m0 * kLog2e, l = 0.0f;
+  float m = m0, l = 0.0f;
 #pragma unroll
   for (int t = 0; t < kT; ++t)
 #pragma unroll
@@ -260,11 +259,12 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    // register i: key k0 + 8 (i / 4) + i % 4 of query q0 + 32 qt + r
+    // register i: key 32 blk + 4 h + 8 (i / 4) + i % 4 of query q0 + r
     const int64_t left = n_k - (blk * 32 + 4 * h);
     const bool partial = (blk + 1) * 32 > n_k;
-    // scores and max in log2 units
-    s *= c;
+    // (times log2 e only where the max is taken off: scores and an initial max
+    // up to the largest float stay finite)
+    s *= scale;
     if (partial) {
 #pragma unroll
       for (int i = 0; i < 16; ++i)
@@ -280,10 +280,10 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
     float rsum = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      s[i] = exp2_fast(s[i] - m_use);   // masked keys: 0
+      s[i] = exp2_fast((s[i] - m_use) * kLog2e);   // masked keys: 0
       rsum += s[i];
     }
-    const float alpha = exp2_fast(m - m_use);
+    const float alpha = exp2_fast((m - m_use) * kLog2e);
     l = l * alpha + pair32_sum(rsum);
     m = m_new;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
@@ -318,7 +318,7 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
   float mm = m_lds[0][r];
 #pragma unroll
   for (int w = 1; w < kW; ++w) mm = mm >= m_lds[w][r] ? mm : m_lds[w][r];
-  const float f = exp2_fast(m - (mm == -__builtin_inff() ? 0.0f : mm));
+  const float f = exp2_fast((m - (mm == -__builtin_inff() ? 0.0f : mm)) * kLog2e);
   // row 8 (i / 4) + 4 h + i % 4 of tile t: place kT row + t of the query
 #pragma unroll
   for (int i = 0; i < 16; ++i)
@@ -339,7 +339,7 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
     f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < kW; ++w) {
-      lq += l_lds[w][qi] * exp2_fast(m_lds[w][qi] - mq_use);
+      lq += l_lds[w][qi] * exp2_fast((m_lds[w][qi] - mq_use) * kLog2e);
       sum += *reinterpret_cast<const f32x4*>(&o_lds[w][qi][4 * c]);
     }
     if (splits > 1) {
@@ -379,7 +379,7 @@ extern "C" __global__ __launch_bounds__(256) void sile_attn_f32_combine(
       const float other = __shfl_xor(mq, x);
       mq = mq >= other ? mq : other;
     }
-    const float f = exp2_fast(mz - (mq == -__builtin_inff() ? 0.0f : mq));
+    const float f = exp2_fast((mz - (mq == -__builtin_inff() ? 0.0f : mq)) * kLog2e);
     w_lds[j][lane] = f;
     const float l = wave_sum(lane < splits ? lz * f : 0.0f);
     if (lane == 0) l_lds[j] = l;

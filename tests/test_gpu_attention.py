@@ -482,6 +482,33 @@ def test_attention_f32_kt_far_pitches(hip, d, ldkt, ldv):
         b.close()
 
 
+@pytest.mark.parametrize("n_k", [40, 1000])
+@pytest.mark.parametrize("m0", [-np.finfo(np.float32).max, -np.inf, -3.2e38])
+def test_attention_f32_kt_largest_floats(hip, n_k, m0):
+    """Scores and initial maxima up to the largest float, as a program that masks
+    with the type's lowest value has them: the products with log2 e that exp needs
+    must not overflow on their own.  Rows: every score -3e38 (below m0 = -3.2e38's
+    reach: a uniform average), 3e38 at one key and 1e38 at the others (that key's V
+    row), -3e38 but for one 0 (that one's), ordinary scores."""
+    n_q, d = 4, 8
+    say(f"attention_f32_kt largest floats n_k={n_k} m0={m0}")
+    q, kt, v = _dsl_attn_inputs(n_q, n_k, d, 5)
+    q[:] = np.eye(n_q, d)
+    kt[0], kt[1], kt[2] = -3e38, 1e38, -3e38
+    kt[1, n_k // 2], kt[2, n_k - 1] = 3e38, 0.0
+    kt[3] = rng(6).normal(size=n_k)
+    bufs = [hip.DeviceBuffer.from_array(x) for x in (q, kt, v)]
+    do = hip.DeviceBuffer(n_q * d * 4)
+    hip.attention_f32_kt(n_q, n_k, d, bufs[0].ptr, d, bufs[1].ptr, n_k, bufs[2].ptr, d, do.ptr, d,
+                         1.0, float(m0))
+    hip.synchronize()
+    ref = cpuref.dsl_attention_f32(q, kt, v, n_k, 1.0, float(m0), d=d, n_q=n_q, s_k=n_k)
+    assert np.isfinite(ref).all()
+    assert_close(do.download(np.float32, (n_q, d)), ref, atol=1e-5, rtol=1e-4, what="largest floats")
+    for b in bufs + [do]:
+        b.close()
+
+
 def test_attention_f32_kt_closed_forms(hip):
     """An initial max above every score gives 0 / 0 everywhere, as the
     program does; no keys gives 0 / 0 too."""
