@@ -453,7 +453,8 @@ SILE_SOFTMAX_NARROW_WIDTHS(f16_f32, kF16, kF32)
 // (the sum rescaled when the max grows), then the workgroup combines them:
 // M = max of the maxima, S = sum of sum_t * exp(m_t - M).  Pass 2 reads the
 // row again (mostly from L2 / MALL) and writes exp(x - M) / S.  3 row
-// accesses per element instead of 2.
+// accesses per element instead of 2.  A NaN never enters a max and always the
+// sum, so it makes the whole row NaN, as in the kernels that hold a row.
 template <int kIn, int kOut>
 __device__ __forceinline__ void softmax_rows_wide_kernel(const void* x, void* y, int64_t rows,
                                                          int64_t cols, int64_t ldx,
@@ -482,11 +483,15 @@ __device__ __forceinline__ void softmax_rows_wide_kernel(const void* x, void* y,
   for (int64_t c0 = (int64_t)t * kE; c0 < cols; c0 += (int64_t)kT * kE) {
     float v[kE];
     load(c0, v);
-    float cm = v[0];
+    float mn = m;
 #pragma unroll
-    for (int i = 1; i < kE; ++i) cm = fmax_ordered(cm, v[i]);
-    const float mn = fmax_ordered(m, cm);
-    if (mn == -__builtin_inff()) continue;   // nothing but -inf so far: s stays 0
+    for (int i = 0; i < kE; ++i) mn = fmax_ordered(mn, v[i]);
+    if (mn == -__builtin_inff()) {   // nothing but -inf (s stays 0) and NaN so far
+#pragma unroll
+      for (int i = 0; i < kE; ++i)
+        if (v[i] != v[i]) s = v[i];
+      continue;
+    }
     s = (m == mn ? s : s * exp2_fast((m - mn) * kLog2e));   // m = -inf: s is 0
 #pragma unroll
     for (int i = 0; i < kE; ++i) s += exp2_fast((v[i] - mn) * kLog2e);
@@ -498,7 +503,7 @@ __device__ __forceinline__ void softmax_rows_wide_kernel(const void* x, void* y,
   M = part[0][0];
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) M = fmax_ordered(M, part[0][w]);
-  float S = wave_sum(m == -__builtin_inff() ? 0.0f : s * exp2_fast((m - M) * kLog2e));
+  float S = wave_sum(m == -__builtin_inff() ? s : s * exp2_fast((m - M) * kLog2e));
   if (lane == 0) part[1][wave] = S;
   __syncthreads();
   S = part[1][0];

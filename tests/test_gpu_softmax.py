@@ -437,3 +437,35 @@ def test_reduce_wide_rows_by_row_count(hip, dt, rows, cols):
             <= 1e-5 * np.abs(xf).sum(1, dtype=np.float64)).all()
     for b in (dx, out):
         b.close()
+
+
+@pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("cols,off", [(65544, 0), (65543, 1), (70000, 1), (4000, 0), (100, 1)])
+def test_softmax_nan_reaches_the_whole_row(hip, dt, cols, off):
+    """exp(NaN - m) enters the row's sum, so one NaN makes its row NaN, wherever
+    it lies: at a thread's first chunk of a two-pass row (alone, over the whole
+    chunk, beside -inf), later, in the last element.  Rows without one stay
+    within tolerance; all of -inf is 0 / 0."""
+    x = (rng(cols).normal(size=(8, cols)) * 2.0).astype(np.float32)
+    x[0, 8] = np.nan
+    x[1, 16:24] = np.nan
+    x[2, :8] = -np.inf
+    x[2, 1] = np.nan
+    x[3, cols - 1] = np.nan
+    x[4, cols // 2] = np.nan
+    x[5, :] = -np.inf
+    x[6, :cols // 2] = -np.inf
+    say(f"softmax NaN {dt} {cols} off={off}")
+    t = hip.F32 if dt == "f32" else hip.F16
+    bits, xf = (x, x) if dt == "f32" else f16_round(x)
+    dx, px = _offset_rows(hip, bits, 8, cols, cols + 8 + off, off)
+    dy = hip.DeviceBuffer(8 * cols * bits.itemsize)
+    hip.softmax_rows(t, t, 8, cols, px, cols + 8 + off, dy.ptr, cols)
+    hip.synchronize()
+    y = dy.download(bits.dtype, (8, cols))
+    y = y if dt == "f32" else y.view(np.float16).astype(np.float32)
+    assert np.isnan(y[:6]).all()
+    e = np.exp(xf[6:].astype(np.float64) - xf[6:].max(1, keepdims=True))
+    assert_close(y[6:], e / e.sum(1, keepdims=True), atol=1e-6, rtol=2e-5 if dt == "f32" else 1e-2)
+    for b in (dx, dy):
+        b.close()
