@@ -406,10 +406,11 @@ int sile_hip_reduce_rows_fused_sum(int64_t rows, int64_t cols, const float *x, i
  * dim t at kt[t * ldkt + j]), v [n_k, ldv], o [n_q, ldo]; head_dim <= 128;
  * results within fp32 rounding of the program (sums in another order; exp
  * is the device's).  Where the query tiles are fewer than the CUs the keys are
- * split into ranges computed side by side, their partial results kept in the
- * device scratch of sile_hip_gemm (about 17 MiB at most) and added in range
- * order by a second kernel; not under graph capture, where one plain launch
- * is recorded. */
+ * split into ranges computed side by side, their partial results kept in a
+ * device scratch buffer shared by these calls (2 x CUs x 32 rows of 130 floats,
+ * 8.1 MiB on 256 CUs, allocated on first use; calls on different streams are
+ * ordered on the GPU by an event) and added in range order by a second kernel;
+ * not under graph capture, where one plain launch is recorded. */
 int sile_hip_attention_f32_kt(int64_t n_q, int64_t n_k, int64_t head_dim, const float *q,
                               int64_t ldq, const float *kt, int64_t ldkt, const float *v,
                               int64_t ldv, float *o, int64_t ldo, float scale, float m0,

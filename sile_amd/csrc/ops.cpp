@@ -1060,8 +1060,9 @@ int sile_hip_attention_f32_kt(int64_t n_q, int64_t n_k, int64_t head_dim, const 
   int splits = 1, cus = 0;
   int64_t per_split = key_blocks;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  const bool capturing =
-      hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+  const hipError_t cap_e = hipStreamIsCapturing(s, &cap);
+  if (cap_e != hipSuccess) (void)hipGetLastError();   // (the null stream beside a capture)
+  const bool capturing = cap_e != hipSuccess || cap != hipStreamCaptureStatusNone;
   if (!capturing && device_cus(&cus) == SILE_OK) {
     double best = 1e30;
     for (int64_t z = 1; z <= std::min<int64_t>(64, key_blocks) && (z == 1 || z * q_tiles <= 2 * cus);
@@ -1080,7 +1081,8 @@ int sile_hip_attention_f32_kt(int64_t n_q, int64_t n_k, int64_t head_dim, const 
   if (splits > 1) {
     per_split = (key_blocks + splits - 1) / splits;
     splits = (int)((key_blocks + per_split - 1) / per_split);
-    if (scratch_acquire((size_t)(splits * n_q) * (pitch + 2) * sizeof(float), s, &ws) != SILE_OK) {
+    // (splits * n_q rows of pitch + 2 floats at most: 8.1 MiB on 256 CUs)
+    if (scratch_acquire((size_t)(2 * cus) * 32 * (128 + 2) * sizeof(float), s, &ws, 2) != SILE_OK) {
       ws = nullptr;
       splits = 1;
       per_split = key_blocks;
@@ -1102,7 +1104,7 @@ int sile_hip_attention_f32_kt(int64_t n_q, int64_t n_k, int64_t head_dim, const 
       rc = launch(Module::kAttention, "sile_attn_f32_combine",
                   dim3((unsigned)((n_q + 7) / 8)), dim3(256), cp, s);
     }
-    scratch_release(s);
+    scratch_release(s, 2);
   }
   return rc == SILE_OK ? ok() : rc;
 }

@@ -164,7 +164,17 @@ struct DeviceScratch {
   bool used = false;
 };
 DeviceScratch g_scratch[kScratchDevices][kScratchSlots];
-thread_local int t_scratch_dev[kScratchSlots] = {-1, -1};  // device whose slot lock this thread holds
+thread_local int t_scratch_dev[kScratchSlots] = {-1, -1, -1};  // device whose slot lock this thread holds
+
+// For its lifetime this thread's allocations and frees do not invalidate a
+// stream capture in progress on another stream (they belong to none).
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  ~RelaxedCapture() {
+    if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
 }  // namespace
 
 int scratch_acquire(size_t bytes, hipStream_t s, void** out, int slot) {
@@ -176,8 +186,10 @@ int scratch_acquire(size_t bytes, hipStream_t s, void** out, int slot) {
   if (slot < 0 || slot >= kScratchSlots) return fail(SILE_ERR_SHAPE, "scratch slot %d", slot);
   DeviceScratch& d = g_scratch[dev][slot];
   d.mu.lock();
+  const RelaxedCapture relaxed;
   auto bail = [&](hipError_t e, const char* what) {
     d.mu.unlock();
+    (void)hipGetLastError();
     return hip_fail(e, what);
   };
   hipError_t e = hipSuccess;

@@ -10,6 +10,10 @@ result, the two GEMMs whose scratch-using forms are left out under capture
 against the oracle (|g - r| <= 2e-2 + 1e-2 |r|, fp32 out 1e-4) and against
 the first replay bit for bit.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -111,3 +115,64 @@ def test_graph_replays_op_calls(hip):
         buf.close()
     st.close()
     other.close()
+
+
+# First use and growth of every scratch slot by eager calls, from the thread that
+# is capturing another stream (in a process of its own: the slots are empty).
+_CAPTURE_CODE = r"""
+import numpy as np
+from sile_amd import _abi as hip
+hip.init(0)
+st, other = hip.Stream(), hip.Stream()
+r = np.random.default_rng(1)
+x = r.normal(size=(64, 1000)).astype(np.float32)
+dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(x.nbytes)
+nq, nk, d = 64, 2000, 64
+att = [r.normal(size=z).astype(np.float32) for z in ((nq, d), (d, nk), (nk, d))]
+da = [hip.DeviceBuffer.from_array(t) for t in att]
+do, do2 = hip.DeviceBuffer(nq * d * 4), hip.DeviceBuffer(nq * d * 4)
+m = 256
+ab = r.integers(0x3f00, 0x3f80, size=(2, 512, 4096)).astype(np.uint16)   # bf16 in [0.5, 1)
+dab = [hip.DeviceBuffer.from_array(t) for t in ab]
+dbt = hip.DeviceBuffer.from_array(np.ascontiguousarray(ab[1][:100].T))
+outs = [hip.DeviceBuffer(512 * 512 * 4) for _ in range(6)]
+def attention(out, s):
+    hip.attention_f32_kt(nq, nk, d, da[0].ptr, d, da[1].ptr, nk, da[2].ptr, d, out.ptr, d, 0.125, -1e30, s)
+def gemm(n, splits, out, s):
+    hip.gemm(hip.BF16, hip.BF16, hip.F32, n, n, 4096, dab[0].ptr, 4096, hip.ROW_MAJOR, dab[1].ptr, 4096,
+             hip.COL_MAJOR, out.ptr, n, 1.0, 1.0, 0, s, tile=128, splits=splits)
+def brow(out, s):   # B row-major of 100 columns: transposed into the scratch first
+    hip.gemm(hip.BF16, hip.BF16, hip.F32, 512, 100, 4096, dab[0].ptr, 4096, hip.ROW_MAJOR, dbt.ptr, 100,
+             hip.ROW_MAJOR, out.ptr, 100, 1.0, 1.0, 0, s)
+def eager(o, g, s):
+    attention(o, s)
+    gemm(256, 2, g[0], s)
+    gemm(512, 8, g[1], s)    # a larger scratch: the first one is freed
+    brow(g[2], s)
+with hip.Graph(st) as graph:
+    hip.softmax_rows(hip.F32, hip.F32, 64, 1000, dx.ptr, 1000, dy.ptr, 1000, st)
+    eager(do, outs[:3], other)
+graph.launch()
+st.synchronize()
+other.synchronize()
+eager(do2, outs[3:], st)
+st.synchronize()
+e = np.exp(x.astype(np.float64) - x.max(1, keepdims=True))
+assert np.abs(dy.download(np.float32, x.shape) - e / e.sum(1, keepdims=True)).max() < 1e-5
+assert (do.download(np.uint32, (nq, d)) == do2.download(np.uint32, (nq, d))).all()
+assert np.isfinite(do.download(np.float32, (nq, d))).all()
+for i, n in enumerate((256 * 256, 512 * 512, 512 * 100)):
+    a, b = outs[i].download(np.float32, (n,)), outs[3 + i].download(np.float32, (n,))
+    assert (a == b).all() and a.min() > 500
+print("CAPTURE_OK", flush=True)
+"""
+
+
+def test_scratch_allocated_beside_a_capture(hip):
+    """Eager calls on one stream, by the thread that captures another: their
+    scratch is allocated, grown and freed without ending the capture."""
+    say("graph: scratch allocated while another stream is captured")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", _CAPTURE_CODE], cwd=root, capture_output=True, text=True,
+                         timeout=100)
+    assert run.returncode == 0 and "CAPTURE_OK" in run.stdout, run.stdout + run.stderr
