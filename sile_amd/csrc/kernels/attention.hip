@@ -100,7 +100,7 @@ extern "C" __global__ __launch_bounds__(256) void sile_attn_fwd_rowwise_bf16(
 //     8 (i / 4) + i % 4 and that + 4.  P never moves between lanes.
 // fp32 matrix instructions hold the SIMD against its VALU instructions
 // (measured: their cycles add up), so the loop is kept lean of those: scalar
-// row pointers, O rescaled only where a max moved.  The
+// row pointers, scores in log2 units, O rescaled only where a max moved.  The
 // next block's K and V are loaded into the registers right behind the products
 // that read them, a whole block (8192 matrix-core cycles at d = 128) ahead.
 //
@@ -125,6 +125,11 @@ SILE_DEV int attn_f32_dim(int place, int tiles, int d) {
   return min(place / tiles * tiles, d - tiles) + place % tiles;
 }
 constexpr int kF32Waves = 8;
+// Scores and maxima are kept times log2 e / 4, so that those up to the largest float
+// (a program that masks with the type's lowest value) do not overflow, and their
+// differences are taken times 4.  (Times log2 e, rows past 2.4e38 came out NaN; in
+// the scores' own units two registers are spilt at d = 128.)
+SILE_DEV float f32_weight(float score, float max) { return exp2_fast((score - max) * 4.0f); }
 
 template <int kDp, bool kFar>
 __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t ldq,
@@ -229,8 +234,9 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
   }
   __syncthreads();
 
+  const float c = scale * (kLog2e / 4);
   f32x16 oacc[kT];
-  float m = m0, l = 0.0f;
+  float m = m0 * (kLog2e / 4), l = 0.0f;
 #pragma unroll
   for (int t = 0; t < kT; ++t)
 #pragma unroll
@@ -262,9 +268,7 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
     // register i: key 32 blk + 4 h + 8 (i / 4) + i % 4 of query q0 + r
     const int64_t left = n_k - (blk * 32 + 4 * h);
     const bool partial = (blk + 1) * 32 > n_k;
-    // (times log2 e only where the max is taken off: scores and an initial max
-    // up to the largest float stay finite)
-    s *= scale;
+    s *= c;
     if (partial) {
 #pragma unroll
       for (int i = 0; i < 16; ++i)
@@ -280,10 +284,10 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
     float rsum = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      s[i] = exp2_fast((s[i] - m_use) * kLog2e);   // masked keys: 0
+      s[i] = f32_weight(s[i], m_use);   // masked keys: 0
       rsum += s[i];
     }
-    const float alpha = exp2_fast((m - m_use) * kLog2e);
+    const float alpha = f32_weight(m, m_use);
     l = l * alpha + pair32_sum(rsum);
     m = m_new;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
@@ -318,7 +322,7 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
   float mm = m_lds[0][r];
 #pragma unroll
   for (int w = 1; w < kW; ++w) mm = mm >= m_lds[w][r] ? mm : m_lds[w][r];
-  const float f = exp2_fast((m - (mm == -__builtin_inff() ? 0.0f : mm)) * kLog2e);
+  const float f = f32_weight(m, mm == -__builtin_inff() ? 0.0f : mm);
   // row 8 (i / 4) + 4 h + i % 4 of tile t: place kT row + t of the query
 #pragma unroll
   for (int i = 0; i < 16; ++i)
@@ -339,7 +343,7 @@ __device__ __forceinline__ void attn_f32_kt(const float* __restrict__ q, int64_t
     f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < kW; ++w) {
-      lq += l_lds[w][qi] * exp2_fast((m_lds[w][qi] - mq_use) * kLog2e);
+      lq += l_lds[w][qi] * f32_weight(m_lds[w][qi], mq_use);
       sum += *reinterpret_cast<const f32x4*>(&o_lds[w][qi][4 * c]);
     }
     if (splits > 1) {
@@ -379,7 +383,7 @@ extern "C" __global__ __launch_bounds__(256) void sile_attn_f32_combine(
       const float other = __shfl_xor(mq, x);
       mq = mq >= other ? mq : other;
     }
-    const float f = exp2_fast((mz - (mq == -__builtin_inff() ? 0.0f : mq)) * kLog2e);
+    const float f = f32_weight(mz, mq == -__builtin_inff() ? 0.0f : mq);
     w_lds[j][lane] = f;
     const float l = wave_sum(lane < splits ? lz * f : 0.0f);
     if (lane == 0) l_lds[j] = l;
