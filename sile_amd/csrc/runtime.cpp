@@ -186,16 +186,16 @@ int scratch_acquire(size_t bytes, hipStream_t s, void** out, int slot) {
   if (slot < 0 || slot >= kScratchSlots) return fail(SILE_ERR_SHAPE, "scratch slot %d", slot);
   DeviceScratch& d = g_scratch[dev][slot];
   d.mu.lock();
-  const RelaxedCapture relaxed;
   auto bail = [&](hipError_t e, const char* what) {
     d.mu.unlock();
     (void)hipGetLastError();
     return hip_fail(e, what);
   };
   hipError_t e = hipSuccess;
-  if (!d.last && (e = hipEventCreateWithFlags(&d.last, hipEventDisableTiming)) != hipSuccess)
-    return bail(e, "hipEventCreateWithFlags");
-  if (d.cap < bytes) {
+  if (!d.last || d.cap < bytes) {
+    const RelaxedCapture relaxed;
+    if (!d.last && (e = hipEventCreateWithFlags(&d.last, hipEventDisableTiming)) != hipSuccess)
+      return bail(e, "hipEventCreateWithFlags");
     if (d.p) {
       // the previous buffer may still be in use on another stream
       if (d.used && (e = hipEventSynchronize(d.last)) != hipSuccess)
