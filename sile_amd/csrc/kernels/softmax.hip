@@ -16,9 +16,9 @@
 //    the fastest copy measured on the device; the row max and sum are wave
 //    all-reductions plus one exchange of per-wave partials through LDS;
 //  * other widths: kL lanes per row for rows of up to 32 chunks (4..32 rows
-//    per wave, four times as many in flight in large launches), a wave a row up
-//    to 256 chunks, then a workgroup a row with the row in registers up to
-//    65536 elements, two passes over the row by one workgroup beyond that.
+//    per wave), a wave a row up to 256 chunks, then a workgroup a row with the
+//    row in registers up to 65536 elements, two passes over the row by one
+//    workgroup beyond that.
 // Rows may start at any element: the 128-bit accesses need no alignment.
 // Wave all-reductions use DPP row permutes (common.h); exp(x - m) is
 // 2^((x - m) * log2 e) on v_exp_f32.
@@ -369,79 +369,74 @@ SILE_DEV float group_sum(float v) {
   return v;
 }
 
-// kR rows a group of lanes, every load before the first value is used: with one
-// row a launch of many rows has too few bytes in flight (f16 65536 x 100: 10 us).
-// The chunk a row ends in is moved back to end there, as in the tile kernel;
-// rows shorter than a chunk go element by element.
-template <int kIn, int kOut, int kL, int kR>
+// The chunk a row ends in is moved back to end there, as in the tile kernel; rows
+// shorter than a chunk go element by element.  Both are the same choice for every
+// lane, so that the lanes past a row only skip a load (as an element path of
+// theirs alone they took longer than the row: f16 131072 x 200 22.0 against 19.0
+// us).  Four rows a group, all loaded first, ran 0 to 40 % slower (f16 16384 x 200
+// 7.2 against 4.3 us).
+template <int kIn, int kOut, int kL>
 __device__ __forceinline__ void softmax_rows_narrow_kernel(const void* x, void* y, int64_t rows,
                                                            int64_t cols, int64_t ldx,
                                                            int64_t ldy) {
   static_assert(kL == 4 || kL == 8 || kL == 16 || kL == 32, "lanes per row");
   constexpr int kE = chunk_elems<kIn, kOut>();
-  constexpr int kWaveRows = 64 / kL;
   const int lane = threadIdx.x & 63, li = lane % kL;
-  const int64_t row0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (kWaveRows * kR) + lane / kL;
+  const int64_t row = (int64_t)blockIdx.x * (256 / kL) + (threadIdx.x >> 6) * (64 / kL) + lane / kL;
   using TI = typename Elem<kIn>::Storage;
   using TO = typename Elem<kOut>::Storage;
   const int n = (int)cols, c0 = li * kE, at = min(c0, n - kE), twice = c0 + kE - n;
-  float v[kR][kE];
+  const bool live = row < rows && c0 < n;
+  const TI* xr = static_cast<const TI*>(x) + (row < rows ? row : 0) * ldx;
+  float v[kE];
 #pragma unroll
-  for (int r = 0; r < kR; ++r) {
-    const int64_t row = row0 + r * kWaveRows;
-    const bool live = row < rows && c0 < n;
-    const TI* xr = static_cast<const TI*>(x) + (row < rows ? row : 0) * ldx;
-    if (live && n >= kE) {
-      load_chunk<kIn, kE>(xr + at, v[r]);
-    } else {
+  for (int i = 0; i < kE; ++i) v[i] = -__builtin_inff();
+  if (n >= kE) {
+    if (live) load_chunk<kIn, kE>(xr + at, v);
+  } else if (live) {
 #pragma unroll
-      for (int i = 0; i < kE; ++i)
-        v[r][i] = live && c0 + i < n ? Elem<kIn>::load1(xr + c0 + i) : -__builtin_inff();
-    }
+    for (int i = 0; i < kE; ++i)
+      if (c0 + i < n) v[i] = Elem<kIn>::load1(xr + c0 + i);
   }
+  float m = -__builtin_inff();
 #pragma unroll
-  for (int r = 0; r < kR; ++r) {
-    const int64_t row = row0 + r * kWaveRows;
-    float m = -__builtin_inff();
+  for (int i = 0; i < kE; ++i) m = fmax_ordered(m, v[i]);
+  m = group_max<kL>(m);
 #pragma unroll
-    for (int i = 0; i < kE; ++i) m = fmax_ordered(m, v[r][i]);
-    m = group_max<kL>(m);
-    float s = 0.0f;
+  for (int i = 0; i < kE; ++i) v[i] = exp2_fast((v[i] - m) * kLog2e);   // -inf -> 0
+  float s = 0.0f;
+  if (n % kE == 0 || n < kE) {
 #pragma unroll
-    for (int i = 0; i < kE; ++i) {
-      v[r][i] = exp2_fast((v[r][i] - m) * kLog2e);   // -inf -> 0
-      s += i >= twice || n < kE ? v[r][i] : 0.0f;
-    }
-    s = group_sum<kL>(s);
-    if (row >= rows || c0 >= n) continue;   // (no lane exchanges below)
-    const float inv = 1.0f / s;
+    for (int i = 0; i < kE; ++i) s += v[i];
+  } else {
 #pragma unroll
-    for (int i = 0; i < kE; ++i) v[r][i] = normalise<kOut>(v[r][i], s, inv);
-    TO* yr = static_cast<TO*>(y) + row * ldy;
-    if (n >= kE) {
-      store_chunk<kOut, kE>(yr + at, v[r]);
-    } else {
+    for (int i = 0; i < kE; ++i) s += i >= twice ? v[i] : 0.0f;
+  }
+  s = group_sum<kL>(s);
+  if (!live) return;
+  const float inv = 1.0f / s;
 #pragma unroll
-      for (int i = 0; i < kE; ++i)
-        if (c0 + i < n) Elem<kOut>::store1(yr + c0 + i, v[r][i]);
-    }
+  for (int i = 0; i < kE; ++i) v[i] = normalise<kOut>(v[i], s, inv);
+  TO* yr = static_cast<TO*>(y) + row * ldy;
+  if (n >= kE) {
+    store_chunk<kOut, kE>(yr + at, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < kE; ++i)
+      if (c0 + i < n) Elem<kOut>::store1(yr + c0 + i, v[i]);
   }
 }
 
-#define SILE_SOFTMAX_NARROW(NAME, IN, OUT, L, R)                                                 \
+#define SILE_SOFTMAX_NARROW(NAME, IN, OUT, L)                                                    \
   extern "C" __global__ __launch_bounds__(256) void NAME(const void* x, void* y, int64_t rows,   \
                                                          int64_t cols, int64_t ldx, int64_t ldy) { \
-    softmax_rows_narrow_kernel<IN, OUT, L, R>(x, y, rows, cols, ldx, ldy);                       \
+    softmax_rows_narrow_kernel<IN, OUT, L>(x, y, rows, cols, ldx, ldy);                          \
   }
-#define SILE_SOFTMAX_NARROW_WIDTHS(TAG, IN, OUT)                       \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n4, IN, OUT, 4, 1)     \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n8, IN, OUT, 8, 1)     \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n16, IN, OUT, 16, 1)   \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n32, IN, OUT, 32, 1)   \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n4r4, IN, OUT, 4, 4)   \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n8r4, IN, OUT, 8, 4)   \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n16r4, IN, OUT, 16, 4) \
-  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n32r4, IN, OUT, 32, 4)
+#define SILE_SOFTMAX_NARROW_WIDTHS(TAG, IN, OUT)                 \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n4, IN, OUT, 4)   \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n8, IN, OUT, 8)   \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n16, IN, OUT, 16) \
+  SILE_SOFTMAX_NARROW(sile_softmax_rows_##TAG##_n32, IN, OUT, 32)
 SILE_SOFTMAX_NARROW_WIDTHS(f16_f16, kF16, kF16)
 SILE_SOFTMAX_NARROW_WIDTHS(bf16_bf16, kBF16, kBF16)
 SILE_SOFTMAX_NARROW_WIDTHS(f32_f32, kF32, kF32)
@@ -622,8 +617,10 @@ __device__ __forceinline__ void reduce_rows_tile_kernel(int op, const void* x, f
   if (t == 0) out[row] = acc;
 }
 
-// Narrow rows (up to 32 chunks): kL lanes per row, one chunk per lane, kR rows
-// a group of lanes (the narrow softmax's shapes).
+// Narrow rows (up to 32 chunks): kL lanes per row, one chunk per lane (the
+// narrow softmax's shapes).  kR = 4: four rows a group of lanes, all loaded before
+// the first is added, for the sums of large launches (bf16 500000 x 200 44.9 ->
+// 36.3 us); the max, with its columns, gains nothing.
 template <int kIn, int kL, int kR>
 __device__ __forceinline__ void reduce_rows_narrow_kernel(int op, const void* x, float* out,
                                                           int64_t rows, int64_t cols,
@@ -641,20 +638,22 @@ __device__ __forceinline__ void reduce_rows_narrow_kernel(int op, const void* x,
     const int64_t row = row0 + r * kWaveRows;
     const bool live = row < rows && c0 < n;
     const TI* xr = static_cast<const TI*>(x) + (row < rows ? row : 0) * ldx;
-    if (live && n >= kE) {
-      load_chunk<kIn, kE>(xr + at, v[r]);
-    } else {
-      const float pad = op == 0 ? __builtin_nanf("") : 0.0f;
+    const float pad = kR == 1 && op == 0 ? __builtin_nanf("") : 0.0f;
+#pragma unroll
+    for (int i = 0; i < kE; ++i) v[r][i] = pad;
+    if (n >= kE) {   // (the same for every lane)
+      if (live) load_chunk<kIn, kE>(xr + at, v[r]);
+    } else if (live) {
 #pragma unroll
       for (int i = 0; i < kE; ++i)
-        v[r][i] = live && c0 + i < n ? Elem<kIn>::load1(xr + c0 + i) : pad;
+        if (c0 + i < n) v[r][i] = Elem<kIn>::load1(xr + c0 + i);
     }
   }
 #pragma unroll
   for (int r = 0; r < kR; ++r) {
     const int64_t row = row0 + r * kWaveRows;
     const TI* xr = static_cast<const TI*>(x) + (row < rows ? row : 0) * ldx;
-    if (op == 0) {
+    if (kR == 1 && op == 0) {
       float m = -__builtin_inff();
       int mi = kNoCol;
 #pragma unroll
@@ -663,8 +662,13 @@ __device__ __forceinline__ void reduce_rows_narrow_kernel(int op, const void* x,
       if (row < rows && li == 0) out[row] = max_result<kIn>(m, xr);
     } else {
       float acc = 0.0f;
+      if (n % kE == 0) {
 #pragma unroll
-      for (int i = 0; i < kE; ++i) acc = acc + (i >= twice ? v[r][i] : 0.0f);
+        for (int i = 0; i < kE; ++i) acc = acc + v[r][i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < kE; ++i) acc = acc + (i >= twice ? v[r][i] : 0.0f);
+      }
       acc = group_sum<kL>(acc);
       if (row < rows && li == 0) out[row] = acc;
     }

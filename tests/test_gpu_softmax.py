@@ -393,8 +393,8 @@ def test_reduce_rows_at_any_element(hip, dt, cols):
 @pytest.mark.parametrize("dt", ["f16", "f32"])
 @pytest.mark.parametrize("cols", [3, 13, 64, 101, 250])
 def test_narrow_rows_four_a_group(hip, dt, cols):
-    """Launches large enough to take four rows a group of lanes, the last
-    workgroup and wave partly empty."""
+    """Large launches of narrow rows, the last workgroup and wave partly empty (a
+    row a group of lanes; the sums, four a group, below)."""
     rows = 140003 if cols <= 16 else 70001 if cols <= 64 else 40001
     say(f"narrow many {dt} {rows}x{cols}")
     x = rng(cols).normal(size=(rows, cols)).astype(np.float32)
@@ -468,4 +468,31 @@ def test_softmax_nan_reaches_the_whole_row(hip, dt, cols, off):
     e = np.exp(xf[6:].astype(np.float64) - xf[6:].max(1, keepdims=True))
     assert_close(y[6:], e / e.sum(1, keepdims=True), atol=1e-6, rtol=2e-5 if dt == "f32" else 1e-2)
     for b in (dx, dy):
+        b.close()
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("cols", [3, 13, 64, 101, 128, 250])
+@pytest.mark.parametrize("pad", [0, 5])
+def test_narrow_sums_four_a_group(hip, dt, cols, pad):
+    """Row sums of launches large enough to take four rows a group of lanes (8192
+    workgroups of one), the last one partly empty, whole and moved-back chunks;
+    within 1e-5 of the row's absolute sum."""
+    per = 4 if dt == "f32" else 8
+    lanes = next((n for n in (4, 8, 16, 32) if n * per >= cols), None)
+    if lanes is None:
+        pytest.skip("more than 32 chunks: not a narrow row")
+    rows, ldx = (1 << 21) // lanes + 3, cols + pad
+    say(f"narrow sums {dt} {rows}x{cols} pad={pad}")
+    x = rng(cols).normal(size=(rows, ldx)).astype(np.float32)
+    bits, xf = (x, x) if dt == "f32" else bf16_round(x) if dt == "bf16" else f16_round(x)
+    xf = xf[:, :cols]
+    dx, out = hip.DeviceBuffer.from_array(bits), hip.DeviceBuffer(4 * rows)
+    hip.reduce_rows(hip.REDUCE_SUM, {"f32": hip.F32, "f16": hip.F16, "bf16": hip.BF16}[dt], rows, cols,
+                    dx.ptr, ldx, out.ptr)
+    hip.synchronize()
+    got = out.download(np.float32, (rows,)).astype(np.float64)
+    assert (np.abs(got - xf.sum(1, dtype=np.float64))
+            <= 1e-5 * np.abs(xf).sum(1, dtype=np.float64)).all()
+    for b in (dx, out):
         b.close()
