@@ -26,7 +26,8 @@
 
 using namespace sile;
 
-enum DType : int { kF32 = 0, kF16 = 1, kBF16 = 2 };
+// kF32Merged: fp32 results of 16-bit rows, stored so that L2 merges them
+enum DType : int { kF32 = 0, kF16 = 1, kBF16 = 2, kF32Merged = 3 };
 
 // 16 bytes at any element address: rows of any pitch and start take the
 // 128-bit accesses (the memory pipeline takes unaligned ones).
@@ -59,6 +60,17 @@ struct Elem<kF32> {
   }
   SILE_DEV static float load1(const float* p) { return *p; }
   SILE_DEV static void store1(float* p, float v) { *p = v; }
+};
+// The fp32 results of 16-bit rows: a lane's 8 are two stores of 16 bytes, each
+// half of the lines it touches.  From 40 MiB on, plain stores let L2 merge the
+// halves (f16 16384 x 4000 105 -> 74 us); below, what the caches take as it comes,
+// non-temporal ones are faster (f16 8192 x 512 7.3 against 5.8).
+template <>
+struct Elem<kF32Merged> : Elem<kF32> {
+  SILE_DEV static void store8(float* p, const float v[8]) {
+    *reinterpret_cast<f32x4_any*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<f32x4_any*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
+  }
 };
 template <>
 struct Elem<kF16> {
@@ -150,7 +162,7 @@ SILE_DEV float waves_sum(const float* part) {
 // host libm expf of the reference (whose bits are not pinned by it).
 template <int kOut>
 SILE_DEV float normalise(float e, float s, float inv) {
-  if constexpr (kOut == kF32)
+  if constexpr (kOut == kF32 || kOut == kF32Merged)
     return e / s;
   else
     return e * inv;
@@ -267,6 +279,7 @@ SILE_SOFTMAX_TILES(f16_f16, kF16, kF16)
 SILE_SOFTMAX_TILES(bf16_bf16, kBF16, kBF16)
 SILE_SOFTMAX_TILES(f32_f32, kF32, kF32)
 SILE_SOFTMAX_TILES(f16_f32, kF16, kF32)
+SILE_SOFTMAX_TILES(f16_f32m, kF16, kF32Merged)
 // (4-element chunks: 64 values a thread at 16)
 SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 10)
 SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 12)
@@ -343,6 +356,7 @@ SILE_SOFTMAX_BLOCK_WIDTHS(f16_f16, kF16, kF16)
 SILE_SOFTMAX_BLOCK_WIDTHS(bf16_bf16, kBF16, kBF16)
 SILE_SOFTMAX_BLOCK_WIDTHS(f32_f32, kF32, kF32)
 SILE_SOFTMAX_BLOCK_WIDTHS(f16_f32, kF16, kF32)
+SILE_SOFTMAX_BLOCK_WIDTHS(f16_f32m, kF16, kF32Merged)
 
 // ---- narrow rows: kL lanes per row, one chunk per lane ----
 // cols <= kL * E; a wave holds 64 / kL rows and a workgroup of 4 waves
@@ -529,6 +543,7 @@ SILE_SOFTMAX_WIDE(f16_f16, kF16, kF16)
 SILE_SOFTMAX_WIDE(bf16_bf16, kBF16, kBF16)
 SILE_SOFTMAX_WIDE(f32_f32, kF32, kF32)
 SILE_SOFTMAX_WIDE(f16_f32, kF16, kF32)
+SILE_SOFTMAX_WIDE(f16_f32m, kF16, kF32Merged)
 
 // ---- row reduce (ReduceMax / ReduceSum along axis 1), fp32 result ----
 // op 0 = max, the reference's fold from x0 bit for bit (first_max_* in

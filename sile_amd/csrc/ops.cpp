@@ -821,6 +821,10 @@ int sile_hip_softmax_rows(sile_dtype in_type, sile_dtype out_type, int64_t rows,
   const int64_t elems = f32_rows ? 4 : 8;
   char name[64];
   int rc;
+  // (stores of fp32 results that L2 merges: from 40 MiB of them on, rows of more
+  // than 32 chunks)
+  if (in_type == SILE_F16 && out_type == SILE_F32 && cols > 32 * elems && rows * cols >= (10ll << 20))
+    tag = "f16_f32m";
   // rows of 256 / 512 / 1024 threads x 2 chunks: one row per workgroup
   int block_threads = 0;
   for (int t : {256, 512, 1024})

@@ -496,3 +496,28 @@ def test_narrow_sums_four_a_group(hip, dt, cols, pad):
             <= 1e-5 * np.abs(xf).sum(1, dtype=np.float64)).all()
     for b in (dx, out):
         b.close()
+
+
+def _softmax_check(hip, tin, tout, rows, cols, seed):
+    x = (rng(seed).normal(size=(rows, cols)) * 2.0).astype(np.float32)
+    bits, xf = (x, x) if tin == hip.F32 else f16_round(x)
+    dx, dy = hip.DeviceBuffer.from_array(bits), hip.DeviceBuffer(rows * cols * 4 + 64)
+    dy.fill_bytes(0x33)
+    hip.softmax_rows(tin, tout, rows, cols, dx.ptr, cols, dy.ptr, cols)
+    hip.synchronize()
+    raw = dy.download(np.float32, (rows * cols + 16,))
+    assert (raw[rows * cols:].view(np.uint32) == 0x33333333).all()
+    e = np.exp(xf.astype(np.float64) - xf.max(1, keepdims=True))
+    assert_close(raw[:rows * cols].reshape(rows, cols), e / e.sum(1, keepdims=True), atol=1e-6, rtol=2e-5)
+    for b in (dx, dy):
+        b.close()
+
+
+@pytest.mark.parametrize("rows,cols", [(41000, 257), (5500, 2000), (2100, 5001), (1300, 8192), (700, 16384),
+                                       (330, 32003), (161, 65535), (150, 70001)])
+def test_f16_to_f32_softmax_merged_stores(hip, rows, cols):
+    """fp32 results of 16-bit rows past 40 MiB: the plain stores, in every shape of
+    row kernel."""
+    say(f"softmax f16 -> f32 merged stores {rows}x{cols}")
+    assert rows * cols >= 10 << 20
+    _softmax_check(hip, hip.F16, hip.F32, rows, cols, cols)
