@@ -285,6 +285,15 @@ SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 10)
 SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 12)
 SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 14)
 SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 1024, 16)
+// (a wave a row past 4 chunks: the host's rule has the row counts)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 64, 5)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 64, 6)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 64, 7)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 64, 8)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 64, 10)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 64, 12)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 64, 14)
+SILE_SOFTMAX_TILE(f32_f32, kF32, kF32, 64, 16)
 
 // ---- one row per workgroup: cols == kThreads * kChunks * E ----
 // The copy shape that moves the most bytes on MI355X (two 16-byte chunks per
@@ -866,9 +875,11 @@ SILE_REDUCE_SHAPES(bf16, kBF16)
   SILE_REDUCE_TILE(TAG, IN, 64, 2)    \
   SILE_REDUCE_TILE(TAG, IN, 64, 3)    \
   SILE_REDUCE_TILE(TAG, IN, 64, 4)    \
+  SILE_REDUCE_TILE(TAG, IN, 128, 3)   \
   SILE_REDUCE_TILE(TAG, IN, 256, 2)   \
   SILE_REDUCE_TILE(TAG, IN, 256, 3)   \
   SILE_REDUCE_TILE(TAG, IN, 256, 4)   \
+  SILE_REDUCE_TILE(TAG, IN, 512, 2)   \
   SILE_REDUCE_TILE(TAG, IN, 512, 3)   \
   SILE_REDUCE_TILE(TAG, IN, 512, 4)   \
   SILE_REDUCE_TILE(TAG, IN, 512, 5)   \

@@ -850,7 +850,19 @@ int sile_hip_softmax_rows(sile_dtype in_type, sile_dtype out_type, int64_t rows,
   }
   // other widths: in registers up to 65536 elements (64 a thread), in two
   // passes over the row beyond
-  const RowTile tile = row_tile((cols + elems - 1) / elems, f32_rows ? 16 : 8);
+  const int64_t n = (cols + elems - 1) / elems;
+  RowTile tile = row_tile(n, f32_rows ? 16 : 8);
+  int cus = 0;
+  // fp32 rows of 5 to 16 chunks a lane: workgroups of 256, eight a CU, would need
+  // a second round where waves of a row each, 16 (12 past 8 chunks) a CU, are
+  // resident at once.  Workgroup / wave: 2500 x 2000 8.8 / 8.3 us, 4096 x 2000 13.0 /
+  // 12.2, 3000 x 4000 17.9 / 16.7; but 2000 x 2000 6.4 / 7.0 (start of the range),
+  // 5000 x 2000 15.3 / 15.4, 2500 x 4000 15.6 / 17.0
+  if (f32_rows && n > 256 && n <= 1024 && device_cus(&cus) == SILE_OK &&
+      rows > (n <= 640 ? 8 : 10) * cus && rows <= (n <= 512 ? 16 : 12) * cus) {
+    const int c = (int)((n + 63) / 64);
+    tile = {64, c > 8 ? c + (c & 1) : c};
+  }
   void* params[] = {&x, &y, &rows, &cols, &ldx, &ldy};
   if (tile.threads)
     snprintf(name, sizeof name, "sile_softmax_rows_%s_t%dc%d", tag, tile.threads, tile.chunks);
@@ -910,8 +922,16 @@ int sile_hip_reduce_rows(sile_reduce_op op, sile_dtype in_type, int64_t rows, in
     }
   }
   // (16-bit rows at 5 chunks a thread, 40 values: bf16 1000 x 40000 14.7 us, the loop 13.4)
-  const RowTile tile = row_tile((cols + elems - 1) / elems, in_type == SILE_F32 ? 5 : 4);
+  const int64_t n = (cols + elems - 1) / elems;
+  RowTile tile = row_tile(n, in_type == SILE_F32 ? 5 : 4);
   int cus = 0;
+  if (op == SILE_REDUCE_MAX && n > 256 && n <= 320)
+    tile = {128, 3};   // fp32 40000 x 1100: 35.6 -> 31.0 us with fewer idle lanes than 256 x 2
+  // (full 512 x 2 rather than 256 x 4: fp32 max 16384 x 4000 42.3 -> 37.8 us, sum 41.5
+  // -> 40.4; 2500 x 4000 8.3 against 8.8)
+  if (n > 896 && n <= 1024 && device_cus(&cus) == SILE_OK && rows >= 16 * cus) tile = {512, 2};
+  if (cols >= 16384 && device_cus(&cus) == SILE_OK && rows <= 2 * cus)
+    tile.threads = 0;   // few wide rows: the loop (bf16 300 x 32768 5.6 -> 5.2 us)
   if (tile.threads)
     snprintf(kname, sizeof kname, "%s_t%dc%d", name, tile.threads, tile.chunks);
   else

@@ -521,3 +521,38 @@ def test_f16_to_f32_softmax_merged_stores(hip, rows, cols):
     say(f"softmax f16 -> f32 merged stores {rows}x{cols}")
     assert rows * cols >= 10 << 20
     _softmax_check(hip, hip.F16, hip.F32, rows, cols, cols)
+
+
+@pytest.mark.parametrize("cols", [1025, 1281, 1537, 2047, 2049, 2560, 2561, 3073, 3585, 4093])
+def test_f32_softmax_a_wave_a_row(hip, cols):
+    """fp32 rows of 5 to 16 chunks a lane at the row counts where a wave takes a
+    row: the first count past 8 (10 from 641 chunks on) workgroups a CU."""
+    cus = hip.device_info(0)["compute_units"]
+    rows = (8 if cols <= 2560 else 10) * cus + 1
+    say(f"softmax f32 wave a row {rows}x{cols}")
+    _softmax_check(hip, hip.F32, hip.F32, rows, cols, cols)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,chunks", [(7, 257), (7, 319.5), (7, 320), (7, 321), (4099, 896.5), (4097, 897),
+                                         (4099, 1000.25), (4096, 1024), (511, 4096.5), (513, 4096)])
+def test_reduce_rows_tile_choices(hip, dt, rows, chunks):
+    """Row max (exact) and sum (within 1e-5 of the row's absolute sum) around the
+    edges of the row counts and widths that choose a tile: 257 .. 320 chunks, 897 ..
+    1024 chunks of many rows, wide rows of few."""
+    cols = int(chunks * (4 if dt == "f32" else 8))
+    say(f"reduce tiles {dt} {rows}x{cols}")
+    tin = hip.F32 if dt == "f32" else hip.BF16
+    x = rng(rows + cols).normal(size=(rows, cols)).astype(np.float32)
+    bits, xf = (x, x) if dt == "f32" else bf16_round(x)
+    dx, out = hip.DeviceBuffer.from_array(bits), hip.DeviceBuffer(4 * rows)
+    hip.reduce_rows(hip.REDUCE_MAX, tin, rows, cols, dx.ptr, cols, out.ptr)
+    hip.synchronize()
+    np.testing.assert_array_equal(out.download(np.float32, (rows,)), xf.max(1))
+    hip.reduce_rows(hip.REDUCE_SUM, tin, rows, cols, dx.ptr, cols, out.ptr)
+    hip.synchronize()
+    got = out.download(np.float32, (rows,)).astype(np.float64)
+    assert (np.abs(got - xf.sum(1, dtype=np.float64))
+            <= 1e-5 * np.abs(xf).sum(1, dtype=np.float64)).all()
+    for b in (dx, out):
+        b.close()
