@@ -121,20 +121,6 @@ SILE_DEV float wave_sum(float v) {
   return pair32_sum(v);
 }
 
-// max and sum over each 16-lane row of the wave (all 16 lanes hold the result)
-SILE_DEV float group_max16(float v) {
-  v = fmax_ordered(v, dpp<kDppXor1>(v));
-  v = fmax_ordered(v, dpp<kDppXor2>(v));
-  v = fmax_ordered(v, dpp<kDppHalfMirror>(v));
-  return fmax_ordered(v, dpp<kDppMirror>(v));
-}
-SILE_DEV float group_sum16(float v) {
-  v += dpp<kDppXor1>(v);
-  v += dpp<kDppXor2>(v);
-  v += dpp<kDppHalfMirror>(v);
-  return v + dpp<kDppMirror>(v);
-}
-
 // ---- the reference's row max, computed in parallel ----
 // ReduceMax folds from the row's first element, acc = x0; acc = x > acc ? x : acc
 // (crates/sile-tile-ir/src/passes/lowering/tile_compute/reduce.rs:10-30), so
@@ -270,5 +256,51 @@ SILE_DEV float fused_sum_rows_tiled(const float* __restrict__ x, int64_t cols, i
 
 // 2^x on the transcendental unit (v_exp_f32).
 SILE_DEV float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// One query row of softmax(q K^T * scale) V by a wave, fp32 throughout with an
+// online softmax (running max m, running sum l, rescaled accumulator): keys
+// 0 .. nkeys - 1 of K and V [.., d], d <= 256, scale_log2 = scale * log2 e.  Keys
+// past nkeys are not read, so what they hold cannot reach the row.
+template <bool kBF16>
+SILE_DEV void attn_row(const uint16_t* qi, const uint16_t* kb, const uint16_t* vb, uint16_t* oi,
+                       int64_t nkeys, int d, float scale_log2) {
+  const int lane = threadIdx.x & 63;
+  auto ld16 = [](const uint16_t* p) { return kBF16 ? bf16_to_f32(*p) : f16_to_f32(*p); };
+  float qv[4], acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int dd = lane + 64 * t;
+    qv[t] = dd < d ? ld16(qi + dd) * scale_log2 : 0.0f;
+    acc[t] = 0.0f;
+  }
+  float m = -__builtin_inff(), l = 0.0f;
+  for (int64_t j = 0; j < nkeys; ++j) {
+    const uint16_t* kj = kb + j * d;
+    float s = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int dd = lane + 64 * t;
+      if (dd < d) s += qv[t] * ld16(kj + dd);
+    }
+    s = wave_sum(s);  // score in log2 units
+    const float m_new = fmax_ordered(m, s);
+    const float alpha = exp2_fast(m - m_new);
+    const float p = exp2_fast(s - m_new);
+    l = l * alpha + p;
+    const uint16_t* vj = vb + j * d;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int dd = lane + 64 * t;
+      if (dd < d) acc[t] = acc[t] * alpha + p * ld16(vj + dd);
+    }
+    m = m_new;
+  }
+  const float inv = 1.0f / l;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int dd = lane + 64 * t;
+    if (dd < d) oi[dd] = kBF16 ? bf16_rne(acc[t] * inv) : f16_rne(acc[t] * inv);
+  }
+}
 
 }  // namespace sile

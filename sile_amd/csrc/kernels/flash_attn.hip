@@ -118,9 +118,11 @@ struct AttnArgs {
 //
 // A head_dim that is an odd multiple of 8 has zeros in the upper half of its
 // last 16-dim step (both operands) and O^T rows past it that are not stored.
-// Without this kernel such calls take a wave a query row on the VALU with P in
-// fp32, so here P goes into the product as two 16-bit parts, its value and the
-// rest (16 bits of it in bf16, 22 in f16), and its sum is of the fp32 values.
+// Without this kernel such calls take a wave a query row on the VALU, with P in
+// fp32 and no key past a causal query read, and they keep both here: P goes into
+// the product as two 16-bit parts, value and rest (16 bits of it in bf16, 22 in
+// f16), its sum in fp32; and a row whose result is not finite, as an Inf or NaN
+// in a masked key's V makes it (0 times Inf), is taken again by attn_row.
 // 2 x 2814 x 72 causal: 2355 us on the VALU, 27 here (22 with P in one part); 64 x
 // 4096 x 120 causal: 380 us (270).
 //
@@ -178,7 +180,8 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
   constexpr int kKK = (kDh + 15) / 16;   // d-steps of S^T = K . Q^T
   constexpr int kDT = (kDh + 31) / 32;   // 32-d tiles of O^T
   constexpr int kDmaRows = 1024 / kRow;  // rows one 1 KiB DMA instruction fills
-  // P in two 16-bit parts (the header comment on odd multiples of 8)
+  // P in two 16-bit parts, and rows with a result that is not finite taken again
+  // by attn_row (the header comment on odd multiples of 8)
   constexpr bool kFullP = kDh % 16 == 8;
   constexpr int kPV = 2 * kST;                 // 16-key chunks of a P block
   constexpr int kPN = kFullP ? 2 * kPV : kPV;  // register quads of it: chunks, then their rests
@@ -663,7 +666,23 @@ __device__ __forceinline__ void attn_fwd_v2(const uint16_t* __restrict__ Q,
       const float l = pair32_sum(l_run[qt]);
       const float inv = 1.0f / l;
       const int q = wq0 + 32 * qt + l32;
-      if (q >= S) continue;
+      bool again = false;
+      if constexpr (kFullP) {
+        float z = l * 0.0f;
+  #pragma unroll
+        for (int dt = 0; dt < kDT; ++dt)
+  #pragma unroll
+          for (int i = 0; i < 16; ++i) z = __builtin_fmaf(oacc[qt][dt][i] * inv, 0.0f, z);
+        const uint64_t bad = __builtin_amdgcn_ballot_w64(!(z == 0.0f) && q < S);
+        uint32_t rows = (uint32_t)bad | (uint32_t)(bad >> 32);   // query l32: bit l32
+        again = (rows >> l32) & 1;
+        for (; rows; rows &= rows - 1) {
+          const int64_t row = wq0 + 32 * qt + __builtin_ctz(rows);
+          attn_row<kBF16>(Q + head_off + row * kDh, K + head_off, V + head_off,
+                          O + head_off + row * kDh, a.causal ? row + 1 : S, kDh, c);
+        }
+      }
+      if (q >= S || again) continue;
       uint16_t* orow = O + head_off + (int64_t)q * kDh;
   #pragma unroll
       for (int dt = 0; dt < kDT; ++dt)

@@ -378,6 +378,34 @@ def test_flash_head_dims_of_8_precision(hip, dt, causal, h, s, d):
         assert_close(got[0, hi], p @ vf[hi] / p.sum(1, keepdims=True), atol=atol, rtol=rtol, what=f"h{hi}")
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("h,s,d", [(1, 70, 8), (3, 300, 40), (8, 300, 72), (8, 1500, 120), (2, 200, 136),
+                                   (3, 100, 100)])
+def test_flash_masked_keys_do_not_reach_a_row(hip, dt, h, s, d):
+    """Causal, head dims that are no multiple of 16: Inf in one element of V, then
+    NaN in a row of V and of K, at keys in the middle.  Rows before them are as if
+    these keys held zeros; from the Inf on its dim is Inf, or NaN where its weight
+    is 0; from the NaN rows on everything is NaN."""
+    say(f"flash masked Inf / NaN D={d} {dt} H={h} S={s}")
+    scale = 1.0 / np.sqrt(d)
+    k1, k2 = s // 3, 2 * s // 3
+    (_, q), (_, k), (_, v) = _inputs(1, h, s, d, dt, seed=d)
+    rnd = f16_round if dt == "f16" else bf16_round
+    bad_k, bad_v = k.copy(), v.copy()
+    bad_v[0, :, k1, 3] = np.inf
+    bad_v[0, :, k2] = np.nan
+    bad_k[0, 0, k2 + 1] = np.nan
+    got = _run(hip, dt, 1, h, s, d, [rnd(x)[0] for x in (q, bad_k, bad_v)], True, scale)
+    for hi in range(h):
+        ref = cpuref.attention_fwd(q[0, hi], k[0, hi], v[0, hi], scale, causal=True)
+        assert_close(got[0, hi, :k1], ref[:k1], atol=ATOL, rtol=RTOL, what=f"h{hi} before the Inf")
+        other = np.arange(d) != 3
+        assert not np.isfinite(got[0, hi, k1:k2, 3]).any()
+        assert_close(got[0, hi, k1:k2, other].T, ref[k1:k2, other], atol=ATOL, rtol=RTOL,
+                     what=f"h{hi} beside the Inf")
+        assert np.isnan(got[0, hi, k2:]).all()
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_flash_long_sequence(hip, causal):
     """S = 65536 (B = 1, H = 8, D = 128, f16): block, key and byte offsets at
