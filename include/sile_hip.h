@@ -425,9 +425,10 @@ int sile_hip_attention_f32_kt(int64_t n_q, int64_t n_k, int64_t head_dim, const 
  * in 16 bits, for D an odd multiple of 8 as two 16-bit parts; with D a multiple
  * of 16 a causal row takes in 0 times the V rows of later keys of its block, so
  * an Inf or NaN there makes it NaN, with any other D it does not); other D up to
- * 256 (or unaligned operands) on a VALU kernel of one wave per query row.  No
- * reference counterpart: sile's DSL cannot express attention (no mask/iota/transpose); built from the Tile IR
- * ops MmaF, ReduceMax, Exp, ReduceSum (crates/sile-tile-ir/src/ir.rs:128-262). */
+ * 256, unaligned operands and a scale that is not positive on a VALU kernel of
+ * one wave per query row.  No reference counterpart: sile's DSL cannot express
+ * attention (no mask/iota/transpose); built from the Tile IR ops MmaF, ReduceMax,
+ * Exp, ReduceSum (crates/sile-tile-ir/src/ir.rs:128-262). */
 int sile_hip_flash_attn_fwd(sile_dtype dtype, int64_t batch, int64_t heads, int64_t seq_len,
                             int64_t head_dim, const void *q, const void *k, const void *v,
                             void *o, float scale, int causal, sile_hip_stream stream);

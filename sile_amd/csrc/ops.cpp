@@ -1154,9 +1154,11 @@ int sile_hip_flash_attn_fwd(sile_dtype dtype, int64_t batch, int64_t heads, int6
   // (32-query waves, key blocks through LDS-DMA; keys and queries past S
   // masked; laid out by flash_plan), one instantiation per head dimension (a
   // multiple of 8 up to 256) and key group count: 8 waves up to 128 (32-key
-  // blocks, or 64-key blocks over 128-byte rows up to 64), 4 waves past 128.
+  // blocks, or 64-key blocks over 128-byte rows up to 64), 4 waves past 128.  Its
+  // running max is of the scores before the scale, so that a scale that is not
+  // positive goes to the wave-a-row kernel.
   const bool aligned = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o);
-  if (head_dim % 8 == 0 && aligned) {
+  if (head_dim % 8 == 0 && aligned && scale > 0.0f) {
     const char* dt = dtype == SILE_F16 ? "f16" : "bf16";
     const int waves = head_dim <= 128 ? 8 : 4;
     const FlashPlan plan = flash_plan(bh, seq_len, (int)head_dim, causal != 0);

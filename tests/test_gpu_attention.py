@@ -406,6 +406,22 @@ def test_flash_masked_keys_do_not_reach_a_row(hip, dt, h, s, d):
         assert np.isnan(got[0, hi, k2:]).all()
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("scale", [-0.3, 0.0])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("h,s,d", [(1, 33, 8), (2, 130, 40), (2, 300, 72), (2, 130, 64), (1, 130, 128),
+                                   (1, 70, 136), (1, 70, 36)])
+def test_flash_scale_not_positive(hip, h, s, d, causal, scale, dt):
+    """Negative and zero scales, every kind of head dim."""
+    say(f"flash scale={scale} D={d} {dt} H={h} S={s} causal={causal}")
+    qkv = _inputs(1, h, s, d, dt, seed=d)
+    q, k, v = (x[1] for x in qkv)
+    got = _run(hip, dt, 1, h, s, d, [x[0] for x in qkv], causal, scale)
+    for hi in range(h):
+        ref = cpuref.attention_fwd(q[0, hi], k[0, hi], v[0, hi], scale, causal=causal)
+        assert_close(got[0, hi], ref, atol=ATOL, rtol=RTOL, what=f"h{hi}")
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_flash_long_sequence(hip, causal):
     """S = 65536 (B = 1, H = 8, D = 128, f16): block, key and byte offsets at
