@@ -341,6 +341,130 @@ __device__ __forceinline__ void matvec_rows_block(const float* __restrict__ x,
   if (t < rows) out[row0 + t] = acc;
 }
 
+// Short rows: a wave a row (or 8 of them), so that few threads idle past a row's
+// end and no barrier stands between rows.  The same tiles, chains and order, a span
+// of 256 elements (64 lanes x 16 bytes) at a time.  300000 rows of 64: 49 - 118 us
+// (BK 4 - 64) a workgroup for four rows, 17 - 57 here; rows of 768 are up to 1.5
+// times slower here.  BK 16, 32 and 64: the partials are added through readlane.
+template <int kL>
+__device__ __forceinline__ void matvec_rows_wave(const float* __restrict__ x,
+                                                 const float* __restrict__ y,
+                                                 float* __restrict__ out, const MatvecArgs& a) {
+#pragma clang fp contract(off)
+  typedef float Chunk __attribute__((ext_vector_type(4), aligned(4)));   // any element
+  constexpr int kU = 2;              // spans in flight
+  const int lane = threadIdx.x & 63, s = lane % kL;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= a.m) return;   // the whole wave
+  const float* xr = x + row * a.ldx;
+  const int64_t n = a.tiles * 4 * kL;   // elements of the whole tiles
+  float acc = a.seed;
+  for (int64_t base = 0; base < n; base += 256 * kU) {
+    f32x4 xv[kU], yv[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int64_t e = base + 256 * u + 4 * lane;
+      xv[u] = yv[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (e < n) {
+        xv[u] = __builtin_nontemporal_load(reinterpret_cast<const Chunk*>(xr + e));
+        yv[u] = *reinterpret_cast<const Chunk*>(y + e);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int64_t b = base + 256 * u;
+      if (b >= n) break;
+      const float p0 = xv[u][0] * yv[u][0], p1 = xv[u][1] * yv[u][1];
+      const float p2 = xv[u][2] * yv[u][2], p3 = xv[u][3] * yv[u][3];
+      float p = 0.0f, carry = 0.0f;
+#pragma unroll
+      for (int step = 0; step < kL; ++step) {
+        float c = step == 0 ? p0 : carry + p0;
+        c = c + p1;
+        c = c + p2;
+        c = c + p3;
+        p = s == step ? c : p;
+        if (step + 1 < kL) carry = dpp<0x111>(p);   // row_shr:1
+      }
+      const int g_n = (int)min<int64_t>(64 / kL, (n - b) / (4 * kL));
+      for (int g = 0; g < g_n; ++g)
+        acc = acc + __builtin_bit_cast(
+                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), g * kL + kL - 1));
+    }
+  }
+  if (lane == 0) out[row] = acc;
+}
+
+// LDS written by a wave before, read by the wave after (and the reverse): in order
+// in hardware, so this only holds the compiler.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// BK 4 and 8 (up to 64 tiles a span): kR rows a wave, their partials in LDS, and
+// lane r adds row r's, so that one add serves kR rows.
+template <int kL, int kR>
+__device__ __forceinline__ void matvec_rows_multi(const float* __restrict__ x,
+                                                  const float* __restrict__ y,
+                                                  float* __restrict__ out, const MatvecArgs& a) {
+#pragma clang fp contract(off)
+  typedef float Chunk __attribute__((ext_vector_type(4), aligned(4)));   // any element
+  constexpr int kG = 64 / kL;        // tiles per span
+  __shared__ float part[4][kR][kG];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, s = lane % kL;
+  const int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * kR;
+  if (row0 >= a.m) return;   // the whole wave
+  const int64_t n = a.tiles * 4 * kL;   // elements of the whole tiles
+  float acc = a.seed;                   // lane r < kR: row row0 + r
+  for (int64_t base = 0; base < n; base += 256) {
+    const int64_t e = base + 4 * lane;
+    f32x4 yv = {0.0f, 0.0f, 0.0f, 0.0f}, xv[kR];
+    if (e < n) yv = *reinterpret_cast<const Chunk*>(y + e);
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      xv[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (e < n && row0 + r < a.m)
+        xv[r] = __builtin_nontemporal_load(
+            reinterpret_cast<const Chunk*>(x + (row0 + r) * a.ldx + e));
+    }
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      const float p0 = xv[r][0] * yv[0], p1 = xv[r][1] * yv[1];
+      const float p2 = xv[r][2] * yv[2], p3 = xv[r][3] * yv[3];
+      float p = 0.0f, carry = 0.0f;
+#pragma unroll
+      for (int step = 0; step < kL; ++step) {
+        float c = step == 0 ? p0 : carry + p0;
+        c = c + p1;
+        c = c + p2;
+        c = c + p3;
+        p = s == step ? c : p;
+        if (step + 1 < kL) carry = dpp<0x111>(p);   // row_shr:1
+      }
+      if (s == kL - 1) part[wave][r][lane / kL] = p;
+    }
+    wave_order();
+    const int g_n = (int)min<int64_t>(kG, (n - base) / (4 * kL));
+    if (lane < kR)
+      for (int g = 0; g < g_n; ++g) acc = acc + part[wave][lane][g];
+    wave_order();
+  }
+  if (lane < kR && row0 + lane < a.m) out[row0 + lane] = acc;
+}
+
+#define SILE_MATVEC_WAVE(L, BODY)                                                              \
+  extern "C" __global__ __launch_bounds__(256) void sile_dsl_matvec_f32_l##L##_wave(           \
+      const float* x, const float* y, float* out, MatvecArgs a) {                              \
+    BODY(x, y, out, a);                                                                        \
+  }
+SILE_MATVEC_WAVE(1, (matvec_rows_multi<1, 8>))
+SILE_MATVEC_WAVE(2, (matvec_rows_multi<2, 8>))
+SILE_MATVEC_WAVE(4, matvec_rows_wave<4>)
+SILE_MATVEC_WAVE(8, matvec_rows_wave<8>)
+SILE_MATVEC_WAVE(16, matvec_rows_wave<16>)
+
 #define SILE_MATVEC_BLOCK(L, R, U)                                                             \
   extern "C" __global__ __launch_bounds__(256) void sile_dsl_matvec_f32_l##L##_r##R(           \
       const float* x, const float* y, float* out, MatvecArgs a) {                              \

@@ -777,11 +777,25 @@ int sile_hip_matvec_f32(int64_t m, int64_t k, int64_t bk, const float* x, int64_
   char name[40];
   int64_t rows_per_block = 4;
   if (bk == 4 || bk == 8 || bk == 16 || bk == 32 || bk == 64) {
-    // a row a workgroup (four spans of it in flight) while that is needed to
-    // fill the CUs: 512 x 8192, BK 32: 6.2 us against 9.0 with four rows; 2048 x
-    // 8192: 14.3 against 13.8, 2048 x 2048, BK 8: 6.3 against 5.9
-    rows_per_block = m <= 1024 ? 1 : 4;
-    snprintf(name, sizeof name, "sile_dsl_matvec_f32_l%d_r%d", (int)(bk / 4), (int)rows_per_block);
+    int cus = 0;
+    int rc = device_cus(&cus);
+    if (rc != SILE_OK) return rc;
+    // Short rows: a wave a row, 8 rows for BK 4 and 8.  20000 rows, us a call by
+    // workgroups / waves: BK 4, 256 elements 6.0 / 5.6, 384 6.9 / 7.2 (131072 rows of
+    // 288: 28.0 / 24.1); BK 16, 128 6.1 / 5.7, 192 6.3 / 6.4; BK 32, 256 7.1 / 6.6,
+    // 384 7.7 / 8.3; BK 64, 512 10.7 / 9.3, 640 12.1 / 12.6
+    const int64_t row = args.tiles * bk;
+    const int64_t most = bk == 64 ? 512 : bk == 16 ? 128 : bk <= 8 && m >= 256ll * cus ? 384 : 256;
+    if (row <= most) {
+      rows_per_block = bk <= 8 ? 32 : 4;
+      snprintf(name, sizeof name, "sile_dsl_matvec_f32_l%d_wave", (int)(bk / 4));
+    } else {
+      // a row a workgroup (four spans of it in flight) while that is needed to
+      // fill the CUs: 512 x 8192, BK 32: 6.2 us against 9.0 with four rows; 2048 x
+      // 8192: 14.3 against 13.8, 2048 x 2048, BK 8: 6.3 against 5.9
+      rows_per_block = m <= 4ll * cus ? 1 : 4;
+      snprintf(name, sizeof name, "sile_dsl_matvec_f32_l%d_r%d", (int)(bk / 4), (int)rows_per_block);
+    }
   } else {
     const bool vec4 = bk % 4 == 0 && ldx % 4 == 0 && aligned16(x) && aligned16(y);
     snprintf(name, sizeof name, "%s", vec4 ? "sile_dsl_matvec_f32_v4" : "sile_dsl_matvec_f32");

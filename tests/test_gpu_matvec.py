@@ -49,9 +49,15 @@ def _matvec(hip, x, y, bk, m=None, k=None, seed=0.0, x_off=0, y_off=0):
     (16, 1000, 16, 1000, 0),     # 62 tiles, K truncated to 992
     (16, 4096, 64, 4096, 0),     # 16 lanes a tile
     (8, 8200, 8, 8204, 0),       # pitch > K, 1025 tiles
-    # BK 4 and 8: eight rows a wave
-    (13, 1000, 8, 1000, 0),      # a wave with 5 rows past m
-    (37, 520, 4, 520, 0),        # 130 tiles, a partial last span
+    # BK 4 and 8 past the short rows: the block kernel
+    (13, 1000, 8, 1000, 0), (37, 520, 4, 520, 0),
+    # short rows, a wave a row or 8 rows (BK 4 and 8): rows past m in the last wave,
+    # partial spans, rows at any element, the longest row of each BK and one past it
+    (13, 256, 8, 256, 0), (37, 252, 4, 253, 1), (1, 4, 4, 4, 0), (9, 255, 8, 257, 3),
+    (33, 260, 4, 260, 0), (5, 128, 16, 131, 2), (6, 144, 16, 144, 0), (3, 16, 16, 16, 0),
+    (7, 256, 32, 256, 0), (2, 287, 32, 301, 1), (5, 512, 64, 515, 1), (3, 575, 64, 575, 0),
+    (4, 64, 64, 64, 0), (2050, 200, 8, 201, 1), (65537, 384, 4, 384, 0), (65540, 383, 8, 385, 1),
+    (65536, 388, 4, 388, 0),
     # the block kernel: one and four rows a workgroup (from 1025 rows on), spans
     # of 1024 elements, blocks of one or four of them, rows at any element
     (1, 4096, 4, 4096, 0), (3, 4100, 4, 4101, 1), (1024, 1028, 4, 1029, 3),
