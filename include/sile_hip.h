@@ -280,6 +280,11 @@ int sile_hip_kernel_parallel_reduce(void *const *buffers, int64_t num_threadgrou
  *                        once (plain launch, also under capture) takes the
  *                        place of either, wherever it is modelled faster or
  *                        the tiles cannot take the shape.
+ *                        Pitches past 2^31 bytes in 256 rows are refused for
+ *                        the tiles' own shapes (C rows of 16-byte aligned
+ *                        multiples of 4; N below one tile and M a multiple of
+ *                        4 from 128 on); other shapes, and operands of at most
+ *                        64 rows, take a kernel without such panels.
  * When the tiles are fewer than the device's CUs and K' is long, K' may be
  * split into ranges computed side by side: their fp32 partial C planes go
  * to a device scratch buffer shared by all calls on the device (allocated on

@@ -522,10 +522,18 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
   // the header names
   const int64_t min_tile = tile_req ? tile_req : 128;
   const bool lds_ok = (min_tile == 128 || m >= min_tile) && n >= min_tile;
-  if (tile_req && !(lds_ok && n % 4 == 0 && (ldc * cb) % 16 == 0 && aligned16(c)))
+  const bool c_rows_ok = n % 4 == 0 && (ldc * cb) % 16 == 0 && aligned16(c);
+  if (tile_req && !(lds_ok && c_rows_ok))
     return fail(SILE_ERR_SHAPE,
                 "%d x %d tiles need %sN >= %d, N a multiple of 4 and C's rows 16-byte aligned",
                 tile_req, tile_req, tile_req == 256 ? "M, " : "", tile_req);
+  // The tiles address a panel of 256 rows of A or B as one buffer resource, a
+  // 32-bit byte range.  Larger pitches are refused where the tiles are the form
+  // asked for (C's rows as the header names them, or M a multiple of 4 in the
+  // transposed form); the shapes that only stores to any element of C bring to the
+  // tiles run on the any-shape kernel instead.
+  const bool panels_fit = 256 * std::max(lda, b_row ? 0 : ldb) * (int64_t)eb <= 0x7fffffffLL;
+  const bool direct = lds_ok && (panels_fit || c_rows_ok);
   // The transposed form runs C^T = B . A^T (A and B swapped) into fp32
   // planes of C^T and writes them back transposed, where N is below one tile
   // and M, as the column extent, is not.
@@ -545,7 +553,7 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
   // start on a 16-byte boundary; B's rows 0 .. K as one buffer resource).
   // Other row-major shapes and fp8 write B column-major into the device
   // scratch first (slot 1) and take the column-major path below.
-  if (b_row && !(eb == 2 && lds_ok && n % 8 == 0 && (ldb * eb) % 16 == 0 && aligned16(b) &&
+  if (b_row && !(eb == 2 && direct && n % 8 == 0 && (ldb * eb) % 16 == 0 && aligned16(b) &&
                  (double)k * (double)ldb * (double)eb <= 2147483647.0)) {
     if (capturing)
       return fail(SILE_ERR_UNSUPPORTED_BACKEND, "row-major B of this shape needs the device "
@@ -582,8 +590,8 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
       64 * std::max(lda, ldb) * (int64_t)eb <= 0x7fffffffLL) {
     double few_t = 0.0;
     const int r = gemm_few_tiles(rows_s, rows_l, kp * (int64_t)eb, &few_t);
-    bool use = !lds_ok;
-    if (lds_ok) {
+    bool use = !direct || !panels_fit;
+    if (!use) {
       const GemmPlan plan = gemm_plan(m, n, kp, (kp + kstep - 1) / kstep, (int64_t)cb, fp8, 0);
       // (the tiles' model leaves out the operands' bytes and ~4 us of what a
       // launch of few tiles with a deep split measures)
@@ -613,9 +621,10 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
       return rc == SILE_OK ? ok() : rc;
     }
   }
-  const bool transposed = !b_row && !lds_ok && !capturing && m >= 128 &&
+  const bool transposed = !b_row && !direct && !capturing && m >= 128 &&
+                          (panels_fit || m % 4 == 0) &&
                           (m + 3) / 4 * 4 * n * 4 <= kScratchPlanesMax;
-  if (!lds_ok && !transposed) {
+  if (!direct && !transposed) {
     // the any-shape kernel, 64 x 64 tiles with fragments loaded straight
     // from the operands
     const int64_t gx = (n + 63) / 64, gy = (m + 63) / 64;
@@ -638,8 +647,7 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
   const int64_t rlda = transposed ? ldb : lda, rldb = transposed ? lda : ldb;
   const int64_t rm = transposed ? n : m, rn = transposed ? m : n;
   const int64_t pitch = (rn + 3) / 4 * 4;   // of a row of the fp32 planes
-  // a tile's panel of A or B is one buffer resource: 32-bit byte range
-  if (256 * std::max(lda, b_row ? 0 : ldb) * (int64_t)eb > 0x7fffffffLL)
+  if (!panels_fit)
     return fail(SILE_ERR_SHAPE, "leading dimension too large for a 256-row panel (%lld, %lld)",
                 (long long)lda, (long long)ldb);
   if (m > 0x7fffffffLL || n > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "GEMM too large");

@@ -762,3 +762,42 @@ def test_any_pitch_of_c(hip, kind, out, layout, m, n, k, pad):
     assert_close(got, ref, atol=atol * rms, rtol=rtol)
     for b in (da, db, dc):
         b.close()
+
+
+@pytest.mark.parametrize("m,n,layout,pad", [(100, 131, "col", 0), (131, 101, "col", 0),
+                                            (100, 136, "row", 1), (40, 130, "col", 3),
+                                            (140, 64, "col", 0)])
+def test_pitches_past_a_panel(hip, m, n, layout, pad):
+    """A pitch of A that 256 rows of do not fit a 32-bit byte range: shapes that are
+    not the tiles' own (N no multiple of 4, C's rows unaligned, M or N small) run on
+    the kernels that need no panel of 256 rows."""
+    k, lda = 72, 5000000
+    say(f"gemm lda={lda} {m}x{n}x{k} B {layout}")
+    r = rng(m + n)
+    (qa, a_f), (qb, b_f) = (bf16_round((r.normal(size=(x, k)) / np.sqrt(k)).astype(np.float32)) for x in (m, n))
+    da = hip.DeviceBuffer(((m - 1) * lda + k) * 2)
+    for i in range(m):
+        hip.call("sile_hip_memcpy_htod", da.ptr + i * lda * 2, qa[i].ctypes.data, 2 * k)
+    db = hip.DeviceBuffer.from_array(qb if layout == "col" else np.ascontiguousarray(qb.T))
+    ldc = n + pad
+    dc = hip.DeviceBuffer(m * ldc * 4)
+    dc.fill_bytes(0xFF)
+    hip.gemm(hip.BF16, hip.BF16, hip.F32, m, n, k, da.ptr, lda, hip.ROW_MAJOR, db.ptr,
+             k if layout == "col" else n, hip.COL_MAJOR if layout == "col" else hip.ROW_MAJOR, dc.ptr, ldc)
+    hip.synchronize()
+    raw = dc.download(np.uint32, (m, ldc))
+    assert (raw[:, n:] == 0xFFFFFFFF).all()
+    assert_close(raw[:, :n].copy().view(np.float32), a_f.astype(np.float64) @ b_f.astype(np.float64).T,
+                 atol=1e-5, rtol=1e-5)
+    for x in (da, db, dc):
+        x.close()
+
+
+@pytest.mark.parametrize("m,n", [(100, 132), (256, 128), (132, 100)])
+def test_pitches_past_a_panel_refused(hip, m, n):
+    """The tiles' own shapes refuse such a pitch (before any launch)."""
+    buf = hip.DeviceBuffer(m * 5000000 * 2)
+    with pytest.raises(hip.SileError, match="256-row panel"):
+        hip.gemm(hip.BF16, hip.BF16, hip.F32, m, n, 72, buf.ptr, 5000000, hip.ROW_MAJOR, buf.ptr, 72,
+                 hip.COL_MAJOR, buf.ptr, n)
+    buf.close()
