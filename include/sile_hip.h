@@ -272,14 +272,18 @@ int sile_hip_kernel_parallel_reduce(void *const *buffers, int64_t num_threadgrou
  *                        path (N >= 128, any M, any pitch and start of C:
  *                        256 x 256 or 128 x 128 tiles
  *                        through LDS,
- *                        the size chosen by shape; when N is below one tile
- *                        but M is not, the same kernels compute C^T into fp32
- *                        scratch and a second kernel writes C; other shapes:
- *                        64 x 64 tiles).  When A or a column-major B has at
- *                        most 64 rows, a kernel that streams the other operand
- *                        once (plain launch, also under capture) takes the
- *                        place of either, wherever it is modelled faster or
- *                        the tiles cannot take the shape.
+ *                        the size chosen by shape).  With N below one tile
+ *                        the form with the least modelled time runs: 64 x 64
+ *                        tiles straight from the operands, or, when M is at
+ *                        least one tile, the same kernels computing C^T into
+ *                        fp32 scratch with a second kernel writing C.  When A
+ *                        or a column-major B has at most 64 rows, a kernel
+ *                        that streams the other operand once (plain launch,
+ *                        also under capture) takes the place of any of these
+ *                        where it is modelled faster.  The form depends on
+ *                        M, N, K' and the types, so a row's rounding can
+ *                        depend on M and N, and in the last kernel on which
+ *                        row it is (its sums start at different k).
  *                        Pitches past 2^31 bytes in 256 rows are refused for
  *                        the tiles' own shapes (C rows of 16-byte aligned
  *                        multiples of 4; N below one tile and M a multiple of
@@ -429,7 +433,8 @@ int sile_hip_attention_f32_kt(int64_t n_q, int64_t n_k, int64_t head_dim, const 
  * rounding can depend on B, H and S; the probabilities enter the second product
  * in 16 bits, for D an odd multiple of 8 as two 16-bit parts; with D a multiple
  * of 16 a causal row takes in 0 times the V rows of later keys of its block, so
- * an Inf or NaN there makes it NaN, with any other D it does not); other D up to
+ * an Inf or NaN there makes it NaN, and an Inf in V can come out NaN; with any
+ * other D neither happens); other D up to
  * 256, unaligned operands and a scale that is not positive on a VALU kernel of
  * one wave per query row.  No reference counterpart: sile's DSL cannot express
  * attention (no mask/iota/transpose); built from the Tile IR ops MmaF, ReduceMax,

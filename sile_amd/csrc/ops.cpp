@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -72,12 +73,16 @@ struct GemmPlan {
   double seconds;  // modelled time
 };
 
-// compute units of the current device
+// compute units of the current device (asked of the runtime once a device)
 int device_cus(int* cus) {
+  static std::atomic<int> known[64];
   int dev = 0;
   SILE_HIP_CHECK(hipGetDevice(&dev));
+  if (dev >= 0 && dev < 64 && (*cus = known[dev].load(std::memory_order_relaxed)) > 0) return SILE_OK;
   SILE_HIP_CHECK(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
-  return *cus > 0 ? SILE_OK : SILE_ERR_RUNTIME;
+  if (*cus <= 0) return fail(SILE_ERR_RUNTIME, "device %d reports no compute units", dev);
+  if (dev >= 0 && dev < 64) known[dev].store(*cus, std::memory_order_relaxed);
+  return SILE_OK;
 }
 
 // seconds per element of K' for one tile, with w workgroups of that size
@@ -95,11 +100,8 @@ double tile_time_per_k(int tile, int64_t w, int cus) {
 GemmPlan gemm_plan(int64_t m, int64_t n, int64_t kp, int64_t half_steps, int64_t cb, bool fp8,
                    int only_tile) {
   GemmPlan best{only_tile ? only_tile : m >= 256 && n >= 256 ? 256 : 128, 1, 0.0};
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus <= 0)
-    return best;
+  int cus = 0;
+  if (device_cus(&cus) != SILE_OK) return best;
   double best_t = 1e30, best_unsplit_t = 1e30;
   GemmPlan best_unsplit = best;
   for (int tile : {256, 128}) {
@@ -131,23 +133,57 @@ GemmPlan gemm_plan(int64_t m, int64_t n, int64_t kp, int64_t half_steps, int64_t
   return best.splits > 1 && !(best_t < 0.95 * best_unsplit_t) ? best_unsplit : best;
 }
 
-// 16-row tiles of the large operand a workgroup of the few-rows GEMM takes: the
-// most (1, 2 or 4) that still give a workgroup to nine CUs of ten.  *seconds:
-// its modelled time, the operands' bytes at 5.4 TB/s or the rounds of
-// workgroups (one a CU), each its rows' bytes at 105 GB/s and 1.5 us.  Measured
-// with 1 / 2 / 4 tiles: bf16 16 x 8192 x 8192 29.9 / 28.0 / 31.1 us, 16 x 1024 x
-// 16384 15.1 / 18.5 / 26.6, 16 x 16384 x 1024 12.3 / 9.3 / 7.9, 64 x 8192 x 8192
-// 46.9 / 33.4 / 41.9, 64 x 16384 x 8192 91.6 / 64.2 / 50.7.
-int gemm_few_tiles(int64_t rows_s, int64_t rows_l, int64_t row_bytes, double* seconds) {
-  int cus = 0;
-  if (device_cus(&cus) != SILE_OK) cus = 256;
-  int r = 4;
-  while (r > 1 && rows_l < (int64_t)(0.9 * 16 * r * cus)) r /= 2;
-  const int64_t s16 = rows_s <= 16 ? 16 : rows_s <= 32 ? 32 : 64;
-  const int64_t rounds = ((rows_l + 16 * r - 1) / (16 * r) + cus - 1) / cus;
-  *seconds = 3e-6 + std::max((double)((rows_s + rows_l) * row_bytes) / 5.4e12 + 1.5e-6,
-                             (double)rounds * ((double)((16 * r + s16) * row_bytes) / 105e9 + 1.5e-6));
-  return r;
+// The forms a column-major GEMM can run in beside the direct tiles, and their
+// modelled times in seconds, among back-to-back calls.  Fitted to timings of 1062
+// shapes, operands rotated through 0.8 GB: M or N = 1 .. 64 and N = 65 .. 127
+// against 1 .. 2^20 of the other and K' = 64 .. 65536, bf16 and fp8; the chosen
+// form is within 1 % of the fastest on average.
+
+// Few rows (one operand of at most 64): 16-row tiles of the large operand a
+// workgroup takes, 1 or 2 where that is one round of workgroups (one a CU), else
+// 4: bf16 16 x 8192 x 8192 28.6 / 24.9 / 29.6 us with 1 / 2 / 4, 64 x 10000 x 8192
+// 66.4 / 56.9 / 43.2, 64 x 4096 x 4096 14.0 / 16.4 / 22.1.
+int gemm_few_tiles(int64_t rows_l, int cus) {
+  return rows_l <= 16ll * cus ? 1 : rows_l <= 32ll * cus ? 2 : 4;
+}
+// The longest of: the operands' bytes at 6.2 TB/s with the rounds' starts and ends
+// between; the rounds, each its k-steps (128 bytes of a row, a quarter of them a
+// wave); and every workgroup reading all of the small operand, from L2 up to 3 MB.
+double gemm_few_time(int64_t rows_s, int64_t rows_l, int64_t row_bytes, int cus) {
+  const int r = gemm_few_tiles(rows_l, cus), sm = rows_s <= 16 ? 1 : rows_s <= 32 ? 2 : 4;
+  const double wgs = (double)((rows_l + 16 * r - 1) / (16 * r)), rounds = std::ceil(wgs / cus);
+  const double steps = std::ceil((double)row_bytes / 512), small = (double)(rows_s * row_bytes);
+  const double hbm = (double)((rows_s + rows_l) * row_bytes) / 6.2e12 + 3.2e-6 + 0.9e-6 * sm * (rounds - 1);
+  const double run = 0.9e-6 + rounds * (0.55e-6 * sm + 0.11e-6 * r + steps * (0.05e-6 * sm + 0.24e-6 * r));
+  const double reads = 0.9e-6 + wgs * small / (small > 3e6 ? 8.3e12 : 10.3e12);
+  return std::max({5.1e-6, hbm, run, reads});
+}
+
+// 64 x 64 tiles straight from the operands: rounds of workgroups, each a chain of
+// K' bytes by the rows a workgroup loads.
+double gemm_small_time(int64_t m, int64_t n, int64_t row_bytes, int cus) {
+  const double rounds = std::ceil((double)((m + 63) / 64) * (double)((n + 63) / 64) / cus);
+  const double rows = (double)(std::min<int64_t>(m, 64) + std::min<int64_t>(n, 64));
+  return std::max(4.2e-6, 0.8e-6 + rounds * (1.1e-6 + (double)row_bytes * std::max(1.9e-9, 0.2e-9 + 0.056e-9 * rows)));
+}
+
+// The transposed form of an M x N product (its plan is of N x M): the host's part
+// of two launches and the scratch's events, the tiles, the operands' bytes, and the
+// fp32 planes written and read.
+double gemm_transposed_time(const GemmPlan& plan, int64_t m, int64_t n, int64_t row_bytes, int64_t cb) {
+  const double mn = (double)m * (double)n, sp = (double)plan.splits;
+  return std::max(10.8e-6, 8e-6 + 0.46 * plan.seconds +
+                               (0.75 * (double)((m + n) * row_bytes) + 1.15 * (8 * sp + (double)cb) * mn) / 5e12 +
+                               1.5e-6 * std::log2(sp));
+}
+
+// The direct tiles of at most 64 rows of A, where a launch is mostly the operands'
+// bytes and a deep split.
+double gemm_tiles_few_time(const GemmPlan& plan, int64_t m, int64_t n, int64_t row_bytes, int64_t cb) {
+  const double mn = (double)m * (double)n, sp = (double)plan.splits;
+  double t = -1.6e-6 + 0.96 * plan.seconds + (0.5 * (double)((m + n) * row_bytes) + 0.72 * (double)cb * mn) / 5e12;
+  if (plan.splits > 1) t += 0.72 * 8 * sp * mn / 5e12 + 3.4e-6 * std::log2(sp) - 7.5e-6;
+  return std::max(5e-6, t);
 }
 
 // How the flash kernel's work is laid out: the keys of a query block shared by
@@ -583,22 +619,34 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
     return rc;
   }
   // few rows of A or of a column-major B: the kernel that streams the other
-  // operand once, where it is modelled faster than the tiles (or those cannot
-  // take the shape)
+  // operand once.  It and the transposed form are taken where they are modelled
+  // faster by 7 and 13 %, or where they alone can run.
   const int64_t rows_s = std::min(m, n), rows_l = std::max(m, n);
-  if (!b_row && !tile_req && !splits_req && rows_s <= 64 &&
-      64 * std::max(lda, ldb) * (int64_t)eb <= 0x7fffffffLL) {
-    double few_t = 0.0;
-    const int r = gemm_few_tiles(rows_s, rows_l, kp * (int64_t)eb, &few_t);
-    bool use = !direct || !panels_fit;
-    if (!use) {
-      const GemmPlan plan = gemm_plan(m, n, kp, (kp + kstep - 1) / kstep, (int64_t)cb, fp8, 0);
-      // (the tiles' model leaves out the operands' bytes and ~4 us of what a
-      // launch of few tiles with a deep split measures)
-      const double bytes = (double)((rows_s + rows_l) * kp) * (double)eb;
-      use = few_t < std::max(plan.seconds, bytes / 5.1e12 + 4e-6 + (plan.splits > 1 ? 5.5e-6 : 0.0)) + 4e-6;
+  const int64_t row_bytes = kp * (int64_t)eb, half_steps = (kp + kstep - 1) / kstep;
+  const bool few_ok = !b_row && !tile_req && !splits_req && rows_s <= 64 &&
+                      64 * std::max(lda, ldb) * (int64_t)eb <= 0x7fffffffLL &&
+                      (rows_l + 15) / 16 <= 0x7fffffffLL;
+  bool transposed = !b_row && !direct && !capturing && m >= 128 &&
+                    (panels_fit || (m % 4 == 0 && !few_ok)) &&
+                    (m + 3) / 4 * 4 * n * 4 <= kScratchPlanesMax;
+  const bool small_ok = (m + 63) / 64 <= 65535;
+  int cus = 0;
+  if (!b_row && !tile_req && !splits_req && (!direct || few_ok)) {
+    int rc = device_cus(&cus);
+    if (rc != SILE_OK) return rc;
+    const double small_t = gemm_small_time(m, n, row_bytes, cus);
+    double t = direct ? gemm_tiles_few_time(gemm_plan(m, n, kp, half_steps, (int64_t)cb, fp8, 0), m,
+                                            n, row_bytes, (int64_t)cb)
+                      : small_t;
+    if (transposed && panels_fit) {
+      const double tr = gemm_transposed_time(gemm_plan(n, m, kp, half_steps, (int64_t)cb, fp8, 0), m,
+                                             n, row_bytes, (int64_t)cb) / 0.87;
+      transposed = tr < t || !small_ok;
+      if (transposed) t = tr;
     }
-    if (use) {
+    const bool others = direct ? panels_fit : transposed || small_ok;
+    if (few_ok && (!others || gemm_few_time(rows_s, rows_l, row_bytes, cus) / 0.93 < t)) {
+      const int r = gemm_few_tiles(rows_l, cus);
       const bool l_is_b = m <= n;
       struct {
         int64_t ldl, lds, ldc, rows_l, kp;
@@ -608,22 +656,18 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
            // past what the 256 MB Infinity Cache holds beside other operands,
            // non-temporal loads stream faster (16 x 8192 x 8192, 134 MB: 28.0 ->
            // 24.7 us); below they lose its hits (67 MB: 12.9 -> 13.5)
-           rows_l * kp * (int64_t)eb >= (96ll << 20) ? 1 : 0, scale_a * scale_b};
+           rows_l * row_bytes >= (96ll << 20) ? 1 : 0, scale_a * scale_b};
       const void* lop = l_is_b ? b : a;
       const void* sop = l_is_b ? a : b;
       const int64_t wgs = (rows_l + 16 * r - 1) / (16 * r);
-      if (wgs > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "GEMM too large");
       char fname[64];
       snprintf(fname, sizeof fname, "sile_gemm_few_%s_r%dm%d", name + strlen("sile_gemm_nt_"), r,
                rows_s <= 16 ? 1 : rows_s <= 32 ? 2 : 4);
       void* fp[] = {&lop, &sop, &c, &fg};
-      int rc = launch(Module::kGemm, fname, dim3((unsigned)wgs), dim3(256), fp, s);
+      rc = launch(Module::kGemm, fname, dim3((unsigned)wgs), dim3(256), fp, s);
       return rc == SILE_OK ? ok() : rc;
     }
   }
-  const bool transposed = !b_row && !direct && !capturing && m >= 128 &&
-                          (panels_fit || m % 4 == 0) &&
-                          (m + 3) / 4 * 4 * n * 4 <= kScratchPlanesMax;
   if (!direct && !transposed) {
     // the any-shape kernel, 64 x 64 tiles with fragments loaded straight
     // from the operands
@@ -651,7 +695,6 @@ int gemm_impl(sile_dtype a_type, sile_dtype b_type, sile_dtype c_type, int64_t m
     return fail(SILE_ERR_SHAPE, "leading dimension too large for a 256-row panel (%lld, %lld)",
                 (long long)lda, (long long)ldb);
   if (m > 0x7fffffffLL || n > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "GEMM too large");
-  const int64_t half_steps = (kp + kstep - 1) / kstep;
   if (half_steps > 0x7fffffffLL) return fail(SILE_ERR_SHAPE, "GEMM K too large");
   GemmPlan plan = gemm_plan(rm, rn, kp, half_steps, (int64_t)cb, fp8, tile_req);
   if (splits_req) plan.splits = splits_req;

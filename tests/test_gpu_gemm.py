@@ -536,13 +536,27 @@ def test_tile128(hip, kind, out, m, n, k, bk, tile):
     ("fp8", "bf16", 512, 258, 256, 0, 0),
     ("fp8", "bf16", 512, 64, 320, 0, 0),
     ("fp8", "f32", 256, 300, 320, 5, 0),
+    # N of 65 .. 127 and a K' long enough: C^T = B . A^T, one and several k-ranges,
+    # M a multiple of 4 and not
+    ("bf16", "bf16", 512, 96, 4096, 8, 0),
+    ("f16", "f32", 1030, 100, 8192, 0, 0),
+    ("bf16", "f32", 131, 127, 5000, 3, 70),
+    ("f16", "f16", 4097, 65, 2056, 0, 0),
+    ("bf16", "bf16", 20001, 120, 1024, 1, 0),
+    ("fp8", "bf16", 515, 81, 8192, 0, 0),
+    ("fp8", "f32", 4096, 127, 4096, 5, 0),
+    # N of at most 64 and a very long K', or very many rows
+    ("bf16", "bf16", 128, 64, 65536, 0, 0),
+    ("bf16", "f32", 300, 33, 131072, 1, 0),
 ])
 def test_transposed_form(hip, kind, out, m, n, k, ldc_pad, bk):
-    """Shapes the direct LDS form cannot take (N below one tile, N not a
-    multiple of 4, C's rows not 16-byte aligned) with M a multiple of 4 and at
-    least one tile run C^T = B . A^T on the LDS kernels into fp32 planes,
-    written back transposed with element stores.  Every element is checked,
-    the pitch past N keeps its fill, and a second call gives the same bits."""
+    """Shapes around the one whose N is below one tile and M is not, which runs
+    C^T = B . A^T on the LDS kernels into fp32 planes, written back transposed
+    with element stores, where that is modelled faster than the any-shape and
+    the few-rows kernels (the first ten shapes are what it was tested with when
+    it also took N that is no multiple of 4 and unaligned C rows; most now run on
+    the few-rows kernel or the direct tiles).  Every element is checked, the
+    pitch past N keeps its fill, and a second call gives the same bits."""
     kp = (k // bk) * bk if bk else k
     ldc = n + ldc_pad
     say(f"gemm transposed {kind} {m}x{n}x{k} ldc={ldc} bk={bk} -> {out}")
@@ -584,10 +598,13 @@ def test_split_k_scratch_across_streams_and_growth(hip):
     other's planes (the library orders them with an event), and a call that
     needs more scratch than an earlier one grows it while the earlier work
     may still be running.  Sequence: small split on stream 1, large split on
-    stream 2 (grows the scratch), transposed form on stream 1, small split on
-    stream 2, each with its own inputs; every result against the oracle."""
+    stream 2 (grows the scratch), a few-rows GEMM (no scratch) on stream 1,
+    small split on stream 2, transposed form with several k-ranges on stream 1,
+    another split on stream 2, each with its own inputs; every result against the
+    oracle."""
     say("gemm scratch: two streams, growth")
-    cases = [(256, 256, 4096, 1), (512, 512, 8192, 2), (512, 64, 2048, 1), (256, 256, 2048, 2)]
+    cases = [(256, 256, 4096, 1), (512, 512, 8192, 2), (512, 64, 2048, 1), (256, 256, 2048, 2),
+             (512, 96, 8192, 1), (300, 256, 8192, 2)]
     s1, s2 = hip.Stream(), hip.Stream()
     streams = {1: s1, 2: s2}
     runs = []

@@ -130,7 +130,8 @@ def test_row_major_b_split_k(hip, kind, out, m, n, k, splits, tile):
     ("f16", "f16", 256, 512, 128, 1, 0),      # B's rows not 16-byte aligned
     ("bf16", "bf16", 1, 1, 8, 0, 0),          # the any-shape kernel (A's rows 16 bytes)
     ("bf16", "f32", 16, 300, 136, 0, 5),
-    ("bf16", "bf16", 130, 64, 200, 0, 1),     # the transposed form after the transpose
+    ("bf16", "bf16", 130, 64, 200, 0, 1),     # the few-rows or any-shape kernel after the transpose
+    ("bf16", "bf16", 300, 96, 4096, 0, 1),    # the transposed form after the transpose
 ])
 def test_row_major_b_other_shapes(hip, kind, out, m, n, k, ldb_pad, ldc_pad):
     say(f"gemm B row-major (scratch path) {kind}->{out} {m}x{n}x{k} ldb+{ldb_pad} ldc+{ldc_pad}")
