@@ -313,7 +313,8 @@ def test_flash_head_dims_of_8(hip, dt, causal, d, s):
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("trend", ["flat", "rising"])
 @pytest.mark.parametrize("causal,h,s,d", [
-    (False, 8, 33, 128), (True, 8, 97, 96),      # 2 groups, one with no key for some queries
+    (False, 8, 33, 128),                          # one group
+    (True, 8, 97, 96),                            # 2 groups, one with no key for some queries
     (True, 8, 5, 64), (False, 3, 1, 40),
     (True, 40, 520, 128), (False, 32, 700, 128),  # 2 groups, ragged ends; longest blocks first
     (True, 32, 1100, 64),
@@ -342,6 +343,41 @@ def test_flash_key_groups(hip, dt, trend, causal, h, s, d):
     for hi in sorted({0, 7, h // 2, h - 1} & set(range(h))):
         ref = cpuref.attention_fwd(qf[0, hi], kf[0, hi], vf[0, hi], scale, causal=causal)
         assert_close(got[0, hi], ref, atol=ATOL, rtol=RTOL, what=f"h{hi}")
+
+
+@pytest.mark.parametrize("causal,h,s,d", [(True, 8, 97, 96), (True, 40, 520, 128), (False, 16, 1000, 64),
+                                          (True, 8, 1500, 128)])
+def test_flash_key_groups_repeat(hip, causal, h, s, d):
+    """2 and 4 key groups: the same bits from call to call."""
+    say(f"flash groups repeat causal={causal} H={h} S={s} D={d}")
+    bits = [x[0] for x in _inputs(1, h, s, d, "f16", seed=s)]
+    first = _run(hip, "f16", 1, h, s, d, bits, causal, 1.0 / np.sqrt(d))
+    for _ in range(3):
+        assert (_run(hip, "f16", 1, h, s, d, bits, causal, 1.0 / np.sqrt(d)) == first).all()
+
+
+@pytest.mark.parametrize("h,s,d", [(8, 97, 96), (16, 1000, 64), (8, 700, 40)])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+def test_flash_key_groups_inf_nan(hip, h, s, d, dt):
+    """Not causal, keys in groups: an Inf in V reaches its dim of every row and no
+    other dim, whichever group holds it (NaN there in the first block for head dims
+    of 16: the pipeline's first product is of its V and zeros); a NaN in K every dim
+    of every row."""
+    say(f"flash groups Inf / NaN {dt} H={h} S={s} D={d}")
+    scale = 1.0 / np.sqrt(d)
+    qkv = _inputs(1, h, s, d, dt, seed=s + d)
+    rnd = f16_round if dt == "f16" else bf16_round
+    for key in (0, s // 2, s - 1):
+        q, k, v = (x[1].copy() for x in qkv)
+        v[0, :, key, 3] = np.inf
+        got = _run(hip, dt, 1, h, s, d, [rnd(x)[0] for x in (q, k, v)], False, scale)
+        other = np.arange(d) != 3
+        assert (got[0, :, :, 3] == np.inf).all() if d % 16 else not np.isfinite(got[0, :, :, 3]).any()
+        for hi in (0, h - 1):
+            ref = cpuref.attention_fwd(q[0, hi], k[0, hi], qkv[2][1][0, hi], scale, causal=False)
+            assert_close(got[0, hi][:, other], ref[:, other], atol=ATOL, rtol=RTOL, what=f"h{hi} key {key}")
+        k[0, :, key, 0] = np.nan
+        assert np.isnan(_run(hip, dt, 1, h, s, d, [rnd(x)[0] for x in (q, k, v)], False, scale)).all()
 
 
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
@@ -505,12 +541,14 @@ def test_attention_f32_kt_tiles_and_ranges(hip, n_q, n_k, d, pad, m0):
     test_attention_f32_kt_matches_the_program(hip, n_q, n_k, d, pad, m0)
 
 
-@pytest.mark.parametrize("d,ldkt,ldv", [(3, (1 << 26) + 1, 3), (33, 40, (1 << 26) + 1)])
-def test_attention_f32_kt_far_pitches(hip, d, ldkt, ldv):
+@pytest.mark.parametrize("d,ldkt,ldv,n_k", [(3, (1 << 26) + 1, 3, 3), (33, 40, (1 << 26) + 1, 3),
+                                            # several key blocks a wave, key ranges
+                                            (3, (1 << 26) + 1, 3, 1000), (34, (1 << 26) + 5, 35, 2100)])
+def test_attention_f32_kt_far_pitches(hip, d, ldkt, ldv, n_k):
     """Row pitches past the 32-bit lane offsets (kt's rows 256 MiB apart, or
     v's): the kernels with a 64-bit address a load."""
-    n_q, n_k = 33, 3
-    say(f"attention_f32_kt d={d} ldkt={ldkt} ldv={ldv}")
+    n_q = 33
+    say(f"attention_f32_kt d={d} ldkt={ldkt} ldv={ldv} n_k={n_k}")
     q, kt, v = _dsl_attn_inputs(n_q, n_k, d, d)
     dq, do = hip.DeviceBuffer.from_array(q), hip.DeviceBuffer(n_q * d * 4)
     dk = hip.DeviceBuffer(((d - 1) * ldkt + n_k) * 4)
@@ -551,6 +589,60 @@ def test_attention_f32_kt_largest_floats(hip, n_k, m0):
     assert_close(do.download(np.float32, (n_q, d)), ref, atol=1e-5, rtol=1e-4, what="largest floats")
     for b in bufs + [do]:
         b.close()
+
+
+def test_attention_f32_kt_ranges_beside_split_gemms(hip):
+    """Calls with key ranges on two streams, between GEMMs whose K' is split (another
+    part of the device scratch), none waited for: all right, and with the bits of
+    the same calls one by one."""
+    say("attention_f32_kt with ranges beside split GEMMs, two streams")
+    s1, s2 = hip.Stream(), hip.Stream()
+    att = []
+    for n_q, n_k, d in ((33, 4096, 128), (70, 2000, 40), (256, 3000, 64)):
+        q, kt, v = _dsl_attn_inputs(n_q, n_k, d, n_k + d)
+        scale = 1 / np.sqrt(d)
+        ref = cpuref.dsl_attention_f32(q, kt, v, n_k, scale, -1e30, d=d, n_q=n_q, s_k=n_k)
+        att.append((n_q, n_k, d, scale, ref, [hip.DeviceBuffer.from_array(x) for x in (q, kt, v)]))
+    m, k = 256, 8192
+    a, b = (bf16_round((rng(i).normal(size=(m, k)) / np.sqrt(k)).astype(np.float32)) for i in (1, 2))
+    da, db = hip.DeviceBuffer.from_array(a[0]), hip.DeviceBuffer.from_array(b[0])
+    gref = cpuref.gemm_nt(a[1], b[1])
+
+    def queue(streams, wait):
+        outs = []
+        for i in range(12):
+            n_q, n_k, d, scale, ref, bufs = att[i % 3]
+            do, dc = hip.DeviceBuffer(n_q * d * 4), hip.DeviceBuffer(m * m * 4)
+            for b in (do, dc):
+                b.fill_bytes(0xFF)
+            outs.append((i % 3, do, dc))
+        hip.synchronize()
+        for i, (j, do, dc) in enumerate(outs):
+            n_q, n_k, d, scale, ref, bufs = att[j]
+            hip.attention_f32_kt(n_q, n_k, d, bufs[0].ptr, d, bufs[1].ptr, n_k, bufs[2].ptr, d, do.ptr, d,
+                                 scale, -1e30, streams[i % 2])
+            hip.gemm(hip.BF16, hip.BF16, hip.F32, m, m, k, da.ptr, k, hip.ROW_MAJOR, db.ptr, k,
+                     hip.COL_MAJOR, dc.ptr, m, 1.0, 1.0, 0, streams[(i // 2) % 2])
+            if wait:
+                hip.synchronize()
+        for st in streams:
+            st.synchronize()
+        res = []
+        for j, do, dc in outs:
+            n_q, n_k, d, scale, ref, bufs = att[j]
+            res.append((do.download(np.float32, (n_q, d)), dc.download(np.float32, (m, m))))
+            assert_close(res[-1][0], ref, atol=1e-5, rtol=1e-4, what="attention")
+            assert_close(res[-1][1], gref, atol=1e-4, rtol=1e-4, what="split GEMM")
+            do.close()
+            dc.close()
+        return res
+
+    for (o1, c1), (o2, c2) in zip(queue((s1, s2), False), queue((s1, s2), True)):
+        assert (o1 == o2).all() and (c1 == c2).all()
+    for x in [da, db] + [x for c in att for x in c[5]]:
+        x.close()
+    s1.close()
+    s2.close()
 
 
 def test_attention_f32_kt_closed_forms(hip):

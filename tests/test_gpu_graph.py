@@ -1,14 +1,15 @@
 """GPU: op calls captured into a HIP graph (sile_hip_graph_begin / end) and
 replayed.
 
-A graph of GEMMs (one that splits K' when run eagerly, one that takes the
-transposed form eagerly, one plain), a row softmax and a causal flash
-attention is replayed three times, with eager split GEMMs on another stream
-and device synchronisations in between.  Every replay is checked: the ops
-whose captured form equals the eager one bit for bit against the eager
-result, the two GEMMs whose scratch-using forms are left out under capture
-against the oracle (|g - r| <= 2e-2 + 1e-2 |r|, fp32 out 1e-4) and against
-the first replay bit for bit.
+A graph of GEMMs (one that splits K' when run eagerly, one with N below a tile,
+one plain), a row softmax and a causal flash attention is replayed three times,
+with eager split GEMMs on another stream and device synchronisations in between.
+Every replay is checked: the ops whose captured form equals the eager one bit for
+bit against the eager result, two GEMMs against the oracle (|g - r| <= 2e-2 +
+1e-2 |r|, fp32 out 1e-4) and against the first replay bit for bit.  Another graph
+holds the forms that this one leaves out: a GEMM that takes the transposed form
+eagerly, a few-rows one, one with unaligned C rows, and an fp32 attention with
+key ranges eagerly.
 """
 import os
 import subprocess
@@ -34,7 +35,7 @@ def test_graph_replays_op_calls(hip):
     say("graph: capture gemm x3 + softmax + flash attention, replay x3")
     st, other = hip.Stream(), hip.Stream()
     gemms = []
-    # (m, n, k, out): split K' eagerly; transposed form eagerly (N < 128); plain 128 tiles
+    # (m, n, k, out): split K' eagerly; N < 128; plain 128 tiles
     for idx, (m, n, k, out) in enumerate([(256, 256, 8192, hip.F32), (512, 64, 256, hip.BF16),
                                           (512, 512, 512, hip.BF16)]):
         qa, qb, ref = _bf16_operands(70 + 2 * idx, m, n, k)
@@ -96,7 +97,7 @@ def test_graph_replays_op_calls(hip):
         # plain GEMM, softmax and attention: the captured launches are the eager ones
         for i in (2, 3, 4):
             assert (got[i] == eager[i]).all(), f"replay {rep}: output {i} differs from eager"
-        # the two GEMMs that run without the scratch under capture: the oracle
+        # the two others (the first runs without the scratch under capture): the oracle
         for i in (0, 1):
             m, n, k, out, cb, ref, _ = gemms[i]
             val = (got[i].view(np.float32) if cb == 4
@@ -113,6 +114,72 @@ def test_graph_replays_op_calls(hip):
     graph.close()
     for buf in [x for *_, bufs in gemms for x in bufs] + [dx, dy, dq, dk, dv, do, ea, eb, ec]:
         buf.close()
+    st.close()
+    other.close()
+
+
+def test_graph_replays_other_forms(hip):
+    say("graph: C^T shape, few rows, unaligned C, fp32 attention, replay x3")
+    st, other = hip.Stream(), hip.Stream()
+    # (m, n, k, ldc, same launches under capture)
+    gemms = []
+    for idx, (m, n, k, ldc, same) in enumerate([(512, 96, 4096, 96, False), (16, 2048, 2048, 2048, True),
+                                                (300, 258, 256, 259, True)]):
+        qa, qb, ref = _bf16_operands(30 + 2 * idx, m, n, k)
+        gemms.append((m, n, k, ldc, same, ref, (hip.DeviceBuffer.from_array(qa), hip.DeviceBuffer.from_array(qb),
+                                                hip.DeviceBuffer(m * ldc * 4))))
+    n_q, n_k, d = 100, 2000, 64
+    q, kt, v = (rng(50 + i).normal(size=z).astype(np.float32) for i, z in enumerate([(n_q, d), (d, n_k), (n_k, d)]))
+    att = [hip.DeviceBuffer.from_array(x) for x in (q, kt, v)]
+    do = hip.DeviceBuffer(n_q * d * 4)
+    aref = cpuref.dsl_attention_f32(q, kt, v, n_k, 0.125, -1e30, d=d, n_q=n_q, s_k=n_k)
+
+    def calls(stream, outs):
+        for (m, n, k, ldc, _, _, (da, db, _)), out in zip(gemms, outs):
+            hip.gemm(hip.BF16, hip.BF16, hip.F32, m, n, k, da.ptr, k, hip.ROW_MAJOR, db.ptr, k,
+                     hip.COL_MAJOR, out.ptr, ldc, 1.0, 1.0, 0, stream)
+        hip.attention_f32_kt(n_q, n_k, d, att[0].ptr, d, att[1].ptr, n_k, att[2].ptr, d, outs[-1].ptr, d, 0.125,
+                             -1e30, stream)
+
+    outs = [g[-1][2] for g in gemms] + [do]
+    beside = [hip.DeviceBuffer(g[0] * g[3] * 4) for g in gemms] + [hip.DeviceBuffer(n_q * d * 4)]
+
+    def results(bufs):
+        return [b.download(np.float32, (g[0], g[3]))[:, :g[1]] for g, b in zip(gemms, bufs)] + [
+            bufs[-1].download(np.float32, (n_q, d))]
+
+    def check(res, what):
+        for g, got in zip(gemms, res):
+            assert_close(got, g[5], atol=1e-4, rtol=1e-4, what=f"{what} gemm {g[:3]}")
+        assert_close(res[-1], aref, atol=1e-5, rtol=1e-4, what=f"{what} attention")
+
+    calls(st, outs)
+    st.synchronize()
+    eager = results(outs)
+    check(eager, "eager")
+    with hip.Graph(st) as graph:
+        calls(st, outs)
+    first = None
+    for rep in range(3):
+        for b in outs + beside:
+            b.fill_bytes(0xFF)
+        hip.synchronize()
+        graph.launch()
+        calls(other, beside)     # the scratch forms, eagerly beside the replay
+        st.synchronize()
+        other.synchronize()
+        say(f"graph replay {rep}")
+        got, near = results(outs), results(beside)
+        check(got, f"replay {rep}")
+        for i, g in enumerate(gemms):
+            assert not g[4] or (got[i] == eager[i]).all(), f"replay {rep}: gemm {i} differs from eager"
+        for i, x in enumerate(near):
+            assert (x == eager[i]).all(), f"beside replay {rep}: output {i} differs"
+        first = first or got
+        assert all((x == y).all() for x, y in zip(got, first)), f"replay {rep} changed"
+    graph.close()
+    for b in [x for g in gemms for x in g[-1][:2]] + att + outs + beside:
+        b.close()
     st.close()
     other.close()
 
