@@ -975,8 +975,8 @@ EXTRA = ["copy_calibration", "llir_vec_add", "llir_softmax_f32_8192", "llir_soft
          "gemm_f32_exact_512", "reduce_rows_f32_8192", "parallel_reduce_f32",
          # the mlp example's matvec program (BK 32; _bk8: the example's BK)
          "matvec_f32_8192", "matvec_f32_8192_bk8",
-         # shapes off the headline configurations: 128 x 128 tiles, split K', the
-         # transposed form (M x N x K)
+         # shapes off the headline configurations: 128 x 128 tiles, split K', few
+         # columns (M x N x K)
          "gemm_bf16_2048x2048x2048", "gemm_bf16_128x8192x8192", "gemm_bf16_8192x64x8192",
          "gemm_fp8_256x8192x8192",
          # causal attention at an S that is not a multiple of the query block,

@@ -768,8 +768,8 @@ SILE_GEMM_SPLITK_REDUCE_T(sile_gemm_splitk_reduce_t_f16, kOutF16)
 SILE_GEMM_SPLITK_REDUCE_T(sile_gemm_splitk_reduce_t_f32, kOutF32)
 
 // ---------------------------------------------------------------------------
-// Any shape: N below one 128 x 128 tile (and M too, or its C^T scratch not at
-// hand).
+// Any shape: N below one 128 x 128 tile, where the C^T form (M at least a tile)
+// and the few-rows kernel below are not modelled faster or cannot run.
 //
 // 64 x 64 output tile per workgroup of 4 waves (2 x 2), a 32 x 32 block per
 // wave on v_mfma_f32_32x32x16_{bf16,f16} (16 k per MFMA) or
